@@ -16,6 +16,10 @@
 // (adjoint stencils, src/dft_fill_FMT.c:41-189) through the symmetric Hessian
 // of Phi; the mean-field columns collect -I and the +1 of the EL rows.
 // Zero-density columns and rows follow the reference's insertion rules.
+//
+// On 2D/3D grids whose spectra are built the three steps run as spectral products (fft_vjp,
+// tmi_fft.hip); the gathers here serve 1D problems and 2D/3D ones whose stencils stay direct
+// (a small attraction stencil, TMI_FMT_FFT=0 or TMI_MF_FFT=0).
 #include <hip/hip_runtime.h>
 
 #include "tmi_device.hpp"
@@ -102,42 +106,6 @@ __global__ void k_corr_rho(Geo gu, Geo g2, CorrRhoArgs a, int nmf, const T *__re
         for (int k = 0; k < s.L; ++k) acc += w[k] * src[-(long long)s.lo[k]];
     }
     out[(size_t)c * gu.np + p] = acc;
-}
-
-// enumerate the padded positions that map onto node j (itself, periodic and
-// mirror images) and call f(position, reflect mask)
-template <typename F>
-__device__ inline void for_each_image(const Geo &g, int j, F &&f)
-{
-    int c[3];
-    c[0] = j % g.nx[0];
-    const int r = j / g.nx[0];
-    c[1] = r % g.nx[1];
-    c[2] = r / g.nx[1];
-    int cand[3][3], nc[3];
-    for (int d = 0; d < 3; ++d) {
-        nc[d] = 1;
-        cand[d][0] = c[d];
-        if (d >= g.nd) continue;
-        const int n = g.nx[d];
-        if (g.bc[d][0] == TMI_PERIODIC) {
-            cand[d][nc[d]++] = c[d] - n;
-            cand[d][nc[d]++] = c[d] + n;
-        } else {
-            if (g.bc[d][0] == TMI_REFLECT && c[d] != 0) cand[d][nc[d]++] = -c[d];
-            if (g.bc[d][1] == TMI_REFLECT && c[d] != n - 1) cand[d][nc[d]++] = 2 * (n - 1) - c[d];
-        }
-    }
-    for (int a = 0; a < nc[0]; ++a)
-        for (int b = 0; b < nc[1]; ++b)
-            for (int e = 0; e < nc[2]; ++e) {
-                const int q0 = cand[0][a] + g.h[0], q1 = cand[1][b] + g.h[1], q2 = cand[2][e] + g.h[2];
-                if (q0 < 0 || q0 >= g.P[0] || q1 < 0 || q1 >= g.P[1] || q2 < 0 || q2 >= g.P[2]) continue;
-                const long long pos = (long long)q0 + (long long)q1 * g.P[0] + (long long)q2 * g.P[0] * g.P[1];
-                int src = -1, refl = 0;
-                if (map_pad(g, pos, src, refl) != 0 || src != j) continue;
-                f(pos, refl);
-            }
 }
 
 // density columns: y_c(j) = diag * w_EL + [not zero] * sum over images of rho_hat
@@ -358,10 +326,12 @@ void launch_vjp(Problem &P, const double *x, const double *w_in, double *y, hipS
         dev_fill(0.0, rb + (4 + nd) * N, (long long)(nd * N), s);
         w = P.d_w0;
     }
-    switch (P.p.ndim) {
-    case 1: vjp_nd<T, 1>(P, x, w, y, s); break;
-    case 2: vjp_nd<T, 2>(P, x, w, y, s); break;
-    default: vjp_nd<T, 3>(P, x, w, y, s); break;
+    if (!fft_vjp<T>(P, x, w, y, s)) {
+        switch (P.p.ndim) {
+        case 1: vjp_nd<T, 1>(P, x, w, y, s); break;
+        case 2: vjp_nd<T, 2>(P, x, w, y, s); break;
+        default: vjp_nd<T, 3>(P, x, w, y, s); break;
+        }
     }
     hw_apply(P.hw_tr, w + (size_t)P.iu_rb * P.N, y + (size_t)P.iu_rho * P.N, s);   // hard-surface weights
     one_size_transpose(P, w_in + (size_t)P.iu_rb * P.N, y + (size_t)P.iu_rb * P.N, s);

@@ -138,6 +138,47 @@ __device__ inline int map_pad(const Geo &g, long long pos, int &src, int &refl)
     return 0;
 }
 
+// enumerate the padded positions that map onto node j (itself, periodic and
+// mirror images) and call f(q0, q1, q2, position, reflect mask), q the padded coordinates
+template <typename F>
+__device__ inline void for_each_image_at(const Geo &g, int j, F &&f)
+{
+    int c[3];
+    c[0] = j % g.nx[0];
+    const int r = j / g.nx[0];
+    c[1] = r % g.nx[1];
+    c[2] = r / g.nx[1];
+    int cand[3][3], nc[3];
+    for (int d = 0; d < 3; ++d) {
+        nc[d] = 1;
+        cand[d][0] = c[d];
+        if (d >= g.nd) continue;
+        const int n = g.nx[d];
+        if (g.bc[d][0] == TMI_PERIODIC) {
+            cand[d][nc[d]++] = c[d] - n;
+            cand[d][nc[d]++] = c[d] + n;
+        } else {
+            if (g.bc[d][0] == TMI_REFLECT && c[d] != 0) cand[d][nc[d]++] = -c[d];
+            if (g.bc[d][1] == TMI_REFLECT && c[d] != n - 1) cand[d][nc[d]++] = 2 * (n - 1) - c[d];
+        }
+    }
+    for (int a = 0; a < nc[0]; ++a)
+        for (int b = 0; b < nc[1]; ++b)
+            for (int e = 0; e < nc[2]; ++e) {
+                const int q0 = cand[0][a] + g.h[0], q1 = cand[1][b] + g.h[1], q2 = cand[2][e] + g.h[2];
+                if (q0 < 0 || q0 >= g.P[0] || q1 < 0 || q1 >= g.P[1] || q2 < 0 || q2 >= g.P[2]) continue;
+                const long long pos = (long long)q0 + (long long)q1 * g.P[0] + (long long)q2 * g.P[0] * g.P[1];
+                int src = -1, refl = 0;
+                if (map_pad(g, pos, src, refl) != 0 || src != j) continue;
+                f(q0, q1, q2, pos, refl);
+            }
+}
+template <typename F>
+__device__ inline void for_each_image(const Geo &g, int j, F &&f)
+{
+    for_each_image_at(g, j, [&](int, int, int, long long pos, int refl) { f(pos, refl); });
+}
+
 struct StenPtrs {
     const int *lo;
     const void *w;

@@ -42,6 +42,7 @@
 #include <vector>
 
 #include "tmi_device.hpp"
+#include "tmi_fmt.hpp"
 #include "tmi_internal.hpp"
 
 namespace tmi {
@@ -74,7 +75,7 @@ struct RowMap {
 // spectrum table (t >= 0: FMT table t; t < 0: attraction table -t-1), grouped by input field f,
 // terms first[f] .. first[f+1]-1
 constexpr int kMaxTerms = 64;
-constexpr int kMaxIn = kNC * 4 + 1;   // adjoint fields C(1+D)+1
+constexpr int kMaxIn = kNC * 5 + 1;   // adjoint fields C(1+D)+1 and the transpose product's C mean-field weights
 struct Term {
     int o, t, imag;
     int odd;   // axis in which the table is odd (vector delta d: d), -1 if even
@@ -120,6 +121,12 @@ struct FftPlan {
     TermList tfwd[2], tel;      // the same products as terms of the fused x pass (tel: adjoint fields
                                 // A_c, B_c,d, S3; tel_d: the derivative form, when dform)
     TermList tel_d;
+    // transpose products: the density columns (inputs: the row weights as adjoint fields, then the
+    // mean-field weights; outputs: components) and the rho-bar columns (the density product's FMT rows)
+    TermList tvr, tvb;
+    FwdDesc fvb;
+    void *vbuf = nullptr;       // their transform buffers, from the first transpose product on
+    int vz = 0, vo = 0;         // pairs of inputs and outputs in vbuf
     // rows fed by each output of the density product (fused last pass): [w][output][k]
     int onrow[2][kMaxOut] = {}, orow[2][kMaxOut][3] = {};
     double oscale[2][kMaxOut][3] = {};
@@ -321,8 +328,9 @@ __device__ __forceinline__ void nt_store(Cx<T> *p, Cx<T> v)
 // output o feeds rows row[o][0..nrow[o]) with factors scale[o][.], rho-bar
 // rows (< nrb) minus in_rb and sub_rb, mean-field rows minus in_mf and sub_mf.
 // kPassEl writes the Euler-Lagrange rows of components 2 field and 2 field + 1
-// with their local terms, as k_el_extract.
-constexpr int kPassPlain = 0, kPassGather = 1, kPassRows = 2, kPassEl = 3, kPassPc = 4;
+// with their local terms, as k_el_extract.  kPassVjp writes the density columns of the transpose
+// product: the sum (0 where Zero_density_TF) plus the A22 diagonal times the EL row's weight.
+constexpr int kPassPlain = 0, kPassGather = 1, kPassRows = 2, kPassEl = 3, kPassPc = 4, kPassVjp = 5;
 struct PassIO {
     const double *rho = nullptr;
     const unsigned char *zero = nullptr;
@@ -420,6 +428,15 @@ __device__ inline void strided_store(Cx<T> *__restrict__ data, const StridedGeo 
             if (io.add) r += io.add[row];
             io.out_el[row] = r;
             ssq += r * r;
+        }
+    } else if constexpr (MODE == kPassVjp) {
+        const int nd = strided_node(g, io, i, j);
+        for (int h = 0; h < 2; ++h) {
+            const int c = 2 * field + h;
+            if (c >= io.C) break;
+            const size_t row = (size_t)c * io.N + nd;
+            const double diag = io.elzero[row] ? 1.0 : 1.0 / io.x_rho[row];
+            io.out_el[row] = (io.zero[row] ? 0.0 : (double)(h ? v.y : v.x)) + diag * io.el_in_rho[row];
         }
     } else if constexpr (MODE == kPassPc) {
         const int nd = strided_node(g, io, i, j);
@@ -1104,12 +1121,14 @@ __global__ void k_fwd_extract(FftGeo f, Geo g, RowMap rm, const Cx<T> *__restric
 // E_c = K_delta,c A_c - sum_d (i K'_c,d) B_c,d + K_theta,c S3, packed in pairs.
 // DF: the fields are the derivatives of Phi in the rho-bar order (D3 D2 D1 D0 Dv2_d Dv1_d) and
 // A_c = D2 + D1 i4pir_c + D0 i4pirsq_c, B_c,d = Dv2_d + Dv1_d i4pir_c, S3 = D3 are formed here.
+// nmf > 0 (transpose product): fields nf .. nf + nmf - 1 are the mean-field rows' weights w_c', and
+// E_c += sum_c' U_c',c w_c'.
 struct ElConsts {
     double i4pir[kNC], i4pirsq[kNC];
 };
 template <typename T, int ND, bool DF>
 __global__ void k_el_mul(FftGeo f, int C, ElConsts ec, const Cx<T> *__restrict__ Z, const T *__restrict__ tk,
-                         Cx<T> *__restrict__ O)
+                         Cx<T> *__restrict__ O, int nmf, const T *__restrict__ uk)
 {
     const long long m = (long long)blockIdx.x * kBlock + threadIdx.x;
     if (m >= f.n) return;
@@ -1148,6 +1167,8 @@ __global__ void k_el_mul(FftGeo f, int C, ElConsts ec, const Cx<T> *__restrict__
                     B = field(c * (1 + ND) + 1 + dd);
                 e = cadd(e, Cx<T>{kv * B.y, -kv * B.x});   // -(i kv) B
             }
+            for (int cp = 0; cp < nmf; ++cp)
+                e = cadd(e, cscale(field((DF ? 4 + 2 * ND : C * (1 + ND) + 1) + cp), uk[(size_t)(cp + C * c) * f.tg.tn + ix.t]));
             if ((c & 1) == 0) {
                 acc = e;
                 if (c + 1 == C) O[(size_t)(c >> 1) * f.ns + ix.q] = acc;
@@ -1538,6 +1559,167 @@ __global__ void k_el_extract(FftGeo f, Geo g, CompConsts cc, int linear, int nwa
     out_el[row] = r;
 }
 
+// ---- transpose products (y = J(x)^T w) as spectral products.  The reversed correlations of the
+// density columns are the Euler-Lagrange product of the rows' weights (every stencil is even or odd):
+//   rho_hat_c = K_delta,c Delta_c - sum_d (i K'_c,d) V_c,d + K_theta,c Theta + sum_c' U_c',c w_mf,c'
+// with Theta = w_n3, Delta_c = w_n2 + w_n1/4piR_c + w_n0/4piR_c^2, V_c,d = w_nv2d + w_nv1d/4piR_c, and
+// those of the rho-bar columns are the rho-bar product of the EL rows' weights.  On a grid with
+// padded axes the weights are zero outside the nodes and every node collects its images' sums
+// (for_each_image); a wrapping axis has summed them already.
+// Bound by HBM and launches like the fill's passes, where the per-point reversed gather
+// (k_corr_rho) does L_u multiply-adds per padded position: 64^3 with a 71,831-point attraction
+// stencil 84.5 ms -> 0.101 ms, 256^2 rough wall (8217 points) 1.61 ms -> 0.078 ms.
+
+// Input pairs of both products at every FFT-grid point (zero off the nodes): the density columns'
+// fields (DF: the weights themselves, rho-bar order, then w_mf), then the EL rows' weights
+template <typename T, int ND>
+__global__ void k_vjp_gather(FftGeo f, Geo g, const double *__restrict__ w_rb, const double *__restrict__ w_mf, int nmf,
+                             int dform, const double *__restrict__ w_el, const unsigned char *__restrict__ elzero,
+                             CompConsts cc, Cx<T> *__restrict__ Z)
+{
+    const long long m = (long long)blockIdx.x * kBlock + threadIdx.x;
+    if (m >= f.n) return;
+    const int m0 = (int)(m % f.M[0]);
+    const long long r = m / f.M[0];
+    const int m1 = (int)(r % f.M[1]), m2 = (int)(r / f.M[1]);
+    const int x = m0 - f.off[0], y = m1 - f.off[1], z = m2 - f.off[2];
+    const bool in = x >= 0 && x < g.nx[0] && y >= 0 && y < g.nx[1] && z >= 0 && z < g.nx[2];
+    const size_t i = in ? (size_t)x + (size_t)g.nx[0] * ((size_t)y + (size_t)g.nx[1] * z) : 0, N = g.N;
+    const long long q = m0 + m1 * f.S1 + m2 * f.S2;
+    const int C = g.C, nadj = dform ? 4 + 2 * ND : C * (1 + ND) + 1, nf = nadj + nmf;
+    auto field = [&](int j) -> double {
+        if (j >= nadj) return w_mf[(size_t)(j - nadj) * N + i];
+        if (dform) return w_rb[(size_t)j * N + i];
+        if (j == C * (1 + ND)) return w_rb[i];
+        const int c = j / (1 + ND), k = j - c * (1 + ND);
+        if (k == 0) return w_rb[N + i] + cc.i4pir[c] * w_rb[2 * N + i] + cc.i4pirsq[c] * w_rb[3 * N + i];
+        return w_rb[(size_t)(3 + k) * N + i] + cc.i4pir[c] * w_rb[(size_t)(3 + ND + k) * N + i];
+    };
+    for (int j = 0; 2 * j < nf; ++j) {
+        const T re = in ? (T)field(2 * j) : (T)0;
+        const T im = (in && 2 * j + 1 < nf) ? (T)field(2 * j + 1) : (T)0;
+        Z[(size_t)j * f.ns + q] = Cx<T>{re, im};
+    }
+    Z += (size_t)((nf + 1) / 2) * f.ns;
+    for (int j = 0; 2 * j < C; ++j) {
+        const size_t a = (size_t)(2 * j) * N + i, b = a + N;
+        const T re = (in && !elzero[a]) ? (T)w_el[a] : (T)0;
+        const T im = (in && 2 * j + 1 < C && !elzero[b]) ? (T)w_el[b] : (T)0;
+        Z[(size_t)j * f.ns + q] = Cx<T>{re, im};
+    }
+}
+
+// Geometry whose images k_vjp_fold enumerates: halo h on the padded axes, none on the wrapping ones,
+// where the circular product has summed the periodic images
+inline Geo vjp_geo(const FftPlan &F, Geo g)
+{
+    for (int d = 0; d < g.nd; ++d)
+        if (F.off[d] == 0) {
+            g.h[d] = 0;
+            g.P[d] = g.nx[d];
+        }
+    g.np = (long long)g.P[0] * g.P[1] * g.P[2];
+    return g;
+}
+
+// Every column of the transpose product from the two products' outputs (O: the rho-bar product's
+// pairs, then the density columns').  gu, gf: vjp_geo of the density and FMT halos.  fold false
+// (wrapping grid): the density columns are written by the last pass (kPassVjp), the rho-bar
+// product's rows by kPassRows into y_rb.
+template <typename T, int ND, bool FOLD>
+__global__ __launch_bounds__(kBlock) void k_vjp_point(FftGeo f, Geo gu, Geo gf, int func, FwdDesc d, RowMap rm,
+                                                      const Cx<T> *__restrict__ O, const double *__restrict__ x_rho,
+                                                      const double *__restrict__ x_rb, const double *__restrict__ w_el,
+                                                      const double *__restrict__ w_rb, const double *__restrict__ w_mf,
+                                                      int nmf, const unsigned char *__restrict__ zero,
+                                                      const unsigned char *__restrict__ elzero,
+                                                      double *__restrict__ y_rho, double *y_rb, double *__restrict__ y_mf)
+{
+    const int j = blockIdx.x * kBlock + threadIdx.x;
+    if (j >= gu.N) return;
+    constexpr int NR = 4 + 2 * ND, NP = NR / 2;
+    const size_t N = gu.N;
+    const int C = gu.C;
+    double G[NR];   // the rho-bar product's rows, rho-bar order
+    if constexpr (FOLD) {
+        const int npb = (d.nout + 1) / 2;
+        double s[NR];
+#pragma unroll
+        for (int o = 0; o < NR; ++o) s[o] = 0.0;
+        for_each_image_at(gf, j, [&](int q0, int q1, int q2, long long, int refl) {
+            const long long q = (q0 + f.off[0] - gf.h[0]) + (q1 + f.off[1] - gf.h[1]) * f.S1 + (q2 + f.off[2] - gf.h[2]) * f.S2;
+#pragma unroll
+            for (int p = 0; p < NP; ++p) {
+                if (2 * p < d.nout) {
+                    const Cx<T> v = O[(size_t)p * f.ns + q];
+                    const int ka = d.kind[2 * p], kb = 2 * p + 1 < d.nout ? d.kind[2 * p + 1] : 0;
+                    s[2 * p] += (ka >= 2 && ((refl >> (ka - 2)) & 1)) ? -(double)v.x : (double)v.x;
+                    s[2 * p + 1] += (kb >= 2 && ((refl >> (kb - 2)) & 1)) ? -(double)v.y : (double)v.y;
+                }
+            }
+        });
+#pragma unroll
+        for (int q = 0; q < NR; ++q) {
+            double v = 0.0;
+#pragma unroll
+            for (int o = 0; o < NR; ++o)
+                if (o == rm.src[q]) v = s[o];
+            G[q] = v * rm.scale[q];
+        }
+        double h[kNC];
+#pragma unroll
+        for (int c = 0; c < kNC; ++c) h[c] = 0.0;
+        for_each_image_at(gu, j, [&](int q0, int q1, int q2, long long, int) {
+            const long long q = (q0 + f.off[0] - gu.h[0]) + (q1 + f.off[1] - gu.h[1]) * f.S1 + (q2 + f.off[2] - gu.h[2]) * f.S2;
+#pragma unroll
+            for (int p = 0; p < (kNC + 1) / 2; ++p) {
+                if (2 * p < C) {
+                    const Cx<T> v = O[(size_t)(npb + p) * f.ns + q];
+                    h[2 * p] += (double)v.x;
+                    h[2 * p + 1] += (double)v.y;
+                }
+            }
+        });
+#pragma unroll
+        for (int c = 0; c < kNC; ++c) {
+            if (c < C) {
+                const size_t row = (size_t)c * N + j;
+                const double diag = elzero[row] ? 1.0 : 1.0 / x_rho[row];
+                y_rho[row] = (zero[row] ? 0.0 : h[c]) + diag * w_el[row];
+            }
+        }
+    } else {
+#pragma unroll
+        for (int q = 0; q < NR; ++q) G[q] = y_rb[(size_t)q * N + j];
+    }
+    // H(n) G at node j (rho-bar order -> n order and back)
+    double n[NR], g[NR], out[NR];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        n[k] = x_rb[(size_t)(3 - k) * N + j];
+        g[k] = G[3 - k];
+    }
+#pragma unroll
+    for (int k = 0; k < ND; ++k) {
+        n[4 + k] = x_rb[(size_t)(4 + ND + k) * N + j];
+        n[4 + ND + k] = x_rb[(size_t)(4 + k) * N + j];
+        g[4 + k] = G[4 + ND + k];
+        g[4 + ND + k] = G[4 + k];
+    }
+    fmt_hvp<ND>(func, n, g, out);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) y_rb[(size_t)(3 - k) * N + j] = out[k] - w_rb[(size_t)(3 - k) * N + j];
+#pragma unroll
+    for (int k = 0; k < ND; ++k) {
+        y_rb[(size_t)(4 + ND + k) * N + j] = out[4 + k] - w_rb[(size_t)(4 + ND + k) * N + j];
+        y_rb[(size_t)(4 + k) * N + j] = out[4 + ND + k] - w_rb[(size_t)(4 + k) * N + j];
+    }
+    for (int c = 0; c < nmf; ++c) {
+        const size_t row = (size_t)c * N + j;
+        y_mf[row] = -w_mf[row] + (elzero[row] ? 0.0 : w_el[row]);
+    }
+}
+
 // Preconditioner input u_c = rho_c v_c on the free rows (0 on the zero rows), as pairs at the
 // nodes' FFT-grid positions (node + off; the rest of a padded grid is zeroed beforehand)
 __global__ void k_pc_gather(FftGeo f, Geo g, const double *__restrict__ x_rho, const double *__restrict__ v,
@@ -1802,6 +1984,8 @@ long long fft_pass(const FftPlan &F, Cx<T> *data, int nfield, int sign, int axis
                 launch_strided_reg<T, 1, kPassEl>(F, data, nfield, axis, R1, R2, s, io);
             else if (mode == kPassPc)
                 launch_strided_reg<T, 1, kPassPc>(F, data, nfield, axis, R1, R2, s, io);
+            else if (mode == kPassVjp)
+                launch_strided_reg<T, 1, kPassVjp>(F, data, nfield, axis, R1, R2, s, io);
             else
                 launch_strided_reg<T, 1, kPassPlain>(F, data, nfield, axis, R1, R2, s, io);
         }
@@ -1828,6 +2012,8 @@ long long fft_pass(const FftPlan &F, Cx<T> *data, int nfield, int sign, int axis
             go(k_fft_axis<T, 1, kPassEl>);
         else if (mode == kPassPc)
             go(k_fft_axis<T, 1, kPassPc>);
+        else if (mode == kPassVjp)
+            go(k_fft_axis<T, 1, kPassVjp>);
         else
             go(k_fft_axis<T, 1, kPassPlain>);
     }
@@ -1969,6 +2155,7 @@ void free_plan(FftPlan *F)
     if (!F) return;
     (void)hipFree(F->zbuf);
     (void)hipFree(F->obuf);
+    (void)hipFree(F->vbuf);
     (void)hipFree(F->ud);
     (void)hipFree(F->uf);
     (void)hipFree(F->td);
@@ -2164,6 +2351,29 @@ void fft_setup(Problem &P, bool mf, bool fmt)
             }
             for (int c = 0; c < C; ++c) add_term(tl, c, c * (2 + ND), 0, 1.0);   // S3: theta of every component
             close_input(tl);
+        }
+        if (fmt) {   // transpose products
+            TermList &tl = F->tvr;
+            tl = F->dform ? F->tel_d : F->tel;
+            tl.first[tl.nin + 1] = tl.first[tl.nin];
+            if (mf)
+                for (int cp = 0; cp < C; ++cp) {   // weight of mean-field row cp: U_cp,c into column c
+                    for (int c = 0; c < C; ++c) add_term(tl, c, -(cp + C * c) - 1, 0, 1.0);
+                    close_input(tl);
+                }
+            F->vz = (tl.nin + 1) / 2 + (C + 1) / 2;
+            F->fvb = F->fwd[1];
+            if (mf) F->fvb.nout -= C;   // the FMT rows alone
+            TermList &tb = F->tvb;
+            tb.nout = F->fvb.nout;
+            for (int c = 0; c < C; ++c) {
+                for (int o = 0; o < tb.nout; ++o) {
+                    const int kind = F->fvb.kind[o];
+                    if (F->fvb.coef[o][c] != 0.0) add_term(tb, o, c * (2 + ND) + kind, kind >= 2 ? 1 : 0, F->fvb.coef[o][c]);
+                }
+                close_input(tb);
+            }
+            F->vo = (tb.nout + 1) / 2 + (C + 1) / 2;
         }
         for (int w = 0; w < 2; ++w) {
             const RowMap &rm = F->rows[w];
@@ -2546,18 +2756,20 @@ void fft_el(Problem &P, bool linear, const double *x_rho, const double *in_rho, 
                 ec.i4pirsq[c] = P.bulk.inv_4pirsq[c];
             }
             const long long nthr = F.fold ? group8_count(F) : F.n;
-            auto go = [&](auto kernel) {
-                hipLaunchKernelGGL(kernel, dim3(grid_for(nthr)), dim3(kBlock), 0, s, fg, C, ec, Z, fmt_spectra<T>(F), O);
+            auto go = [&](auto kernel, auto... more) {
+                hipLaunchKernelGGL(kernel, dim3(grid_for(nthr)), dim3(kBlock), 0, s, fg, C, ec, Z, fmt_spectra<T>(F), O,
+                                   more...);
             };
+            const T *no_uk = nullptr;
             if (F.fold) {
                 if (nd == 2)
                     df ? go(k_el_mul8<T, 2, true>) : go(k_el_mul8<T, 2, false>);
                 else
                     df ? go(k_el_mul8<T, 3, true>) : go(k_el_mul8<T, 3, false>);
             } else if (nd == 2) {
-                df ? go(k_el_mul<T, 2, true>) : go(k_el_mul<T, 2, false>);
+                df ? go(k_el_mul<T, 2, true>, 0, no_uk) : go(k_el_mul<T, 2, false>, 0, no_uk);
             } else {
-                df ? go(k_el_mul<T, 3, true>) : go(k_el_mul<T, 3, false>);
+                df ? go(k_el_mul<T, 3, true>, 0, no_uk) : go(k_el_mul<T, 3, false>, 0, no_uk);
             }
             fft_pass<T>(F, O, nop, +1, 0, s);
         }
@@ -2578,6 +2790,112 @@ template void fft_el<double>(Problem &, bool, const double *, const double *, co
                              hipStream_t, double *, long long *);
 template void fft_el<float>(Problem &, bool, const double *, const double *, const double *, const double *, double *,
                             hipStream_t, double *, long long *);
+
+// y = J(x)^T w as spectral products (w, y: node rows of the internal layout).  Both products share
+// their z and y passes.  False where the plan lacks a spectrum (the caller then runs the gathers).
+template <typename T>
+bool fft_vjp(Problem &P, const double *x, const double *w, double *y, hipStream_t s)
+{
+    if (!P.fft || !P.fft->fmt_ok || (P.nmf > 0 && !P.fft->mf)) return false;
+    FftPlan &F = *P.fft;
+    const size_t N = P.N;
+    const int C = P.p.ncomp, nd = P.p.ndim;
+    if (!F.vbuf) TMI_HIP_CHECK(hipMalloc(&F.vbuf, (size_t)(F.vz + F.vo) * F.ns * sizeof(Cx<double>)));
+    const int nic = (C + 1) / 2, nir = F.vz - nic, nob = F.vo - nic;   // pairs: EL weights, density columns' fields, rho-bar outputs
+    Cx<T> *Z = reinterpret_cast<Cx<T> *>(F.vbuf), *O = Z + (size_t)F.vz * F.ns;
+    Cx<T> *Ze = Z + (size_t)nir * F.ns, *Or = O + (size_t)nob * F.ns;
+    const FftGeo fg = fft_geo(F, 0);
+    const Geo gu = vjp_geo(F, make_geo(P, P.pad_u)), gf = vjp_geo(F, make_geo(P, P.pad_f));
+    const CompConsts cc = make_consts(P);
+    const double *w_el = w + (size_t)P.iu_rho * N, *w_rb = w + (size_t)P.iu_rb * N;
+    const double *w_mf = P.nmf ? w + (size_t)P.iu_mf * N : nullptr;
+    const double *x_rho = x + (size_t)P.iu_rho * N, *x_rb = x + (size_t)P.iu_rb * N;
+    double *y_rho = y + (size_t)P.iu_rho * N, *y_rb = y + (size_t)P.iu_rb * N;
+    double *y_mf = P.nmf ? y + (size_t)P.iu_mf * N : nullptr;
+    const int df = F.dform ? 1 : 0;
+    auto by_nd = [&](auto &&fn) {
+        if (nd == 2)
+            fn(std::integral_constant<int, 2>{});
+        else
+            fn(std::integral_constant<int, 3>{});
+    };
+    by_nd([&](auto d) {
+        constexpr int ND = decltype(d)::value;
+        hipLaunchKernelGGL((k_vjp_gather<T, ND>), dim3(grid_for(F.n)), dim3(kBlock), 0, s, fg, gu, w_rb, w_mf, P.nmf, df, w_el,
+                           P.d_elzero, cc, Z);
+    });
+    fft_pass<T>(F, Z, F.vz, -1, 2, s);
+    fft_pass<T>(F, Z, F.vz, -1, 1, s);
+    // the fused x pass where the fill uses it, or where it fits when the fill runs the direct sums
+    const int lpb_b = F.fmt ? F.xlpb[0] : F.xfit[0], lpb_r = F.fmt ? F.xlpb[1] : F.xfit[1];
+    if (lpb_r) {
+        fft_xprod<T>(F, Z, Or, F.tvr, lpb_r, fmt_spectra<T>(F), attr_spectra<T>(F), s);
+    } else {
+        fft_pass<T>(F, Z, nir, -1, 0, s);
+        ElConsts ec{};
+        for (int c = 0; c < C; ++c) {
+            ec.i4pir[c] = P.bulk.inv_4pir[c];
+            ec.i4pirsq[c] = P.bulk.inv_4pirsq[c];
+        }
+        by_nd([&](auto d) {
+            constexpr int ND = decltype(d)::value;
+            auto go = [&](auto kernel) {
+                hipLaunchKernelGGL(kernel, dim3(grid_for(F.n)), dim3(kBlock), 0, s, fg, C, ec, Z, fmt_spectra<T>(F), Or,
+                                   P.nmf, attr_spectra<T>(F));
+            };
+            df ? go(k_el_mul<T, ND, true>) : go(k_el_mul<T, ND, false>);
+        });
+        fft_pass<T>(F, Or, nic, +1, 0, s);
+    }
+    if (lpb_b) {
+        fft_xprod<T>(F, Ze, O, F.tvb, lpb_b, fmt_spectra<T>(F), attr_spectra<T>(F), s);
+    } else {
+        fft_pass<T>(F, Ze, nic, -1, 0, s);
+        by_nd([&](auto d) {
+            constexpr int ND = decltype(d)::value;
+            if (F.fold)
+                hipLaunchKernelGGL((k_fwd_mul4<T, ND>), dim3((unsigned)grid_for(group4_threads(group8_count(F)))), dim3(kBlock),
+                                   0, s, fg, F.fvb, Ze, fmt_spectra<T>(F), attr_spectra<T>(F), O);
+            else
+                hipLaunchKernelGGL((k_fwd_mul<T, ND>), dim3(grid_for(F.n)), dim3(kBlock), 0, s, fg, F.fvb, Ze,
+                                   fmt_spectra<T>(F), attr_spectra<T>(F), O);
+        });
+        fft_pass<T>(F, O, nob, +1, 0, s);
+    }
+    if (F.wraps) {
+        PassIO ib = rows_io(P, 1, nullptr, nullptr, nullptr, y_rb, nullptr, nullptr, nullptr);
+        ib.nout = F.fvb.nout;
+        PassIO ir;
+        ir.C = C;
+        ir.nx0 = P.p.nx[0];
+        ir.nx1 = P.p.nx[1];
+        ir.N = P.N;
+        ir.x_rho = x_rho;
+        ir.el_in_rho = w_el;
+        ir.zero = P.d_zero;
+        ir.elzero = P.d_elzero;
+        ir.out_el = y_rho;
+        const int last = F.M[2] > 1 ? 2 : 1;
+        if (last == 2) fft_pass<T>(F, O, F.vo, +1, 1, s);
+        fft_pass<T>(F, O, nob, +1, last, s, kPassRows, ib);
+        fft_pass<T>(F, Or, nic, +1, last, s, kPassVjp, ir);
+    } else {
+        fft_pass<T>(F, O, F.vo, +1, 1, s);
+        fft_pass<T>(F, O, F.vo, +1, 2, s);
+    }
+    by_nd([&](auto d) {
+        constexpr int ND = decltype(d)::value;
+        auto go = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3(grid_for(P.N)), dim3(kBlock), 0, s, fg, gu, gf, P.p.type_func, F.fvb, F.rows[1],
+                               O, x_rho, x_rb, w_el, w_rb, w_mf, P.nmf, P.d_zero, P.d_elzero, y_rho, y_rb, y_mf);
+        };
+        F.wraps ? go(k_vjp_point<T, ND, false>) : go(k_vjp_point<T, ND, true>);
+    });
+    TMI_HIP_CHECK(hipGetLastError());
+    return true;
+}
+template bool fft_vjp<double>(Problem &, const double *, const double *, double *, hipStream_t);
+template bool fft_vjp<float>(Problem &, const double *, const double *, double *, hipStream_t);
 
 // Times one kernel family of a residual fill in FFT form on the plan's work
 // buffers, in the fill's order and batch sizes, with HIP events on s.
