@@ -221,3 +221,19 @@ def test_batch_2d_newton_matches_single_solves(graph, small2d, monkeypatch):
         assert dp.newton(xs, resid_tol=1e-11, gmres_tol=1e-10, gmres_restart=100, gmres_max_iter=2000,
                          max_iter=60)["converged"]
         assert np.abs(xp[: p.ncomp] - xs.cpu().numpy()[: p.ncomp]).max() < 1e-8
+
+
+@pytest.mark.gpu
+def test_batch_newton_ignores_unwritten_basis_vectors():
+    """The Krylov basis is allocated uninitialised: vectors past a cycle's steps must not enter the
+    solution, whatever their memory held before (here NaN, left by freed tensors)."""
+    from tramonto_amd.batch import DeviceBatch
+    b = slit_pore_batch(npores=3, seed=3, h_range=(3.0, 4.0))
+    junk = [torch.full((4 << 20,), float("nan"), dtype=torch.float64, device="cuda") for _ in range(24)]
+    torch.cuda.synchronize()
+    del junk
+    torch.cuda.empty_cache()
+    db = DeviceBatch(b)
+    x = db.initial_state()
+    st = db.newton(x, resid_tol=1e-10, gmres_tol=1e-9, max_iter=60)
+    assert st["converged"], st

@@ -1,0 +1,93 @@
+"""1D rows in one launch (k_line) against the separate row kernels (TMI_LINE1D=0).
+
+Tolerance: the same FP64 (FP32) products summed in another order, at most a few hundred terms per row:
+1e-12 (1e-5) of the row block's largest value, the parity bounds of the row kernels themselves.
+"""
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+
+from tramonto_amd.batch import DeviceBatch, slit_pore_batch  # noqa: E402
+from tramonto_amd.device import DeviceProblem  # noqa: E402
+from tramonto_amd.problem import (FMT3, IN_BULK, IN_WALL, PERIODIC, REFLECT, hard_wall_1d, slit_pore_1d,  # noqa: E402
+                                  small_case)
+
+
+def _single(kind):
+    if kind == "periodic":   # images one period away on both sides, a span shorter than the attraction's reach
+        sp = slit_pore_1d(H=2.0, dx=0.02, cut_fac=0.99, seed=3)
+        sp.bc, sp.nwall, sp.vext, sp.zero_tf = [[PERIODIC, PERIODIC]], 0, None, None
+        sp.rho0 = np.maximum(sp.rho0, 0.05)
+        return sp
+    if kind in ("reflect", "reflect_bulk", "reflect_hs"):   # the last: no attraction, the FMT halo twice the density halo
+        sp = hard_wall_1d(seed=4, size=3.15 if kind != "reflect_bulk" else 9.6, dx=0.05, rho_b=0.5)
+        sp.bc = [[REFLECT, REFLECT]] if kind == "reflect" else [[IN_BULK, REFLECT]]
+        sp.nwall, sp.vext, sp.zero_tf = 0, None, None
+        sp.rho0 = np.maximum(sp.rho0, 0.3)
+        if kind != "reflect_hs":
+            sp.type_attr, sp.eps_ff, sp.cut_ff = 0, np.full((1, 1), 0.8), np.full((1, 1), 2.5)
+        return sp
+    if kind == "three":   # three components, White Bear
+        sp = slit_pore_1d(H=7.3, dx=0.05, sig=(1.0, 0.9, 0.7), rho_b=(0.1, 0.1, 0.1), seed=5)
+        sp.type_func = FMT3
+        return sp
+    if kind == "long2":
+        return hard_wall_1d(seed=6, size=0.05 * 20000, dx=0.05, rho_b=0.6)
+    if kind == "long4":
+        return slit_pore_1d(H=0.05 * 40001, dx=0.05, seed=7)
+    return small_case(kind)
+
+
+def _problems(make, monkeypatch):
+    monkeypatch.setenv("TMI_AUTOTUNE", "0")
+    monkeypatch.setenv("TMI_LINE1D", "0")
+    a = make()
+    monkeypatch.setenv("TMI_LINE1D", "1")
+    return a, make()
+
+
+def _compare(a, b, blocks, tol):
+    for lo, hi in blocks:
+        if lo < hi:
+            scale = float(a[lo:hi].abs().max())
+            assert float((a[lo:hi] - b[lo:hi]).abs().max()) <= tol * scale, (lo, hi)
+
+
+KINDS = ["1d_hw", "1d_reflect_wca", "1d_pore_mix", "1d_reflect_slab", "periodic", "reflect", "reflect_bulk", "reflect_hs",
+         "three", "long2", "long4", "batch_small", "batch_large"]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", KINDS)
+def test_line_matches_row_kernels(kind, monkeypatch):
+    batch = kind.startswith("batch")
+    if batch:
+        spec = slit_pore_batch(npores=3 if kind == "batch_small" else 60, seed=2)
+        rows, line = _problems(lambda: DeviceBatch(spec), monkeypatch)
+    else:
+        spec = _single(kind)
+        rows, line = _problems(lambda: DeviceProblem(spec), monkeypatch)
+    C = spec.ncomp
+    R = 6
+    x = rows.initial_state()
+    blocks = ((0, C), (C, C + R), (C + R, x.shape[0]))
+    _compare(x, line.initial_state(), blocks, 1e-12)
+    g = torch.Generator(device="cuda").manual_seed(1)
+    noise = lambda: 2 * torch.rand(x.shape, generator=g, device="cuda", dtype=torch.float64) - 1   # noqa: E731
+    x[C:] *= 1.0 + 0.01 * noise()[C:]
+    Fa, sa = rows.fill_residual(x)
+    Fb, sb = line.fill_residual(x)
+    _compare(Fa, Fb, blocks, 1e-12)
+    assert abs(sa - sb) <= 1e-12 * abs(sa)
+    dev = torch.zeros(1, dtype=torch.float64, device="cuda")
+    line.fill_residual_device_norm(x, Fb, dev)
+    _compare(Fa, Fb, blocks, 1e-12)
+    assert abs(float(dev) - sa) <= 1e-12 * abs(sa)
+    v = noise()
+    _compare(rows.apply_jacobian(x, v), line.apply_jacobian(x, v), blocks, 1e-12)
+    _compare(rows.apply_jacobian(x, v, fp32=True), line.apply_jacobian(x, v, fp32=True), blocks, 1e-5)
+    if not batch:   # Schur product, right-hand side and back-substitution: one Newton update
+        da, _ = rows.schur_solve(x, Fa, rtol=1e-12)
+        db, _ = line.schur_solve(x, Fa, rtol=1e-12)
+        _compare(da, db, blocks, 1e-8)

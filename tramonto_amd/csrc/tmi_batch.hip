@@ -100,14 +100,17 @@ __global__ __launch_bounds__(kSegBlock) void k_seg_dots(const double *__restrict
     }
 }
 
-// w[e] += alpha * sum_j V_j[e] coef[pore(e)][j]
+// w[e] += alpha * sum_j V_j[e] coef[pore(e)][j], over the first k vectors or (kp set) the first
+// kp[pore(e)]: a basis vector past a pore's steps may never have been written
 __global__ void k_seg_gemv(const double *__restrict__ V, long long ldv, int k, const double *__restrict__ coef, int ldc,
-                           double alpha, double *__restrict__ w, int rows, int N, const int *__restrict__ pore_of)
+                           double alpha, double *__restrict__ w, int rows, int N, const int *__restrict__ pore_of,
+                           const int *__restrict__ kp)
 {
     const long long e = (long long)blockIdx.x * kBlock + threadIdx.x;
     if (e >= (long long)rows * N) return;
     const int i = (int)(e % N);
     const double *c = coef + (size_t)pore_of[i] * ldc;
+    if (kp) k = kp[pore_of[i]];
     double s = 0.0;
     for (int j = 0; j < k; ++j) s += V[(size_t)j * ldv + e] * c[j];
     w[e] += alpha * s;
@@ -492,11 +495,11 @@ static void stage_cycle_steps(Problem &P, BatchWork &W, const double *x, double 
         hipLaunchKernelGGL(k_seg_dots, dim3(Pn), dim3(kSegBlock), 0, s, W.V, n2, k + 1, W.w, C, N, P.d_pore_off,
                            W.gs.h1, m + 1);
         hipLaunchKernelGGL(k_seg_gemv, dim3(nblk(n2)), dim3(kBlock), 0, s, W.V, n2, k + 1, W.gs.h1, m + 1, -1.0, W.w,
-                           C, N, P.d_pore_of);
+                           C, N, P.d_pore_of, nullptr);
         hipLaunchKernelGGL(k_seg_dots, dim3(Pn), dim3(kSegBlock), 0, s, W.V, n2, k + 1, W.w, C, N, P.d_pore_off,
                            W.gs.h2, m + 1);
         hipLaunchKernelGGL(k_seg_gemv, dim3(nblk(n2)), dim3(kBlock), 0, s, W.V, n2, k + 1, W.gs.h2, m + 1, -1.0, W.w,
-                           C, N, P.d_pore_of);
+                           C, N, P.d_pore_of, nullptr);
         hipLaunchKernelGGL(k_seg_normalize, dim3(Pn), dim3(kSegBlock), 0, s, W.w, W.V + (size_t)(k + 1) * n2, C, N,
                            P.d_pore_off, W.gs.hn);
         hipLaunchKernelGGL(k_gmres_givens, dim3(nblk(Pn)), dim3(kBlock), 0, s, Pn, k, W.gs, tol);
@@ -510,10 +513,10 @@ static void stage_cycle_finish(Problem &P, BatchWork &W, hipStream_t s)
     const int Pn = W.P, C = P.p.ncomp, N = P.N, m = W.m;
     const long long n2 = (long long)W.n2;
     hipLaunchKernelGGL(k_gmres_solve, dim3(nblk(Pn)), dim3(kBlock), 0, s, Pn, W.gs);
-    // x2 += dinv * (V y); y is zero beyond each pore's steps
+    // x2 += dinv * (V y) over each pore's steps
     hipLaunchKernelGGL(k_fill, dim3(nblk(n2)), dim3(kBlock), 0, s, W.z, 0.0, n2);
     hipLaunchKernelGGL(k_seg_gemv, dim3(nblk(n2)), dim3(kBlock), 0, s, W.V, n2, m, W.gs.y, m, 1.0, W.z, C, N,
-                       P.d_pore_of);
+                       P.d_pore_of, W.gs.kdone);
     dev_mul(W.dinv, W.z, W.w, n2, s);
     dev_axpy(1.0, W.w, W.dx, n2, s);
     TMI_HIP_CHECK(hipGetLastError());

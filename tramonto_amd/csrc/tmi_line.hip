@@ -1,0 +1,527 @@
+// The stencil rows of 1D problems and batches of 1D pores in one launch.
+//
+// A 1D fill is six dependent-looking launches (density halo, rho-bar rows, mean-field rows,
+// pointwise derivatives, adjoint halo, Euler-Lagrange rows) of a few microseconds each, and its
+// kernels leave most SIMDs with one wave that waits for its own loads.  Here one workgroup owns TN
+// consecutive padded positions, keeps the densities and the adjoint fields of its span (halos
+// included) in LDS, and its waves share out the stencil sums: one (stencil, component, span) sum per
+// wave at a time, so that the long attraction sums and the short FMT ones run side by side.
+//  * Residual and Jacobian-vector product: the rows and the Euler-Lagrange sums depend on the
+//    inputs alone, so both run in the same pass.
+//  * Schur product (CHAIN): the rho-bar sums are formed on the span and its FMT halo (recomputed by
+//    the neighbours), become adjoint fields in LDS, and feed the Euler-Lagrange sums: no row leaves
+//    the chip.
+// Each lane owns B consecutive outputs and reads B densities per step, so every LDS read feeds B
+// multiply-adds per stencil against weights in scalar registers; at B = 4 the LDS reads (16 cycles a
+// wave for 4 positions) and the FP64 multiply-adds (64 cycles) balance.  Small problems are bound by
+// latency and take B = 1 and 64 positions a workgroup, which puts 401 nodes on 7 CUs instead of 1.
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <type_traits>
+
+#include "tmi_device.hpp"
+#include "tmi_fmt.hpp"
+#include "tmi_internal.hpp"
+
+namespace tmi {
+namespace {
+
+using namespace dev;
+
+constexpr int kLineWaves = 8;
+constexpr int kLineBlock = 64 * kLineWaves;
+constexpr int kLineSlack = 16;           // zero positions past each LDS row (whole steps read past the span)
+constexpr size_t kLineLds = 64 * 1024;   // dynamic LDS of a launch
+
+template <typename T>
+struct LineRow {
+    const T *w, *wv;
+    int lo0, L;
+};
+
+template <typename T>
+struct LineArgs {
+    Geo g;   // the density geometry; the adjoint fields use its positions too (its gaps are at least the FMT halo)
+    LineRow<T> th[kNC], de[kNC], u[kNC * kNC];
+    CompConsts cc;
+    int TN, hr, hf;   // positions per workgroup, density halo in LDS, FMT halo
+    int rho_ld, rb_ld, mf_ld, adj_ld;   // LDS row lengths
+    int nmf, func, nwall;
+    const double *rho, *mul;   // densities or direction [C][N] (null: no rows), optional factor
+    const unsigned char *zero, *elzero;
+    const double *in_rb, *sub_rb, *in_mf, *sub_mf;
+    double *out_rb, *out_mf;
+    const double *x_rb, *dn_rb, *x_rho, *in_rho, *el_mf, *vext, *add;
+    double *out_el;            // null: no Euler-Lagrange rows
+    double *ss;                // optional: the workgroup's sum of squares of the rows written
+    const int *done, *pore_of; // optional: skip a workgroup all of whose pores are done
+};
+
+// code and source node of padded position q, which may lie outside the padded copy (map_pad in 1D)
+__device__ inline int line_map(const Geo &g, int q, int &src, int &refl)
+{
+    refl = 0;
+    if (g.pad_node) {
+        src = (q >= 0 && q < (int)g.np) ? g.pad_node[q] : -1;
+        return src >= 0 ? 0 : -2;
+    }
+    const int n = g.nx[0];
+    int v = q - g.h[0];
+    if (v >= 0 && v < n) {
+        src = v;
+        return 0;
+    }
+    const int side = v < 0 ? 0 : 1, b = g.bc[0][side];
+    if (b == TMI_IN_BULK) return -1;
+    if (b == TMI_IN_WALL) return -2;
+    if (b == TMI_PERIODIC) {
+        v += side ? -n : n;
+        if (v < 0 || v >= n) return -2;   // further than one period: read by no output
+    } else {
+        refl = 1;
+        v = side ? 2 * (n - 1) - v : -v;
+        if (v < 0 || v >= n) return g.bc[0][1 - side] == TMI_IN_BULK ? -1 : -2;
+    }
+    src = v;
+    return 0;
+}
+
+// B consecutive LDS values, 16-byte aligned where B values fill 16 bytes
+template <typename T, int B>
+__device__ __forceinline__ void lds_read(const T *p, T (&v)[B])
+{
+    typedef T VB __attribute__((ext_vector_type(B)));
+    const VB t = *reinterpret_cast<const VB *>(p);
+#pragma unroll
+    for (int i = 0; i < B; ++i) v[i] = t[i];
+}
+template <typename T>
+__device__ __forceinline__ void lds_read(const T *p, T (&v)[1])
+{
+    v[0] = *p;
+}
+
+// acc[s][b] += sum_j w_s[j] row[a0 + b + j] for NS weight rows of one stencil (row: LDS, a0: the
+// lane's first position plus the stencil's first offset, a multiple of B apart between lanes)
+template <typename T, int B, int NS>
+__device__ __forceinline__ void line_sum(const T *row, int a0, int lane_a, const T *__restrict__ w0,
+                                         const T *__restrict__ w1, int L, T (&acc)[NS][B])
+{
+    const int sh = a0 & (B - 1);   // wave-uniform: reads start on a multiple of B
+    const T *src = row + (a0 - sh) + lane_a;
+    const int back = kRowPad - sh - (B - 1);
+    const T *w[2] = {w0 + back, NS > 1 ? w1 + back : w0 + back};
+    const int nk = (L + sh + 2 * B - 2) / B;
+    for (int k = 0; k < nk; ++k) {
+        T v[B];
+        lds_read(src + k * B, v);
+#pragma unroll
+        for (int s = 0; s < NS; ++s) {
+            T wk[2 * B - 1];
+#pragma unroll
+            for (int j = 0; j < 2 * B - 1; ++j) wk[j] = w[s][k * B + j];
+#pragma unroll
+            for (int i = 0; i < B; ++i)
+#pragma unroll
+                for (int b = 0; b < B; ++b) acc[s][b] += wk[i - b + B - 1] * v[i];
+        }
+    }
+}
+
+// adjoint fields A_c, B_c (c < C), S3 of node src's derivatives (dn: the linear modes' direction)
+template <typename T, bool LINEAR>
+__device__ inline void line_adjoint(const Geo &g, const CompConsts &cc, int func, const double *__restrict__ x_rb, int src,
+                                    const double *dr, int refl, T *out, int ld)
+{
+    double n[6], o[6];
+    const size_t N = g.N;
+    n[3] = x_rb[src];
+    n[2] = x_rb[N + src];
+    n[1] = x_rb[2 * N + src];
+    n[0] = x_rb[3 * N + src];
+    n[5] = x_rb[4 * N + src];
+    n[4] = x_rb[5 * N + src];
+    if constexpr (LINEAR) {
+        const double dn[6] = {dr[3], dr[2], dr[1], dr[0], dr[5], dr[4]};
+        fmt_hvp<1>(func, n, dn, o);
+    } else {
+        fmt_dphi<1>(func, n, o);
+    }
+    for (int c = 0; c < g.C; ++c) {
+        out[(2 * c) * ld] = (T)(o[0] * cc.i4pirsq[c] + o[1] * cc.i4pir[c] + o[2]);
+        const T b = (T)(o[4] * cc.i4pir[c] + o[5]);
+        out[(2 * c + 1) * ld] = refl ? -b : b;
+    }
+    out[2 * g.C * ld] = (T)o[3];
+}
+
+template <typename T, int B, bool CHAIN, bool LINEAR>
+__global__ __launch_bounds__(kLineBlock) void k_line(LineArgs<T> a)
+{
+    extern __shared__ __attribute__((aligned(32))) char smem_raw[];
+    const Geo &g = a.g;
+    const int C = g.C, TN = a.TN, hf = a.hf, hr = a.hr;
+    const size_t N = g.N;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int p0 = g.h[0] + (int)blockIdx.x * TN;   // first position of the span
+    if (a.done) {
+        int live = 0;
+        for (int t = tid; t < TN; t += kLineBlock) {
+            int src, refl;
+            if (line_map(g, p0 + t, src, refl) == 0 && !a.done[a.pore_of[src]]) live = 1;
+        }
+        if (!__syncthreads_or(live)) return;
+    }
+    const int rb_n = CHAIN ? TN + 2 * hf : TN, adj_n = TN + 2 * hf, ext = CHAIN ? hf : 0;
+    T *rho = reinterpret_cast<T *>(smem_raw);               // [C][rho_ld]
+    T *adj = rho + (a.rho ? C * a.rho_ld : 0);              // [2 C + 1][adj_ld]
+    T *srb = adj + (a.out_el ? (2 * C + 1) * a.adj_ld : 0); // [C][3][rb_ld]: theta, delta, vector delta
+    T *smf = srb + (a.rho ? 3 * C * a.rb_ld : 0);           // [C][C][mf_ld]
+    T *sel = CHAIN ? srb : smf + (a.rho && a.nmf ? C * C * a.mf_ld : 0);   // [C][3][mf_ld]
+    // densities with their halo
+    if (a.rho) {
+        for (int r = tid; r < a.rho_ld; r += kLineBlock) {
+            int src = 0, refl = 0, code = -2;
+            if (r < TN + 2 * hr) code = line_map(g, p0 - hr + r, src, refl);
+            for (int c = 0; c < C; ++c) {
+                double v = 0.0;
+                if (code == 0) {
+                    const size_t q = (size_t)c * N + src;
+                    v = a.zero[q] ? 0.0 : a.rho[q] * (a.mul ? a.mul[q] : 1.0);
+                } else if (code == -1 && !LINEAR) {
+                    v = a.cc.rho_b[c];
+                }
+                rho[c * a.rho_ld + r] = (T)v;
+            }
+        }
+    }
+    // adjoint fields with their halo
+    auto adjoint_halo = [&](int r, int code) {   // no node: bulk or wall values
+        const bool bulk = code == -1 && !LINEAR;
+        for (int c = 0; c < C; ++c) {
+            adj[(2 * c) * a.adj_ld + r] = bulk ? (T)a.cc.Ab[c] : (T)0;
+            adj[(2 * c + 1) * a.adj_ld + r] = (T)0;
+        }
+        adj[2 * C * a.adj_ld + r] = bulk ? (T)a.cc.S3b : (T)0;
+    };
+    if (!CHAIN && a.out_el) {
+        for (int r = tid; r < a.adj_ld; r += kLineBlock) {
+            int src = 0, refl = 0, code = -2;
+            if (r < adj_n) code = line_map(g, p0 - hf + r, src, refl);
+            if (code == 0) {
+                double dr[6];
+                if constexpr (LINEAR) {
+#pragma unroll
+                    for (int q = 0; q < 6; ++q) dr[q] = a.dn_rb[(size_t)q * N + src];
+                }
+                line_adjoint<T, LINEAR>(g, a.cc, a.func, a.x_rb, src, dr, refl, adj + r, a.adj_ld);
+            } else {
+                adjoint_halo(r, code);
+            }
+        }
+    }
+    __syncthreads();
+    // stencil sums, one item per wave at a time, the longest first
+    constexpr int W = 64 * B;
+    const int nt = (TN + W - 1) / W, ntr = (rb_n + W - 1) / W;
+    const int n_mf = a.rho && a.nmf ? C * C * nt : 0, n_rb = a.rho ? C * ntr : 0, n_el = !CHAIN && a.out_el ? C * nt : 0;
+    auto put = [&](T *row, int t0, int n, const T (&v)[B]) {
+#pragma unroll
+        for (int b = 0; b < B; ++b)
+            if (t0 + lane * B + b < n) row[t0 + lane * B + b] = v[b];
+    };
+    auto el_item = [&](int it) {   // three items per component and span: delta A, vector delta B, theta S3
+        const int kind = it % 3, t = (it / 3) % nt, c = it / (3 * nt);
+        const LineRow<T> st = kind == 2 ? a.th[c] : a.de[c];
+        const T *row = adj + (kind == 2 ? 2 * C : 2 * c + kind) * a.adj_ld;
+        T acc[1][B] = {};
+        line_sum<T, B, 1>(row, t * W + hf + st.lo0, lane * B, kind == 1 ? st.wv : st.w, nullptr, st.L, acc);
+        put(sel + (3 * c + kind) * a.mf_ld, t * W, TN, acc[0]);
+    };
+    for (int it = wave; it < n_mf + 2 * n_rb + 3 * n_el; it += kLineWaves) {
+        if (it < n_mf) {
+            const int t = it % nt, q = it / nt, c = q / C, cj = q - c * C;
+            const LineRow<T> u = a.u[c + C * cj];
+            T acc[1][B] = {};
+            line_sum<T, B, 1>(rho + cj * a.rho_ld, t * W + hr + u.lo0, lane * B, u.w, nullptr, u.L, acc);
+            put(smf + q * a.mf_ld, t * W, TN, acc[0]);
+        } else if (it < n_mf + 2 * n_rb) {
+            const int j = it - n_mf, th = j >= n_rb, q = th ? j - n_rb : j, t = q % ntr, c = q / ntr;
+            if (th) {
+                const LineRow<T> st = a.th[c];
+                T acc[1][B] = {};
+                line_sum<T, B, 1>(rho + c * a.rho_ld, t * W - ext + hr + st.lo0, lane * B, st.w, nullptr, st.L, acc);
+                put(srb + (3 * c) * a.rb_ld, t * W, rb_n, acc[0]);
+            } else {
+                const LineRow<T> st = a.de[c];
+                T acc[2][B] = {};
+                line_sum<T, B, 2>(rho + c * a.rho_ld, t * W - ext + hr + st.lo0, lane * B, st.w, st.wv, st.L, acc);
+                put(srb + (3 * c + 1) * a.rb_ld, t * W, rb_n, acc[0]);
+                put(srb + (3 * c + 2) * a.rb_ld, t * W, rb_n, acc[1]);
+            }
+        } else {
+            el_item(it - n_mf - 2 * n_rb);
+        }
+    }
+    __syncthreads();
+    // the rho-bar values at index r of the sums, solution order
+    auto rb_vals = [&](int r, double (&vals)[6]) {
+        T n3 = 0, n2 = 0, n1 = 0, n0 = 0, v2 = 0, v1 = 0;
+        for (int c = 0; c < C; ++c) {
+            const T st = srb[(3 * c) * a.rb_ld + r], sd = srb[(3 * c + 1) * a.rb_ld + r], sv = srb[(3 * c + 2) * a.rb_ld + r];
+            n3 += st;
+            n2 += sd;
+            n1 += (T)a.cc.i4pir[c] * sd;
+            n0 += (T)a.cc.i4pirsq[c] * sd;
+            v2 += sv;
+            v1 += (T)a.cc.i4pir[c] * sv;
+        }
+        vals[0] = n3;
+        vals[1] = n2;
+        vals[2] = n1;
+        vals[3] = n0;
+        vals[4] = v2;
+        vals[5] = v1;
+    };
+    if constexpr (CHAIN) {
+        for (int r = tid; r < a.adj_ld; r += kLineBlock) {
+            int src = 0, refl = 0, code = -2;
+            if (r < adj_n) code = line_map(g, p0 - hf + r, src, refl);
+            // across a mirror the node's own sums; a mirror node outside the span serves no output here
+            const int rs = refl ? src + g.h[0] - (p0 - hf) : r;
+            if (code == 0 && rs >= 0 && rs < rb_n) {
+                double dr[6];
+                rb_vals(rs, dr);
+                line_adjoint<T, true>(g, a.cc, a.func, a.x_rb, src, dr, refl, adj + r, a.adj_ld);
+            } else {
+                adjoint_halo(r, code == 0 ? -2 : code);
+            }
+        }
+        __syncthreads();
+        for (int it = wave; it < 3 * C * nt; it += kLineWaves) el_item(it);
+        __syncthreads();
+    }
+    // rows
+    double ssq = 0.0;
+    for (int t = tid; t < TN; t += kLineBlock) {
+        int i = -1, refl = 0;
+        if (line_map(g, p0 + t, i, refl) != 0 || p0 + t >= g.P[0] - g.h[0]) continue;
+        if (!CHAIN && a.rho) {
+            if (a.out_rb) {
+                double vals[6];
+                rb_vals(t, vals);
+#pragma unroll
+                for (int r = 0; r < 6; ++r) {
+                    double o = vals[r];
+                    if (a.in_rb) o -= a.in_rb[(size_t)r * N + i];
+                    if (a.sub_rb) o -= a.sub_rb[(size_t)r * N + i];
+                    a.out_rb[(size_t)r * N + i] = o;
+                    ssq += o * o;
+                }
+            }
+        }
+        for (int c = 0; c < C; ++c) {
+            const size_t row = (size_t)c * N + i;
+            T mf = 0;
+            if (a.rho && a.nmf)
+                for (int cj = 0; cj < C; ++cj) mf += smf[(c * C + cj) * a.mf_ld + t];
+            if (!CHAIN && a.rho && a.nmf) {
+                double o = (double)mf;
+                if (a.in_mf) o -= a.in_mf[row];
+                if (a.sub_mf) o -= a.sub_mf[row];
+                a.out_mf[row] = o;
+                ssq += o * o;
+            }
+            if (a.out_el) {
+                const double in = a.in_rho ? a.in_rho[row] * (a.mul ? a.mul[row] : 1.0) : 0.0;
+                double r;
+                if (a.elzero[row]) {
+                    r = in;
+                } else {
+                    const T *s = sel + 3 * c * a.mf_ld + t;
+                    r = (double)(s[2 * a.mf_ld] + s[0] - s[a.mf_ld]);
+                    const double xv = a.x_rho[row];
+                    if constexpr (!LINEAR) {
+                        r += log(xv) + (g.mu ? g.mu[row] : a.cc.mu[c]);
+                        if (a.nwall > 0) r += a.vext[row];
+                        if (a.el_mf) r += a.el_mf[row];
+                    } else {
+                        if (a.in_rho) r += in / xv;
+                        if (CHAIN && a.nmf) r += (double)mf;
+                        if (!CHAIN && a.el_mf) r += a.el_mf[row];
+                    }
+                }
+                if (a.add) r += a.add[row];
+                a.out_el[row] = r;
+                ssq += r * r;
+            }
+        }
+    }
+    if (a.ss) {
+        __shared__ double sh[kLineWaves];
+        for (int o = 32; o > 0; o >>= 1) ssq += __shfl_down(ssq, o, 64);
+        if (lane == 0) sh[wave] = ssq;
+        __syncthreads();
+        if (tid == 0) {
+            double s = 0.0;
+            for (int w = 0; w < kLineWaves; ++w) s += sh[w];
+            a.ss[blockIdx.x] = s;
+        }
+    }
+}
+
+// Positions per lane by the span: 64 B positions a workgroup, so that small problems still reach many
+// CUs and large ones read LDS once per 4 outputs.  A call's LDS must fit (wide stencils on fine
+// grids and many components keep the row kernels).
+int line_lanes(const Problem &P)
+{
+    const long long span = (long long)P.pad_u.P[0] - 2LL * P.pad_u.h[0];
+    return span <= 64LL * 256 ? 1 : (span <= 128LL * 256 ? 2 : 4);
+}
+struct LineShape {
+    int B, TN, hr, hf, rho_ld, rb_ld, mf_ld, adj_ld, blocks;
+    size_t elems;
+};
+LineShape line_shape(const Problem &P, bool chain, bool rows, bool el)
+{
+    LineShape s;
+    const int C = P.p.ncomp, hu = P.pad_u.h[0];
+    s.B = line_lanes(P);
+    s.TN = 64 * s.B;
+    s.hf = P.pad_f.h[0];
+    s.hr = chain ? std::max(hu, 2 * s.hf) : hu;
+    auto ld = [](int n) { return (n + kLineSlack + 3) & ~3; };
+    s.rho_ld = ld(s.TN + 2 * s.hr);
+    s.rb_ld = ld(chain ? s.TN + 2 * s.hf : s.TN);
+    s.mf_ld = s.TN;
+    s.adj_ld = ld(s.TN + 2 * s.hf);
+    s.elems = 0;
+    if (rows) s.elems += (size_t)C * s.rho_ld + 3 * (size_t)C * s.rb_ld + (P.nmf ? (size_t)C * C * s.mf_ld : 0);
+    if (el) s.elems += (size_t)(2 * C + 1) * s.adj_ld + (chain ? 0 : 3 * (size_t)C * s.mf_ld);
+    const long long span = (long long)P.pad_u.P[0] - 2LL * hu;
+    s.blocks = (int)((span + s.TN - 1) / s.TN);
+    return s;
+}
+
+template <typename T>
+LineRow<T> line_row(const DevRow1DT<T> &d)
+{
+    return LineRow<T>{d.w, d.wv, d.lo0, d.L};
+}
+
+template <typename T>
+LineArgs<T> line_args(const Problem &P, const LineShape &s)
+{
+    LineArgs<T> a{};
+    const int C = P.p.ncomp;
+    a.g = make_geo(P, P.pad_u);
+    for (int c = 0; c < C; ++c) {
+        a.th[c] = line_row(dev_row<T>(P, TMI_THETA, c));
+        a.de[c] = line_row(dev_row<T>(P, TMI_DELTA, c));
+    }
+    if (P.nmf)
+        for (int q = 0; q < C * C; ++q) a.u[q] = line_row(dev_row<T>(P, TMI_UATT, q));
+    a.cc = make_consts(P);
+    a.TN = s.TN;
+    a.hr = s.hr;
+    a.hf = s.hf;
+    a.rho_ld = s.rho_ld;
+    a.rb_ld = s.rb_ld;
+    a.mf_ld = s.mf_ld;
+    a.adj_ld = s.adj_ld;
+    a.nmf = P.nmf;
+    a.func = P.p.type_func;
+    a.nwall = P.p.nwall;
+    a.zero = P.d_zero;
+    a.elzero = P.d_elzero;
+    a.vext = P.d_vext;
+    return a;
+}
+
+template <typename T, bool CHAIN, bool LINEAR>
+void line_launch(const LineShape &s, const LineArgs<T> &a, hipStream_t st)
+{
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)s.blocks), dim3(kLineBlock), s.elems * sizeof(T), st, a);
+    };
+    if (s.B == 1)
+        go(k_line<T, 1, CHAIN, LINEAR>);
+    else if (s.B == 2)
+        go(k_line<T, 2, CHAIN, LINEAR>);
+    else
+        go(k_line<T, 4, CHAIN, LINEAR>);
+    TMI_HIP_CHECK(hipGetLastError());
+}
+
+}  // namespace
+
+// Every call of a 1D problem through k_line: dense row weights, the exact Jacobian's adjoint fields,
+// and LDS for the largest form (FP64).  The FMT halo never exceeds the density halo.
+bool line_available(const Problem &P)
+{
+    if (!P.line1d || !P.use_rows1d || P.pad_f.h[0] > P.pad_u.h[0]) return false;
+    const size_t most = std::max(line_shape(P, true, true, true).elems, line_shape(P, false, true, true).elems);
+    return most * sizeof(double) + 256 <= kLineLds;
+}
+long long line_partials(const Problem &P) { return line_available(P) ? line_shape(P, false, true, true).blocks : 0; }
+
+template <typename T>
+void line_rows_el(Problem &P, bool linear, const double *rho, const double *in_rb, const double *sub_rb, double *out_rb,
+                  const double *in_mf, const double *sub_mf, double *out_mf, const double *x, const double *dn_rb,
+                  const double *in_rho, const double *el_mf, const double *add, double *out_el, hipStream_t s, double *ss)
+{
+    const LineShape sh = line_shape(P, false, rho != nullptr, out_el != nullptr);
+    LineArgs<T> a = line_args<T>(P, sh);
+    const size_t N = P.N;
+    a.rho = rho;
+    a.in_rb = in_rb;
+    a.sub_rb = sub_rb;
+    a.out_rb = out_rb;
+    a.in_mf = in_mf;
+    a.sub_mf = sub_mf;
+    a.out_mf = out_mf;
+    if (out_el) {
+        a.x_rb = x + (size_t)P.iu_rb * N;
+        a.x_rho = x + (size_t)P.iu_rho * N;
+    }
+    a.dn_rb = dn_rb;
+    a.in_rho = in_rho;
+    a.el_mf = el_mf;
+    a.add = add;
+    a.out_el = out_el;
+    a.ss = ss;
+    if (linear)
+        line_launch<T, false, true>(sh, a, s);
+    else
+        line_launch<T, false, false>(sh, a, s);
+}
+template void line_rows_el<double>(Problem &, bool, const double *, const double *, const double *, double *,
+                                   const double *, const double *, double *, const double *, const double *,
+                                   const double *, const double *, const double *, double *, hipStream_t, double *);
+template void line_rows_el<float>(Problem &, bool, const double *, const double *, const double *, double *,
+                                  const double *, const double *, double *, const double *, const double *,
+                                  const double *, const double *, const double *, double *, hipStream_t, double *);
+
+template <typename T>
+void line_schur(Problem &P, const double *x, const double *x2, const double *mul, double *y2, const int *done, hipStream_t s)
+{
+    const LineShape sh = line_shape(P, true, true, true);
+    LineArgs<T> a = line_args<T>(P, sh);
+    const size_t N = P.N;
+    a.rho = x2;
+    a.mul = mul;
+    a.x_rb = x + (size_t)P.iu_rb * N;
+    a.x_rho = x + (size_t)P.iu_rho * N;
+    a.in_rho = x2;
+    a.out_el = y2;
+    a.done = done;
+    a.pore_of = P.d_pore_of;
+    line_launch<T, true, true>(sh, a, s);
+}
+template void line_schur<double>(Problem &, const double *, const double *, const double *, double *, const int *,
+                                 hipStream_t);
+template void line_schur<float>(Problem &, const double *, const double *, const double *, double *, const int *,
+                                hipStream_t);
+
+}  // namespace tmi
