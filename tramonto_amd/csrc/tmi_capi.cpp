@@ -577,6 +577,8 @@ Problem *create_problem(const tmi_params &p_in, const double *vext, const unsign
                     upload_row1d(*P, TMI_UATT, q, q % C, P->rowf[TMI_UATT][q]);
                 }
             P->use_rows1d = true;
+            const char *ln = std::getenv("TMI_LINE1D");
+            P->line1d = !(ln && std::string(ln) == "0");
         }
         // blocked reads run past the last field's halo (times zero weights): up to 2 kColB
         // planes (3D columns) or rows (2D), or 4 kRowPad positions (1D rows)

@@ -147,6 +147,7 @@ struct Problem {
     DevRow1DT<float> rowf[3][kNC * kNC];
     bool use_rows1d = false;
     RowTune tune[2][3];   // [FP64, FP32][rb, mf, el]
+    bool line1d = true;   // 1D rows in one launch where it applies (TMI_LINE1D=0: the row kernels)
     unsigned char *d_zero = nullptr;     // [C][N] Zero_density_TF
     unsigned char *d_elzero = nullptr;   // [C][N] EL row replaced by x (zero density or V_ext = VEXT_MAX)
     double *d_vext = nullptr;            // [C][N]
@@ -224,10 +225,26 @@ void launch_init_fields(Problem &P, double *x, hipStream_t s);
 //   t1 = A12 x2 (block-1 rows of J [x2;0]);  y2 = A22 x2 + A21 t1
 template <typename T>
 void launch_schur_apply(Problem &P, const double *x, const double *x2, double *t1, double *y2, hipStream_t s);
+bool schur_in_line(const Problem &P);   // ... in one launch (line_schur)
 // bS = b2 + A21 b1 (b full length)
 void launch_schur_rhs(Problem &P, const double *x, const double *b, double *bS, hipStream_t s);
 // x1 = A12 x2 - b1 written into dx (full length), x2 already in dx[0:C*N]
 void launch_schur_backsub(Problem &P, const double *x, const double *b, double *dx, hipStream_t s);
+
+// 1D rows in one launch (tmi_line.hip).  line_rows_el: the rho-bar and mean-field rows of rho (null:
+// none) and the Euler-Lagrange rows (out_el null: none), which read x and, in the linear mode, the
+// direction's rho-bar rows dn_rb; ss (optional): line_partials sums of the squares of the rows written.
+// line_schur: y2 = S (mul x2) (mul null: S x2); done (optional, batches): pores whose rows are not wanted.
+bool line_available(const Problem &P);
+long long line_partials(const Problem &P);
+template <typename T>
+void line_rows_el(Problem &P, bool linear, const double *rho, const double *in_rb, const double *sub_rb, double *out_rb,
+                  const double *in_mf, const double *sub_mf, double *out_mf, const double *x, const double *dn_rb,
+                  const double *in_rho, const double *el_mf, const double *add, double *out_el, hipStream_t s,
+                  double *ss = nullptr);
+template <typename T>
+void line_schur(Problem &P, const double *x, const double *x2, const double *mul, double *y2, const int *done,
+                hipStream_t s);
 
 // batched problems (tmi_batch.hip): per-pore Newton-Krylov; per-pore outputs may be NULL
 int batch_newton_solve(Problem &P, double *x, const tmi_newton_opts &o, tmi_newton_stats &st, int *pore_iters,

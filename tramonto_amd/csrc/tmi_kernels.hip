@@ -2090,6 +2090,15 @@ void residual_impl(Problem &P, const double *x, double *F, hipStream_t s, hipEve
     const size_t N = P.N;
     long long n_rb = 0, n_el = 0;
     if (P.hw_fwd.nrows || P.one_size) ss = nullptr;   // the rho-bar rows change after the fused passes
+    if (!ev && line_available(P)) {
+        line_rows_el<double>(P, false, x + P.iu_rho * N, x + P.iu_rb * N, nullptr, F + P.iu_rb * N,
+                             P.nmf ? x + P.iu_mf * N : nullptr, nullptr, F + P.iu_mf * N, x, nullptr, x + P.iu_rho * N,
+                             P.nmf ? x + P.iu_mf * N : nullptr, nullptr, F + P.iu_rho * N, s, ss);
+        hw_apply(P.hw_fwd, x + P.iu_rho * N, F + P.iu_rb * N, s);
+        one_size_rows(P, x + P.iu_rb * N, F + P.iu_rb * N, s);
+        if (nss) *nss = ss ? line_partials(P) : 0;
+        return;
+    }
     if (ev) TMI_HIP_CHECK(hipEventRecord(ev[0], s));
     rb_mf_rows<double>(P, x + P.iu_rho * N, false, x + P.iu_rb * N, nullptr, F + P.iu_rb * N,
                        P.nmf ? x + P.iu_mf * N : nullptr, nullptr, F + P.iu_mf * N, s, ev ? ev[1] : nullptr,
@@ -2224,13 +2233,13 @@ long long residual_sumsq_partials(const Problem &P)
 {
     long long cap = 0;
     fft_ss_buffer(P, &cap);
-    return std::max<long long>(cap, 1024);
+    return std::max<long long>({cap, line_partials(P), 1024});
 }
 
 void residual_sumsq_device(Problem &P, const double *x, double *F, double *partials, double *sumsq_d, hipStream_t s)
 {
     long long cnt = 0;
-    residual_impl(P, x, F, s, nullptr, P.fft ? partials : nullptr, &cnt);
+    residual_impl(P, x, F, s, nullptr, P.fft || line_available(P) ? partials : nullptr, &cnt);
     if (cnt > 0) {
         hipLaunchKernelGGL(k_sum_partials, dim3(1), dim3(kSumBlock), 0, s, partials, (int)cnt, sumsq_d, nullptr);
     } else {   // the blocks and order of dev_dot
@@ -2242,10 +2251,15 @@ void residual_sumsq_device(Problem &P, const double *x, double *F, double *parti
     TMI_HIP_CHECK(hipGetLastError());
 }
 
+constexpr long long kRedPartials = 512 * 1024;   // partial sums in P.d_red, clear of the Arnoldi coefficients past them
 double residual_sumsq(Problem &P, const double *x, double *F, hipStream_t s)
 {
     long long cap = 0, cnt = 0;
     double *ss = fft_ss_buffer(P, &cap);
+    if (line_available(P) && line_partials(P) <= kRedPartials) {
+        ss = P.d_red;
+        cap = kRedPartials;
+    }
     residual_impl(P, x, F, s, nullptr, ss, &cnt);
     if (cnt > cap) throw std::logic_error("partial sums past their buffer");
     if (cnt > 0) {
@@ -2260,6 +2274,14 @@ template <typename T>
 void launch_jvp(Problem &P, const double *x, const double *v, double *Jv, hipStream_t s)
 {
     const size_t N = P.N;
+    if (line_available(P) && !P.jac_ref) {
+        line_rows_el<T>(P, true, v + P.iu_rho * N, v + P.iu_rb * N, nullptr, Jv + P.iu_rb * N,
+                        P.nmf ? v + P.iu_mf * N : nullptr, nullptr, Jv + P.iu_mf * N, x, v + P.iu_rb * N,
+                        v + P.iu_rho * N, P.nmf ? v + P.iu_mf * N : nullptr, nullptr, Jv + P.iu_rho * N, s);
+        hw_apply(P.hw_fwd, v + P.iu_rho * N, Jv + P.iu_rb * N, s);
+        one_size_rows(P, v + P.iu_rb * N, Jv + P.iu_rb * N, s);
+        return;
+    }
     rb_mf_rows<T>(P, v + P.iu_rho * N, true, v + P.iu_rb * N, nullptr, Jv + P.iu_rb * N,
                   P.nmf ? v + P.iu_mf * N : nullptr, nullptr, Jv + P.iu_mf * N, s);
     hw_apply(P.hw_fwd, v + P.iu_rho * N, Jv + P.iu_rb * N, s);
@@ -2275,17 +2297,29 @@ template void launch_jvp<float>(Problem &, const double *, const double *, doubl
 void launch_init_fields(Problem &P, double *x, hipStream_t s)
 {
     const size_t N = P.N;
-    rb_mf_rows<double>(P, x + P.iu_rho * N, false, nullptr, nullptr, x + P.iu_rb * N, nullptr, nullptr,
-                       x + P.iu_mf * N, s);
+    if (line_available(P))
+        line_rows_el<double>(P, false, x + P.iu_rho * N, nullptr, nullptr, x + P.iu_rb * N, nullptr, nullptr,
+                             x + P.iu_mf * N, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, s);
+    else
+        rb_mf_rows<double>(P, x + P.iu_rho * N, false, nullptr, nullptr, x + P.iu_rb * N, nullptr, nullptr,
+                           x + P.iu_mf * N, s);
     hipLaunchKernelGGL(k_cap_n3, dim3(grid_for(P.N)), dim3(kBlock), 0, s, x + P.iu_rb * N, P.N);
     TMI_HIP_CHECK(hipGetLastError());
 }
 
-// t1 = A12 x2 (rho-bar and mean-field rows of J [x2; 0]); y2 = A22 x2 + A21 t1
+// the Schur product in one launch: hard-surface corrections and the reference's Jacobian need the rows
+bool schur_in_line(const Problem &P) { return line_available(P) && !P.jac_ref && P.hw_fwd.nrows == 0; }
+
+// y2 = A22 x2 + A21 t1, t1 = A12 x2 the rho-bar and mean-field rows of J [x2; 0] (scratch: the one-launch
+// 1D form does not write it)
 template <typename T>
 void launch_schur_apply(Problem &P, const double *x, const double *x2, double *t1, double *y2, hipStream_t s)
 {
     const size_t N = P.N;
+    if (schur_in_line(P)) {
+        line_schur<T>(P, x, x2, nullptr, y2, nullptr, s);
+        return;
+    }
     rb_mf_rows<T>(P, x2, true, nullptr, nullptr, t1, nullptr, nullptr, t1 + (size_t)P.nrb * N, s);
     hw_apply(P.hw_fwd, x2, t1, s);
     fmt_point<T>(P, x + P.iu_rb * N, t1, true, s);
@@ -2299,6 +2333,11 @@ template void launch_schur_apply<float>(Problem &, const double *, const double 
 void launch_schur_rhs(Problem &P, const double *x, const double *b, double *bS, hipStream_t s)
 {
     const size_t N = P.N;
+    if (line_available(P) && !P.jac_ref) {
+        line_rows_el<double>(P, true, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, x, b + P.iu_rb * N,
+                             nullptr, P.nmf ? b + P.iu_mf * N : nullptr, b + P.iu_rho * N, bS, s);
+        return;
+    }
     fmt_point<double>(P, x + P.iu_rb * N, b + P.iu_rb * N, true, s);
     el_rows<double>(P, true, x + P.iu_rho * N, nullptr, P.nmf ? b + P.iu_mf * N : nullptr, b + P.iu_rho * N, bS, s);
     TMI_HIP_CHECK(hipGetLastError());
@@ -2309,8 +2348,13 @@ void launch_schur_backsub(Problem &P, const double *x, const double *b, double *
 {
     (void)x;
     const size_t N = P.N;
-    rb_mf_rows<double>(P, dx + P.iu_rho * N, true, nullptr, b + P.iu_rb * N, dx + P.iu_rb * N, nullptr,
-                       P.nmf ? b + P.iu_mf * N : nullptr, P.nmf ? dx + P.iu_mf * N : nullptr, s);
+    if (line_available(P))
+        line_rows_el<double>(P, true, dx + P.iu_rho * N, nullptr, b + P.iu_rb * N, dx + P.iu_rb * N, nullptr,
+                             P.nmf ? b + P.iu_mf * N : nullptr, P.nmf ? dx + P.iu_mf * N : nullptr, nullptr, nullptr,
+                             nullptr, nullptr, nullptr, nullptr, s);
+    else
+        rb_mf_rows<double>(P, dx + P.iu_rho * N, true, nullptr, b + P.iu_rb * N, dx + P.iu_rb * N, nullptr,
+                           P.nmf ? b + P.iu_mf * N : nullptr, P.nmf ? dx + P.iu_mf * N : nullptr, s);
     hw_apply(P.hw_fwd, dx + P.iu_rho * N, dx + P.iu_rb * N, s);
     TMI_HIP_CHECK(hipGetLastError());
 }

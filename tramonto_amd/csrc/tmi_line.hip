@@ -11,10 +11,13 @@
 //  * Schur product (CHAIN): the rho-bar sums are formed on the span and its FMT halo (recomputed by
 //    the neighbours), become adjoint fields in LDS, and feed the Euler-Lagrange sums: no row leaves
 //    the chip.
-// Each lane owns B consecutive outputs and reads B densities per step, so every LDS read feeds B
-// multiply-adds per stencil against weights in scalar registers; at B = 4 the LDS reads (16 cycles a
-// wave for 4 positions) and the FP64 multiply-adds (64 cycles) balance.  Small problems are bound by
-// latency and take B = 1 and 64 positions a workgroup, which puts 401 nodes on 7 CUs instead of 1.
+// Each lane owns B consecutive outputs, so every LDS value read feeds B multiply-adds per stencil
+// against weights in scalar registers.  Small problems are bound by latency and take B = 1 and 64
+// positions a workgroup, which puts 401 nodes on 7 CUs instead of 1; large ones are bound by the FP64
+// multiply-adds and LDS reads of the sums (256 pores, 221,378 nodes: 0.8 GFLOP, 14 us at the FP64
+// peak with the halo's recomputed sums) and take B = 4.
+// Measured, FP64: residual kernels of the 401-node hard wall 40 -> 9 us (with its sum of squares),
+// Schur product of 256 pores 87 -> 34 us.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -31,7 +34,6 @@ using namespace dev;
 
 constexpr int kLineWaves = 8;
 constexpr int kLineBlock = 64 * kLineWaves;
-constexpr int kLineSlack = 16;           // zero positions past each LDS row (whole steps read past the span)
 constexpr size_t kLineLds = 64 * 1024;   // dynamic LDS of a launch
 
 template <typename T>
@@ -46,7 +48,7 @@ struct LineArgs {
     LineRow<T> th[kNC], de[kNC], u[kNC * kNC];
     CompConsts cc;
     int TN, hr, hf;   // positions per workgroup, density halo in LDS, FMT halo
-    int rho_ld, rb_ld, mf_ld, adj_ld;   // LDS row lengths
+    int rho_ld, rb_ld, mf_ld, adj_ld, chain_ld;   // LDS row lengths; CHAIN: of the densities' and adjoint fields' shared space
     int nmf, func, nwall;
     const double *rho, *mul;   // densities or direction [C][N] (null: no rows), optional factor
     const unsigned char *zero, *elzero;
@@ -87,77 +89,105 @@ __device__ inline int line_map(const Geo &g, int q, int &src, int &refl)
     return 0;
 }
 
-// B consecutive LDS values, 16-byte aligned where B values fill 16 bytes
+constexpr int kLineStep = 8;   // positions read per step of a stencil sum
+
+// kLineStep LDS values from a multiple of B
 template <typename T, int B>
-__device__ __forceinline__ void lds_read(const T *p, T (&v)[B])
+__device__ __forceinline__ void lds_read(const T *p, T (&v)[kLineStep])
 {
-    typedef T VB __attribute__((ext_vector_type(B)));
-    const VB t = *reinterpret_cast<const VB *>(p);
+    if constexpr (B > 1) {
+        typedef T VB __attribute__((ext_vector_type(B)));
 #pragma unroll
-    for (int i = 0; i < B; ++i) v[i] = t[i];
-}
-template <typename T>
-__device__ __forceinline__ void lds_read(const T *p, T (&v)[1])
-{
-    v[0] = *p;
+        for (int q = 0; q < kLineStep / B; ++q) {
+            const VB t = reinterpret_cast<const VB *>(p)[q];
+#pragma unroll
+            for (int i = 0; i < B; ++i) v[q * B + i] = t[i];
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < kLineStep; ++i) v[i] = p[i];
+    }
 }
 
 // acc[s][b] += sum_j w_s[j] row[a0 + b + j] for NS weight rows of one stencil (row: LDS, a0: the
-// lane's first position plus the stencil's first offset, a multiple of B apart between lanes)
+// wave's first position plus the stencil's first offset, lane_a: the lane's, a multiple of B).  With
+// B = 1 (few waves on the chip) the next step's values and weights are requested before this step's
+// multiply-adds, so a wave does not wait for each of its LDS and scalar loads in turn; otherwise the
+// CU's other waves cover the wait and the registers buy more of them.
 template <typename T, int B, int NS>
 __device__ __forceinline__ void line_sum(const T *row, int a0, int lane_a, const T *__restrict__ w0,
                                          const T *__restrict__ w1, int L, T (&acc)[NS][B])
 {
+    constexpr int K = kLineStep, NW = K + B - 1;
     const int sh = a0 & (B - 1);   // wave-uniform: reads start on a multiple of B
     const T *src = row + (a0 - sh) + lane_a;
     const int back = kRowPad - sh - (B - 1);
-    const T *w[2] = {w0 + back, NS > 1 ? w1 + back : w0 + back};
-    const int nk = (L + sh + 2 * B - 2) / B;
-    for (int k = 0; k < nk; ++k) {
-        T v[B];
-        lds_read(src + k * B, v);
+    // constant address space: wave-uniform weights go through the scalar cache into scalar registers
+    typedef const T __attribute__((address_space(4))) *ConstW;
+    const ConstW w[2] = {(ConstW)(w0 + back), (ConstW)((NS > 1 ? w1 : w0) + back)};
+    const int nk = (L + sh + B - 1 + K - 1) / K;
+    T v[2][K], wk[2][NS][NW];
+    auto load = [&](int k, int p) {
+        lds_read<T, B>(src + k * K, v[p]);
 #pragma unroll
-        for (int s = 0; s < NS; ++s) {
-            T wk[2 * B - 1];
+        for (int s = 0; s < NS; ++s)
 #pragma unroll
-            for (int j = 0; j < 2 * B - 1; ++j) wk[j] = w[s][k * B + j];
+            for (int j = 0; j < NW; ++j) wk[p][s][j] = w[s][k * K + j];
+    };
+    auto fma_step = [&](int p) {
 #pragma unroll
-            for (int i = 0; i < B; ++i)
+        for (int i = 0; i < K; ++i)
 #pragma unroll
-                for (int b = 0; b < B; ++b) acc[s][b] += wk[i - b + B - 1] * v[i];
+            for (int s = 0; s < NS; ++s)
+#pragma unroll
+                for (int b = 0; b < B; ++b) acc[s][b] += wk[p][s][i - b + B - 1] * v[p][i];
+    };
+    if constexpr (B == 1) {
+        load(0, 0);
+        for (int k = 0; k < nk; k += 2) {   // a step past the last reads zero weights and the row's slack
+            load(k + 1, 1);
+            fma_step(0);
+            load(k + 2, 0);
+            fma_step(1);
+        }
+    } else {
+        for (int k = 0; k < nk; ++k) {
+            load(k, 0);
+            fma_step(0);
         }
     }
 }
 
-// adjoint fields A_c, B_c (c < C), S3 of node src's derivatives (dn: the linear modes' direction)
-template <typename T, bool LINEAR>
-__device__ inline void line_adjoint(const Geo &g, const CompConsts &cc, int func, const double *__restrict__ x_rb, int src,
-                                    const double *dr, int refl, T *out, int ld)
+// the rho-bar rows of node src (solution order)
+__device__ inline void line_rb(const double *__restrict__ rb, size_t N, int src, double (&v)[6])
 {
-    double n[6], o[6];
-    const size_t N = g.N;
-    n[3] = x_rb[src];
-    n[2] = x_rb[N + src];
-    n[1] = x_rb[2 * N + src];
-    n[0] = x_rb[3 * N + src];
-    n[5] = x_rb[4 * N + src];
-    n[4] = x_rb[5 * N + src];
+#pragma unroll
+    for (int q = 0; q < 6; ++q) v[q] = rb[(size_t)q * N + src];
+}
+
+// adjoint fields A_c, B_c (c < C), S3 from the rho-bar values r (LINEAR: and the direction's dr)
+template <typename T, bool LINEAR>
+__device__ inline void line_adjoint(int C, const CompConsts &cc, int func, const double (&r)[6], const double (&dr)[6],
+                                    int refl, T *out, int ld)
+{
+    const double n[6] = {r[3], r[2], r[1], r[0], r[5], r[4]};
+    double o[6];
     if constexpr (LINEAR) {
         const double dn[6] = {dr[3], dr[2], dr[1], dr[0], dr[5], dr[4]};
         fmt_hvp<1>(func, n, dn, o);
     } else {
         fmt_dphi<1>(func, n, o);
     }
-    for (int c = 0; c < g.C; ++c) {
+    for (int c = 0; c < C; ++c) {
         out[(2 * c) * ld] = (T)(o[0] * cc.i4pirsq[c] + o[1] * cc.i4pir[c] + o[2]);
         const T b = (T)(o[4] * cc.i4pir[c] + o[5]);
         out[(2 * c + 1) * ld] = refl ? -b : b;
     }
-    out[2 * g.C * ld] = (T)o[3];
+    out[2 * C * ld] = (T)o[3];
 }
 
 template <typename T, int B, bool CHAIN, bool LINEAR>
-__global__ __launch_bounds__(kLineBlock) void k_line(LineArgs<T> a)
+__global__ __launch_bounds__(kLineBlock, B == 1 ? 2 : 6) void k_line(LineArgs<T> a)
 {
     extern __shared__ __attribute__((aligned(32))) char smem_raw[];
     const Geo &g = a.g;
@@ -175,22 +205,22 @@ __global__ __launch_bounds__(kLineBlock) void k_line(LineArgs<T> a)
     }
     const int rb_n = CHAIN ? TN + 2 * hf : TN, adj_n = TN + 2 * hf, ext = CHAIN ? hf : 0;
     T *rho = reinterpret_cast<T *>(smem_raw);               // [C][rho_ld]
-    T *adj = rho + (a.rho ? C * a.rho_ld : 0);              // [2 C + 1][adj_ld]
-    T *srb = adj + (a.out_el ? (2 * C + 1) * a.adj_ld : 0); // [C][3][rb_ld]: theta, delta, vector delta
+    // CHAIN: the adjoint fields replace the densities once the sums are formed
+    T *adj = CHAIN ? rho : rho + (a.rho ? C * a.rho_ld : 0);   // [2 C + 1][adj_ld]
+    T *srb = CHAIN ? rho + a.chain_ld : adj + (a.out_el ? (2 * C + 1) * a.adj_ld : 0);   // [C][3][rb_ld]: theta, delta, vector delta
     T *smf = srb + (a.rho ? 3 * C * a.rb_ld : 0);           // [C][C][mf_ld]
     T *sel = CHAIN ? srb : smf + (a.rho && a.nmf ? C * C * a.mf_ld : 0);   // [C][3][mf_ld]
-    // densities with their halo
+    // densities with their halo, by the last threads first (the adjoint fields take the first ones)
     if (a.rho) {
-        for (int r = tid; r < a.rho_ld; r += kLineBlock) {
+        for (int r = kLineBlock - 1 - tid; r < a.rho_ld; r += kLineBlock) {
             int src = 0, refl = 0, code = -2;
             if (r < TN + 2 * hr) code = line_map(g, p0 - hr + r, src, refl);
             for (int c = 0; c < C; ++c) {
-                double v = 0.0;
-                if (code == 0) {
+                double v = code == -1 && !LINEAR ? a.cc.rho_b[c] : 0.0;
+                if (code == 0) {   // every load unconditional: none waits for another
                     const size_t q = (size_t)c * N + src;
-                    v = a.zero[q] ? 0.0 : a.rho[q] * (a.mul ? a.mul[q] : 1.0);
-                } else if (code == -1 && !LINEAR) {
-                    v = a.cc.rho_b[c];
+                    const double rv = a.rho[q], m = a.mul ? a.mul[q] : 1.0;
+                    v = a.zero[q] ? 0.0 : rv * m;
                 }
                 rho[c * a.rho_ld + r] = (T)v;
             }
@@ -210,16 +240,72 @@ __global__ __launch_bounds__(kLineBlock) void k_line(LineArgs<T> a)
             int src = 0, refl = 0, code = -2;
             if (r < adj_n) code = line_map(g, p0 - hf + r, src, refl);
             if (code == 0) {
-                double dr[6];
-                if constexpr (LINEAR) {
-#pragma unroll
-                    for (int q = 0; q < 6; ++q) dr[q] = a.dn_rb[(size_t)q * N + src];
-                }
-                line_adjoint<T, LINEAR>(g, a.cc, a.func, a.x_rb, src, dr, refl, adj + r, a.adj_ld);
+                double xr[6], dr[6];
+                line_rb(a.x_rb, N, src, xr);
+                if constexpr (LINEAR) line_rb(a.dn_rb, N, src, dr);
+                line_adjoint<T, LINEAR>(C, a.cc, a.func, xr, dr, refl, adj + r, a.adj_ld);
             } else {
                 adjoint_halo(r, code);
             }
         }
+    }
+    // Node inputs of this thread's first adjoint position (CHAIN) and first output row, with B = 1 requested
+    // before the sums.  Output rows: the Euler-Lagrange rows, then the rho-bar rows, then the mean-field rows;
+    // thread e takes position e mod TN of row e / TN.
+    const int n_out = (a.out_el ? C : 0) + (!CHAIN && a.rho ? 6 + a.nmf : 0);
+    struct AdjIn {
+        int src, refl, code;
+        double x[6];
+    };
+    auto adj_in = [&](int r) {
+        AdjIn v;
+        v.src = v.refl = 0;
+        v.code = -2;
+        if (r < adj_n) v.code = line_map(g, p0 - hf + r, v.src, v.refl);
+        if (v.code == 0) line_rb(a.x_rb, N, v.src, v.x);
+        return v;
+    };
+    struct RowIn {
+        int i;   // node (< 0: none)
+        unsigned char fixed;
+        double x, in, sub, vext, mf, add, mu;
+    };
+    auto row_in = [&](int e) {
+        RowIn v;
+        v.i = -1;
+        v.fixed = 0;
+        v.x = 1.0;
+        v.in = v.sub = v.vext = v.mf = v.add = v.mu = 0.0;
+        const int row = e / TN, q = p0 + e - row * TN;
+        int refl;
+        if (row >= n_out || q >= g.P[0] - g.h[0] || line_map(g, q, v.i, refl) != 0) {
+            v.i = -1;
+            return v;
+        }
+        if (a.out_el && row < C) {
+            const size_t at = (size_t)row * N + v.i;
+            v.fixed = a.elzero[at];
+            v.x = a.x_rho[at];
+            if (a.in_rho) v.in = a.in_rho[at];
+            if (a.mul) v.in *= a.mul[at];
+            if (!LINEAR && a.nwall > 0) v.vext = a.vext[at];
+            if (!CHAIN && a.el_mf) v.mf = a.el_mf[at];
+            if (a.add) v.add = a.add[at];
+            if constexpr (!LINEAR) v.mu = g.mu ? g.mu[at] : a.cc.mu[row];
+        } else {
+            const int r = row - (a.out_el ? C : 0);
+            const size_t at = (size_t)(r < 6 ? r : r - 6) * N + v.i;
+            const double *in = r < 6 ? a.in_rb : a.in_mf, *sub = r < 6 ? a.sub_rb : a.sub_mf;
+            if (in) v.in = in[at];
+            if (sub) v.sub = sub[at];
+        }
+        return v;
+    };
+    AdjIn ain;
+    RowIn rin;
+    if constexpr (B == 1) {
+        if constexpr (CHAIN) ain = adj_in(tid);
+        rin = row_in(tid);
     }
     __syncthreads();
     // stencil sums, one item per wave at a time, the longest first
@@ -265,99 +351,72 @@ __global__ __launch_bounds__(kLineBlock) void k_line(LineArgs<T> a)
         }
     }
     __syncthreads();
-    // the rho-bar values at index r of the sums, solution order
-    auto rb_vals = [&](int r, double (&vals)[6]) {
-        T n3 = 0, n2 = 0, n1 = 0, n0 = 0, v2 = 0, v1 = 0;
+    // rho-bar value q (solution order) at index r of the sums
+    auto rb_val = [&](int q, int r) {
+        const int k = q == 0 ? 0 : (q < 4 ? 1 : 2);
+        T v = 0;
         for (int c = 0; c < C; ++c) {
-            const T st = srb[(3 * c) * a.rb_ld + r], sd = srb[(3 * c + 1) * a.rb_ld + r], sv = srb[(3 * c + 2) * a.rb_ld + r];
-            n3 += st;
-            n2 += sd;
-            n1 += (T)a.cc.i4pir[c] * sd;
-            n0 += (T)a.cc.i4pirsq[c] * sd;
-            v2 += sv;
-            v1 += (T)a.cc.i4pir[c] * sv;
+            const T sum = srb[(3 * c + k) * a.rb_ld + r];
+            const T f = q == 2 || q == 5 ? (T)a.cc.i4pir[c] : (q == 3 ? (T)a.cc.i4pirsq[c] : (T)1);
+            v += f * sum;
         }
-        vals[0] = n3;
-        vals[1] = n2;
-        vals[2] = n1;
-        vals[3] = n0;
-        vals[4] = v2;
-        vals[5] = v1;
+        return (double)v;
     };
     if constexpr (CHAIN) {
-        for (int r = tid; r < a.adj_ld; r += kLineBlock) {
-            int src = 0, refl = 0, code = -2;
-            if (r < adj_n) code = line_map(g, p0 - hf + r, src, refl);
+        auto adj_out = [&](int r, const AdjIn &v) {
             // across a mirror the node's own sums; a mirror node outside the span serves no output here
-            const int rs = refl ? src + g.h[0] - (p0 - hf) : r;
-            if (code == 0 && rs >= 0 && rs < rb_n) {
+            const int rs = v.refl ? v.src + g.h[0] - (p0 - hf) : r;
+            if (v.code == 0 && rs >= 0 && rs < rb_n) {
                 double dr[6];
-                rb_vals(rs, dr);
-                line_adjoint<T, true>(g, a.cc, a.func, a.x_rb, src, dr, refl, adj + r, a.adj_ld);
+#pragma unroll
+                for (int q = 0; q < 6; ++q) dr[q] = rb_val(q, rs);
+                line_adjoint<T, true>(C, a.cc, a.func, v.x, dr, v.refl, adj + r, a.adj_ld);
             } else {
-                adjoint_halo(r, code == 0 ? -2 : code);
+                adjoint_halo(r, v.code == 0 ? -2 : v.code);
             }
-        }
+        };
+        if (B == 1 && tid < a.adj_ld) adj_out(tid, ain);
+        for (int r = B == 1 ? tid + kLineBlock : tid; r < a.adj_ld; r += kLineBlock) adj_out(r, adj_in(r));
         __syncthreads();
         for (int it = wave; it < 3 * C * nt; it += kLineWaves) el_item(it);
         __syncthreads();
     }
     // rows
     double ssq = 0.0;
-    for (int t = tid; t < TN; t += kLineBlock) {
-        int i = -1, refl = 0;
-        if (line_map(g, p0 + t, i, refl) != 0 || p0 + t >= g.P[0] - g.h[0]) continue;
-        if (!CHAIN && a.rho) {
-            if (a.out_rb) {
-                double vals[6];
-                rb_vals(t, vals);
-#pragma unroll
-                for (int r = 0; r < 6; ++r) {
-                    double o = vals[r];
-                    if (a.in_rb) o -= a.in_rb[(size_t)r * N + i];
-                    if (a.sub_rb) o -= a.sub_rb[(size_t)r * N + i];
-                    a.out_rb[(size_t)r * N + i] = o;
-                    ssq += o * o;
-                }
-            }
-        }
-        for (int c = 0; c < C; ++c) {
-            const size_t row = (size_t)c * N + i;
-            T mf = 0;
-            if (a.rho && a.nmf)
-                for (int cj = 0; cj < C; ++cj) mf += smf[(c * C + cj) * a.mf_ld + t];
-            if (!CHAIN && a.rho && a.nmf) {
-                double o = (double)mf;
-                if (a.in_mf) o -= a.in_mf[row];
-                if (a.sub_mf) o -= a.sub_mf[row];
-                a.out_mf[row] = o;
-                ssq += o * o;
-            }
-            if (a.out_el) {
-                const double in = a.in_rho ? a.in_rho[row] * (a.mul ? a.mul[row] : 1.0) : 0.0;
-                double r;
-                if (a.elzero[row]) {
-                    r = in;
+    auto mf_sum = [&](int c, int t) {
+        T mf = 0;
+        for (int cj = 0; cj < C; ++cj) mf += smf[(c * C + cj) * a.mf_ld + t];
+        return (double)mf;
+    };
+    auto row_out = [&](int e, const RowIn &v) {
+        if (v.i < 0) return;
+        const int row = e / TN, t = e - row * TN;
+        double r;
+        if (a.out_el && row < C) {
+            if (v.fixed) {
+                r = v.in;
+            } else {
+                const T *s = sel + 3 * row * a.mf_ld + t;
+                r = (double)(s[2 * a.mf_ld] + s[0] - s[a.mf_ld]);
+                if constexpr (!LINEAR) {
+                    r += log(v.x) + v.mu;
+                    if (a.nwall > 0) r += v.vext;
                 } else {
-                    const T *s = sel + 3 * c * a.mf_ld + t;
-                    r = (double)(s[2 * a.mf_ld] + s[0] - s[a.mf_ld]);
-                    const double xv = a.x_rho[row];
-                    if constexpr (!LINEAR) {
-                        r += log(xv) + (g.mu ? g.mu[row] : a.cc.mu[c]);
-                        if (a.nwall > 0) r += a.vext[row];
-                        if (a.el_mf) r += a.el_mf[row];
-                    } else {
-                        if (a.in_rho) r += in / xv;
-                        if (CHAIN && a.nmf) r += (double)mf;
-                        if (!CHAIN && a.el_mf) r += a.el_mf[row];
-                    }
+                    if (a.in_rho) r += v.in / v.x;
                 }
-                if (a.add) r += a.add[row];
-                a.out_el[row] = r;
-                ssq += r * r;
+                if (CHAIN ? a.nmf > 0 : a.el_mf != nullptr) r += CHAIN ? mf_sum(row, t) : v.mf;
             }
+            if (a.add) r += v.add;
+            a.out_el[(size_t)row * N + v.i] = r;
+        } else {
+            const int q = row - (a.out_el ? C : 0);
+            r = (q < 6 ? rb_val(q, t) : mf_sum(q - 6, t)) - v.in - v.sub;
+            (q < 6 ? a.out_rb + (size_t)q * N : a.out_mf + (size_t)(q - 6) * N)[v.i] = r;
         }
-    }
+        ssq += r * r;
+    };
+    if constexpr (B == 1) row_out(tid, rin);
+    for (int e = B == 1 ? tid + kLineBlock : tid; e < n_out * TN; e += kLineBlock) row_out(e, row_in(e));
     if (a.ss) {
         __shared__ double sh[kLineWaves];
         for (int o = 32; o > 0; o >>= 1) ssq += __shfl_down(ssq, o, 64);
@@ -380,7 +439,7 @@ int line_lanes(const Problem &P)
     return span <= 64LL * 256 ? 1 : (span <= 128LL * 256 ? 2 : 4);
 }
 struct LineShape {
-    int B, TN, hr, hf, rho_ld, rb_ld, mf_ld, adj_ld, blocks;
+    int B, TN, hr, hf, rho_ld, rb_ld, mf_ld, adj_ld, chain_ld, blocks;
     size_t elems;
 };
 LineShape line_shape(const Problem &P, bool chain, bool rows, bool el)
@@ -391,14 +450,15 @@ LineShape line_shape(const Problem &P, bool chain, bool rows, bool el)
     s.TN = 64 * s.B;
     s.hf = P.pad_f.h[0];
     s.hr = chain ? std::max(hu, 2 * s.hf) : hu;
-    auto ld = [](int n) { return (n + kLineSlack + 3) & ~3; };
+    auto ld = [&](int n) { return (n + (s.B == 1 ? 40 : 20) + 3) & ~3; };   // zero positions that a sum's last steps read
     s.rho_ld = ld(s.TN + 2 * s.hr);
-    s.rb_ld = ld(chain ? s.TN + 2 * s.hf : s.TN);
+    s.rb_ld = (s.TN + (chain ? 2 * s.hf : 0) + 3) & ~3;
     s.mf_ld = s.TN;
     s.adj_ld = ld(s.TN + 2 * s.hf);
-    s.elems = 0;
-    if (rows) s.elems += (size_t)C * s.rho_ld + 3 * (size_t)C * s.rb_ld + (P.nmf ? (size_t)C * C * s.mf_ld : 0);
-    if (el) s.elems += (size_t)(2 * C + 1) * s.adj_ld + (chain ? 0 : 3 * (size_t)C * s.mf_ld);
+    const size_t n_rho = (size_t)C * s.rho_ld, n_adj = (size_t)(2 * C + 1) * s.adj_ld;
+    s.chain_ld = (int)std::max(n_rho, n_adj);
+    s.elems = chain ? s.chain_ld : (rows ? n_rho : 0) + (el ? n_adj + 3 * (size_t)C * s.mf_ld : 0);
+    if (rows) s.elems += 3 * (size_t)C * s.rb_ld + (P.nmf ? (size_t)C * C * s.mf_ld : 0);
     const long long span = (long long)P.pad_u.P[0] - 2LL * hu;
     s.blocks = (int)((span + s.TN - 1) / s.TN);
     return s;
@@ -430,6 +490,7 @@ LineArgs<T> line_args(const Problem &P, const LineShape &s)
     a.rb_ld = s.rb_ld;
     a.mf_ld = s.mf_ld;
     a.adj_ld = s.adj_ld;
+    a.chain_ld = s.chain_ld;
     a.nmf = P.nmf;
     a.func = P.p.type_func;
     a.nwall = P.p.nwall;
