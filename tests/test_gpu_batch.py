@@ -237,3 +237,29 @@ def test_batch_newton_ignores_unwritten_basis_vectors():
     x = db.initial_state()
     st = db.newton(x, resid_tol=1e-10, gmres_tol=1e-9, max_iter=60)
     assert st["converged"], st
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nodes,graph", [((1, 2, 3, 40, 900), "1"), ((2049, 2600, 150), "0"), ((4500, 300), "1"),
+                                         ((9000, 500, 120), "1")])
+def test_batch_newton_segment_lengths(nodes, graph, monkeypatch):
+    """One-launch Arnoldi steps over every workgroup shape, and pores too long for one (two components:
+    4096, 8192 and 16384 unknowns are the edges): batch and pore-by-pore profiles agree to the
+    tolerance of the solves, pores of a few nodes and pores that finish early included."""
+    from tramonto_amd.batch import BatchSpec, DeviceBatch
+    from tramonto_amd.device import DeviceProblem
+    from tramonto_amd.problem import slit_pore_1d
+    monkeypatch.setenv("TMI_BATCH_GRAPH", graph)
+    pores = [slit_pore_1d(H=0.02 * max(n - 1, 1) if n > 1 else 0.0, dx=0.02, rho_b=(0.1, 0.1), eps_ff=0.5, seed=i)
+             for i, n in enumerate(nodes)]
+    db = DeviceBatch(BatchSpec(pores))
+    for restart in (60, 7):
+        x = db.initial_state()
+        st = db.newton(x, resid_tol=1e-10, gmres_tol=1e-9, max_iter=60, gmres_restart=restart)
+        assert st["converged"], st
+    o = db.batch.offsets
+    for i, p in enumerate(pores):
+        dp = DeviceProblem(p)
+        xs = dp.initial_state()
+        assert dp.newton(xs, resid_tol=1e-10, gmres_tol=1e-9, max_iter=60, gmres_restart=7)["converged"]
+        assert float((xs - x[:, o[i]:o[i + 1]]).abs().max()) < 1e-8

@@ -676,6 +676,8 @@ void destroy_problem(Problem *P)
     (void)hipFree(P->f_rbw2);
     (void)hipFree(P->d_scratch);
     (void)hipFree(P->d_newton);
+    (void)hipFree(P->d_line_gs);
+    (void)hipFree(P->d_line_gi);
     (void)hipFree(P->d_xi);
     (void)hipFree(P->d_vi);
     (void)hipFree(P->d_fi);
@@ -847,6 +849,8 @@ int gmres_schur_t(Problem &P, const double *x, const double *bS, double *x2, dou
 int gmres_schur(Problem &P, const double *x, const double *bS, double *x2, double rtol, int m, int maxit, int prec,
                 double *work, hipStream_t s)
 {
+    int its = 0;
+    if (gmres_line(P, x, bS, x2, rtol, std::max(1, std::min(m, 500)), maxit, prec, work, &its, s)) return its;
     if (prec == TMI_PREC_MIXED) return gmres_schur_t<float>(P, x, bS, x2, rtol, m, maxit, prec, work, s);
     return gmres_schur_t<double>(P, x, bS, x2, rtol, m, maxit, prec, work, s);
 }

@@ -171,6 +171,9 @@ struct Problem {
     double *d_newton = nullptr;   // [2][nunk][N]: F and dx of tmi_newton_solve, from its first call on
     double *d_scratch = nullptr;
     size_t scratch_bytes = 0;
+    double *d_line_gs = nullptr;   // gmres_line: bookkeeping for restarts of line_gs_m, from its first call on
+    int *d_line_gi = nullptr;
+    int line_gs_m = 0;
     double *d_red = nullptr;     // reduction buffer
     double *h_red = nullptr;     // pinned host mirror (1024 doubles), written by reduction kernels directly
     double *h_red_dev = nullptr; // its device address
@@ -245,6 +248,25 @@ void line_rows_el(Problem &P, bool linear, const double *rho, const double *in_r
 template <typename T>
 void line_schur(Problem &P, const double *x, const double *x2, const double *mul, double *y2, const int *done,
                 hipStream_t s);
+
+// Per-segment GMRES bookkeeping (tmi_batch.hip): P independent Arnoldi processes over the segments
+// [off[p], off[p + 1]) of one packed vector.
+struct GmresState {
+    double *H;       // [P][m+1][m] (rotated: upper triangular)
+    double *cs, *sn; // [P][m]
+    double *g;       // [P][m+1]
+    double *y;       // [P][m]
+    double *h1, *h2; // [P][m+1] Gram-Schmidt coefficients of the two passes (segments too long for one workgroup)
+    double *hn;      // [P]
+    double *bn;      // [P] norm of the right-hand side
+    int *kdone;      // [P] Arnoldi steps taken in this cycle
+    int *done;       // [P] converged (or inactive)
+    int *its;        // [P] GMRES iterations over the whole solve
+    int m;
+};
+// GMRES of one small 1D problem on the segmented kernels: S x2 = bS; false where it does not apply
+bool gmres_line(Problem &P, const double *x, const double *bS, double *x2, double rtol, int m, int maxit, int prec,
+                double *work, int *iters, hipStream_t s);
 
 // batched problems (tmi_batch.hip): per-pore Newton-Krylov; per-pore outputs may be NULL
 int batch_newton_solve(Problem &P, double *x, const tmi_newton_opts &o, tmi_newton_stats &st, int *pore_iters,

@@ -57,7 +57,7 @@ struct LineArgs {
     const double *x_rb, *dn_rb, *x_rho, *in_rho, *el_mf, *vext, *add;
     double *out_el;            // null: no Euler-Lagrange rows
     double *ss;                // optional: the workgroup's sum of squares of the rows written
-    const int *done, *pore_of; // optional: skip a workgroup all of whose pores are done
+    const int *done, *pore_of; // optional: skip a workgroup all of whose pores (null pore_of: the problem) are done
 };
 
 // code and source node of padded position q, which may lie outside the padded copy (map_pad in 1D)
@@ -199,7 +199,7 @@ __global__ __launch_bounds__(kLineBlock, B == 1 ? 2 : 6) void k_line(LineArgs<T>
         int live = 0;
         for (int t = tid; t < TN; t += kLineBlock) {
             int src, refl;
-            if (line_map(g, p0 + t, src, refl) == 0 && !a.done[a.pore_of[src]]) live = 1;
+            if (line_map(g, p0 + t, src, refl) == 0 && !a.done[a.pore_of ? a.pore_of[src] : 0]) live = 1;
         }
         if (!__syncthreads_or(live)) return;
     }
