@@ -1,0 +1,84 @@
+"""One-component 2D rows on the matrix cores (k_plane) against the separate kernels (TMI_PLANE2D=0).
+
+Tolerance: the same FP64 (FP32) products summed in another order; 1e-12 (1e-5) of the row block's
+largest value, the parity bounds of the separate kernels themselves.
+"""
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+
+from tramonto_amd.batch import BatchSpec, DeviceBatch, rough_slit_pore_batch_2d  # noqa: E402
+from tramonto_amd.device import DeviceProblem  # noqa: E402
+from tramonto_amd.problem import (IN_BULK, IN_WALL, PERIODIC, REFLECT, ProblemSpec, SplitMix64, rough_slit_pore_2d,  # noqa: E402
+                                  rough_wall_2d, small_case)
+
+
+def _box(nx, ny, bc, cut=1.5, dx=0.1, func=0, seed=3):
+    rho = 0.5 * (1 + 0.2 * SplitMix64(seed).uniform(nx * ny, -1, 1))
+    return ProblemSpec(name="box", ndim=2, ncomp=1, nx=[nx, ny], dx=[dx, dx], bc=bc, type_func=func,
+                       type_attr=0 if cut else -1, hs_diam=[1.0], sigma_ff=np.ones((1, 1)), eps_ff=np.full((1, 1), 0.8),
+                       cut_ff=np.full((1, 1), cut), rho_b=[0.5], rho0=rho[None, :])
+
+
+SPECS = {
+    "2d_periodic": lambda: small_case("2d_periodic"),
+    "2d_wall_reflect": lambda: small_case("2d_wall_reflect"),
+    "2d_wall_fmt4": lambda: small_case("2d_wall_fmt4"),
+    "2d_rough_wall": lambda: small_case("2d_rough_wall"),
+    "ragged": lambda: _box(33, 47, [[PERIODIC, PERIODIC], [IN_BULK, REFLECT]], func=2),
+    "reflect_both": lambda: _box(17, 31, [[REFLECT, REFLECT], [REFLECT, IN_WALL]]),
+    "hard_only": lambda: _box(18, 16, [[IN_BULK, IN_WALL], [PERIODIC, PERIODIC]], cut=0.0),
+    "reach_plus_one": lambda: _box(20, 35, [[IN_BULK, IN_BULK], [IN_WALL, IN_BULK]], cut=0.6),   # attraction reach FMT + 1
+    "fine": lambda: rough_wall_2d(seed=5, nx=113, ny=112, dx=0.05),   # one 16-wave workgroup per CU
+}
+
+
+def _compare(a, b, blocks, tol):
+    for lo, hi in blocks:
+        if lo < hi:
+            scale = float(a[lo:hi].abs().max())
+            assert float((a[lo:hi] - b[lo:hi]).abs().max()) <= tol * scale, (lo, hi)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", list(SPECS) + ["batch", "batch_walls"])
+def test_plane_matches_separate_kernels(kind, monkeypatch):
+    batch = kind.startswith("batch")
+    monkeypatch.setenv("TMI_PRECOND", "diag")
+    if batch:
+        spec = rough_slit_pore_batch_2d(npores=3, seed=4, nx=53, h_range=(3.0, 5.0))
+        if kind == "batch_walls":
+            spec = BatchSpec([rough_slit_pore_2d(seed=i, nx=37, ny=ny, eps_ff=0.5) for i, ny in enumerate((33, 48, 49))])
+            for p in spec.pores:
+                p.bc = [[IN_WALL, IN_WALL], [IN_WALL, IN_WALL]]
+        make = lambda: DeviceBatch(spec)   # noqa: E731
+    else:
+        spec = SPECS[kind]()
+        make = lambda: DeviceProblem(spec)   # noqa: E731
+    monkeypatch.setenv("TMI_MF_FFT", "0")
+    monkeypatch.setenv("TMI_FMT_FFT", "0")
+    monkeypatch.setenv("TMI_PLANE2D", "0")
+    rows = make()
+    for v in ("TMI_MF_FFT", "TMI_FMT_FFT"):
+        monkeypatch.delenv(v)
+    monkeypatch.setenv("TMI_PLANE2D", "2")   # the matrix-core form without the timing against the others
+    plane = make()
+    C, R = 1, 8
+    x = rows.initial_state()
+    blocks = ((0, C), (C, C + R), (C + R, x.shape[0]))
+    _compare(x, plane.initial_state(), blocks, 1e-12)
+    g = torch.Generator(device="cuda").manual_seed(1)
+    noise = lambda: 2 * torch.rand(x.shape, generator=g, device="cuda", dtype=torch.float64) - 1   # noqa: E731
+    x[C:] *= 1.0 + 0.01 * noise()[C:]
+    Fa, sa = rows.fill_residual(x)
+    Fb, sb = plane.fill_residual(x)
+    _compare(Fa, Fb, blocks, 1e-12)
+    assert abs(sa - sb) <= 1e-12 * abs(sa)
+    v = noise()
+    _compare(rows.apply_jacobian(x, v), plane.apply_jacobian(x, v), blocks, 1e-12)
+    _compare(rows.apply_jacobian(x, v, fp32=True), plane.apply_jacobian(x, v, fp32=True), blocks, 1e-5)
+    if not batch:   # Schur product, right-hand side and back-substitution: one Newton update
+        da, _ = rows.schur_solve(x, Fa, rtol=1e-12)
+        db, _ = plane.schur_solve(x, Fa, rtol=1e-12)
+        _compare(da, db, blocks, 1e-8)

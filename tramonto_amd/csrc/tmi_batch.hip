@@ -695,15 +695,15 @@ static void stage_cycle_steps(Problem &P, BatchWork &W, const double *x, double 
 {
     const int Pn = W.P, C = P.p.ncomp, N = P.N, m = W.m;
     const long long n2 = (long long)W.n2;
-    const bool line = schur_in_line(P), one = ortho_fits((long long)C * W.longest, C, N, m);
+    const bool fused = schur_one_launch(P), one = ortho_fits((long long)C * W.longest, C, N, m);
     const int *done = one ? W.gs.done : nullptr;   // the separate kernels go on with every pore's vectors
     for (int k = k0; k < k1; ++k) {
         double *Vk = W.V + (size_t)k * n2;
-        if (line) {
+        if (fused) {
             if (prec == TMI_PREC_MIXED)
-                line_schur<float>(P, x, Vk, W.dinv, W.w, done, s);
+                one_launch_schur<float>(P, x, Vk, W.dinv, W.w, done, s);
             else
-                line_schur<double>(P, x, Vk, W.dinv, W.w, done, s);
+                one_launch_schur<double>(P, x, Vk, W.dinv, W.w, done, s);
         } else {
             dev_mul(W.dinv, Vk, W.z, n2, s);
             schur_apply(P, x, W.z, W.t1, W.w, prec, s);
@@ -903,7 +903,7 @@ bool gmres_line(Problem &P, const double *x, const double *bS, double *x2, doubl
     constexpr int kLineSteps = 4, kLineMax = 8192;
     const int C = P.p.ncomp, N = P.N;
     const long long n = (long long)C * N;
-    if (P.npores > 0 || !schur_in_line(P) || n > kLineMax || m > kOrthoMaxM) return false;
+    if (P.npores > 0 || !line_available(P) || !schur_one_launch(P) || n > kLineMax || m > kOrthoMaxM) return false;
     if (P.line_gs_m != m) {
         (void)hipFree(P.d_line_gs);
         (void)hipFree(P.d_line_gi);

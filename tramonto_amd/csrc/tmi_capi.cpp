@@ -611,6 +611,8 @@ Problem *create_problem(const tmi_params &p_in, const double *vext, const unsign
         // FFT forms of the stencil sums on 2D/3D grids: the mean-field sums when the attraction
         // stencils are wide (TMI_MF_FFT=1 forces it, 0 keeps the direct sums), the FMT sums when
         // that form fills faster (TMI_FMT_FFT=1 / 0 forces the FFT / direct form)
+        if (!symbol_only) plane_setup(*P);
+        if (batch) plane_set(*P, true);
         if (nd >= 2 && !batch) {   // batches of 2D pieces keep the direct sums (their padded copy has gap rows)
             const char *fe = std::getenv("TMI_MF_FFT"), *fm = std::getenv("TMI_FMT_FFT");
             long long lsum = 0;
@@ -618,6 +620,8 @@ Problem *create_problem(const tmi_params &p_in, const double *vext, const unsign
                 for (int q = 0; q < C * C; ++q) lsum += P->hs[TMI_UATT][q].L;
             const bool mf = p.type_attr >= 0 && (fe ? std::string(fe) == "1" : lsum >= kFftMinStencil);
             const bool fmt = !(fm && std::string(fm) == "0");
+            // a forced direct form of any of the sums means the separate kernels
+            if ((fe && std::string(fe) == "0") || !fmt) plane_free(*P);
             fft_setup(*P, mf, fmt);
             if (!symbol_only) {
                 choose_fmt_form(*P);
@@ -628,6 +632,7 @@ Problem *create_problem(const tmi_params &p_in, const double *vext, const unsign
             precond_setup(*P);
             // an unused plan is kept only for the bulk preconditioner
             if (P->fft && !fft_mf(*P) && !fft_fmt(*P) && !precond_available(*P)) fft_free(*P);
+            if (plane_built(*P) && !plane_on(*P)) plane_free(*P);
         }
     } catch (...) {
         destroy_problem(P);
@@ -651,6 +656,7 @@ void destroy_problem(Problem *P)
         }
     free_batch_work(*P);
     fft_free(*P);
+    plane_free(*P);
     free_geometry_maps(P->pad_u);
     free_geometry_maps(P->pad_f);
     (void)hipFree(P->d_pore_off);

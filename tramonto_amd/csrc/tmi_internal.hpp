@@ -114,6 +114,7 @@ struct Grid {
 struct Problem;
 struct BatchWork;
 struct FftPlan;
+struct PlanePlan;
 
 // kernel-side launch helpers (tmi_kernels.hip)
 template <typename T>
@@ -166,6 +167,7 @@ struct Problem {
     double *d_mu = nullptr;        // [C][N] -ln rho_b - beta mu_hs,ex - beta mu_att of the node's pore
     std::vector<double> pore_rho_b;   // [npores][C]
     BatchWork *batch_work = nullptr;  // batched Newton buffers and graphs (tmi_batch.hip)
+    PlanePlan *plane = nullptr;       // one-component 2D rows on the matrix cores (tmi_plane.hip)
     FftPlan *fft = nullptr;           // FFT forms of the stencil sums (tmi_fft.hip), 2D/3D
     // solver scratch
     double *d_newton = nullptr;   // [2][nunk][N]: F and dx of tmi_newton_solve, from its first call on
@@ -228,26 +230,57 @@ void launch_init_fields(Problem &P, double *x, hipStream_t s);
 //   t1 = A12 x2 (block-1 rows of J [x2;0]);  y2 = A22 x2 + A21 t1
 template <typename T>
 void launch_schur_apply(Problem &P, const double *x, const double *x2, double *t1, double *y2, hipStream_t s);
-bool schur_in_line(const Problem &P);   // ... in one launch (line_schur)
+bool schur_one_launch(const Problem &P);   // ... through one_launch_schur
 // bS = b2 + A21 b1 (b full length)
 void launch_schur_rhs(Problem &P, const double *x, const double *b, double *bS, hipStream_t s);
 // x1 = A12 x2 - b1 written into dx (full length), x2 already in dx[0:C*N]
 void launch_schur_backsub(Problem &P, const double *x, const double *b, double *dx, hipStream_t s);
 
-// 1D rows in one launch (tmi_line.hip).  line_rows_el: the rho-bar and mean-field rows of rho (null:
+// Rows in one launch: of 1D problems (line_*, tmi_line.hip) and of one-component 2D problems on the
+// matrix cores (plane_*, tmi_plane.hip).  *_rows_el: the rho-bar and mean-field rows of rho (null:
 // none) and the Euler-Lagrange rows (out_el null: none), which read x and, in the linear mode, the
-// direction's rho-bar rows dn_rb; ss (optional): line_partials sums of the squares of the rows written.
-// line_schur: y2 = S (mul x2) (mul null: S x2); done (optional, batches): pores whose rows are not wanted.
+// direction's rho-bar rows dn_rb; ss (optional): *_partials sums of the squares of the rows written.
+// *_schur: y2 = S (mul x2) (mul null: S x2); done (optional, batches): pores whose rows are not wanted.
 bool line_available(const Problem &P);
 long long line_partials(const Problem &P);
 template <typename T>
 void line_rows_el(Problem &P, bool linear, const double *rho, const double *in_rb, const double *sub_rb, double *out_rb,
                   const double *in_mf, const double *sub_mf, double *out_mf, const double *x, const double *dn_rb,
-                  const double *in_rho, const double *el_mf, const double *add, double *out_el, hipStream_t s,
-                  double *ss = nullptr);
+                  const double *in_rho, const double *el_mf, const double *add, double *out_el, hipStream_t s, double *ss);
 template <typename T>
 void line_schur(Problem &P, const double *x, const double *x2, const double *mul, double *y2, const int *done,
                 hipStream_t s);
+void plane_setup(Problem &P);
+void plane_free(Problem &P);
+void plane_set(Problem &P, bool on);
+bool plane_built(const Problem &P);
+bool plane_on(const Problem &P);
+long long plane_partials(const Problem &P);
+template <typename T>
+void plane_rows_el(Problem &P, bool linear, const double *rho, const double *in_rb, const double *sub_rb, double *out_rb,
+                   const double *in_mf, const double *sub_mf, double *out_mf, const double *x, const double *dn_rb,
+                   const double *in_rho, const double *el_mf, const double *add, double *out_el, hipStream_t s, double *ss);
+template <typename T>
+void plane_schur(Problem &P, const double *x, const double *x2, const double *mul, double *y2, const int *done,
+                 hipStream_t s);
+// whichever of the two serves the problem
+inline bool one_launch(const Problem &P) { return line_available(P) || plane_on(P); }
+inline long long one_launch_partials(const Problem &P) { return plane_on(P) ? plane_partials(P) : line_partials(P); }
+template <typename T>
+inline void one_launch_rows_el(Problem &P, bool linear, const double *rho, const double *in_rb, const double *sub_rb,
+                               double *out_rb, const double *in_mf, const double *sub_mf, double *out_mf, const double *x,
+                               const double *dn_rb, const double *in_rho, const double *el_mf, const double *add,
+                               double *out_el, hipStream_t s, double *ss = nullptr)
+{
+    (plane_on(P) ? plane_rows_el<T> : line_rows_el<T>)(P, linear, rho, in_rb, sub_rb, out_rb, in_mf, sub_mf, out_mf, x, dn_rb,
+                                                       in_rho, el_mf, add, out_el, s, ss);
+}
+template <typename T>
+inline void one_launch_schur(Problem &P, const double *x, const double *x2, const double *mul, double *y2, const int *done,
+                             hipStream_t s)
+{
+    (plane_on(P) ? plane_schur<T> : line_schur<T>)(P, x, x2, mul, y2, done, s);
+}
 
 // Per-segment GMRES bookkeeping (tmi_batch.hip): P independent Arnoldi processes over the segments
 // [off[p], off[p + 1]) of one packed vector.

@@ -2030,7 +2030,17 @@ void autotune_rows1d(Problem &P)
 // used for both products where it fits, unless TMI_FFT_XFUSE=0).
 void choose_fmt_form(Problem &P)
 {
-    if (!fft_fmt_available(P)) return;
+    if (!fft_fmt_available(P)) {
+        plane_set(P, true);   // against the separate direct kernels
+        return;
+    }
+    const char *pe = std::getenv("TMI_PLANE2D");
+    if (pe && std::string(pe) == "2" && plane_built(P)) {   // no timing
+        plane_set(P, true);
+        fft_set_fmt(P, false);
+        fft_set_fused(P, 0);
+        return;
+    }
     const char *env = std::getenv("TMI_FMT_FFT"), *xf = std::getenv("TMI_FFT_XFUSE");
     if (env) {
         fft_set_fmt(P, std::string(env) == "1");
@@ -2040,10 +2050,12 @@ void choose_fmt_form(Problem &P)
     const size_t n = (size_t)P.nunk * P.N;
     double *x = nullptr, *F = nullptr;
     hipEvent_t e0 = nullptr, e1 = nullptr;
-    // forms: 0 direct; 1 + mask: FFT with the fused x pass for the products in mask (bit 0 density, bit 1 EL)
+    // forms: 0 direct (2D, one component: every row on the matrix cores where its windows fit); 1 + mask:
+    // FFT with the fused x pass for the products in mask (bit 0 density, bit 1 EL)
     const int nform = fft_fused_available(P) ? 5 : 2;
     float ms[5] = {0.f, 0.f, 0.f, 0.f, 0.f};
     auto set_form = [&](int form) {
+        plane_set(P, form == 0);
         fft_set_fmt(P, form > 0);
         fft_set_fused(P, form > 0 ? form - 1 : 0);
     };
@@ -2090,13 +2102,13 @@ void residual_impl(Problem &P, const double *x, double *F, hipStream_t s, hipEve
     const size_t N = P.N;
     long long n_rb = 0, n_el = 0;
     if (P.hw_fwd.nrows || P.one_size) ss = nullptr;   // the rho-bar rows change after the fused passes
-    if (!ev && line_available(P)) {
-        line_rows_el<double>(P, false, x + P.iu_rho * N, x + P.iu_rb * N, nullptr, F + P.iu_rb * N,
+    if (!ev && one_launch(P)) {
+        one_launch_rows_el<double>(P, false, x + P.iu_rho * N, x + P.iu_rb * N, nullptr, F + P.iu_rb * N,
                              P.nmf ? x + P.iu_mf * N : nullptr, nullptr, F + P.iu_mf * N, x, nullptr, x + P.iu_rho * N,
                              P.nmf ? x + P.iu_mf * N : nullptr, nullptr, F + P.iu_rho * N, s, ss);
         hw_apply(P.hw_fwd, x + P.iu_rho * N, F + P.iu_rb * N, s);
         one_size_rows(P, x + P.iu_rb * N, F + P.iu_rb * N, s);
-        if (nss) *nss = ss ? line_partials(P) : 0;
+        if (nss) *nss = ss ? one_launch_partials(P) : 0;
         return;
     }
     if (ev) TMI_HIP_CHECK(hipEventRecord(ev[0], s));
@@ -2233,13 +2245,13 @@ long long residual_sumsq_partials(const Problem &P)
 {
     long long cap = 0;
     fft_ss_buffer(P, &cap);
-    return std::max<long long>({cap, line_partials(P), 1024});
+    return std::max<long long>({cap, one_launch_partials(P), 1024});
 }
 
 void residual_sumsq_device(Problem &P, const double *x, double *F, double *partials, double *sumsq_d, hipStream_t s)
 {
     long long cnt = 0;
-    residual_impl(P, x, F, s, nullptr, P.fft || line_available(P) ? partials : nullptr, &cnt);
+    residual_impl(P, x, F, s, nullptr, P.fft || one_launch(P) ? partials : nullptr, &cnt);
     if (cnt > 0) {
         hipLaunchKernelGGL(k_sum_partials, dim3(1), dim3(kSumBlock), 0, s, partials, (int)cnt, sumsq_d, nullptr);
     } else {   // the blocks and order of dev_dot
@@ -2256,7 +2268,7 @@ double residual_sumsq(Problem &P, const double *x, double *F, hipStream_t s)
 {
     long long cap = 0, cnt = 0;
     double *ss = fft_ss_buffer(P, &cap);
-    if (line_available(P) && line_partials(P) <= kRedPartials) {
+    if (one_launch(P) && one_launch_partials(P) <= kRedPartials) {
         ss = P.d_red;
         cap = kRedPartials;
     }
@@ -2274,8 +2286,8 @@ template <typename T>
 void launch_jvp(Problem &P, const double *x, const double *v, double *Jv, hipStream_t s)
 {
     const size_t N = P.N;
-    if (line_available(P) && !P.jac_ref) {
-        line_rows_el<T>(P, true, v + P.iu_rho * N, v + P.iu_rb * N, nullptr, Jv + P.iu_rb * N,
+    if (one_launch(P) && !P.jac_ref) {
+        one_launch_rows_el<T>(P, true, v + P.iu_rho * N, v + P.iu_rb * N, nullptr, Jv + P.iu_rb * N,
                         P.nmf ? v + P.iu_mf * N : nullptr, nullptr, Jv + P.iu_mf * N, x, v + P.iu_rb * N,
                         v + P.iu_rho * N, P.nmf ? v + P.iu_mf * N : nullptr, nullptr, Jv + P.iu_rho * N, s);
         hw_apply(P.hw_fwd, v + P.iu_rho * N, Jv + P.iu_rb * N, s);
@@ -2297,8 +2309,8 @@ template void launch_jvp<float>(Problem &, const double *, const double *, doubl
 void launch_init_fields(Problem &P, double *x, hipStream_t s)
 {
     const size_t N = P.N;
-    if (line_available(P))
-        line_rows_el<double>(P, false, x + P.iu_rho * N, nullptr, nullptr, x + P.iu_rb * N, nullptr, nullptr,
+    if (one_launch(P))
+        one_launch_rows_el<double>(P, false, x + P.iu_rho * N, nullptr, nullptr, x + P.iu_rb * N, nullptr, nullptr,
                              x + P.iu_mf * N, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, s);
     else
         rb_mf_rows<double>(P, x + P.iu_rho * N, false, nullptr, nullptr, x + P.iu_rb * N, nullptr, nullptr,
@@ -2307,17 +2319,17 @@ void launch_init_fields(Problem &P, double *x, hipStream_t s)
     TMI_HIP_CHECK(hipGetLastError());
 }
 
-// the Schur product in one launch: hard-surface corrections and the reference's Jacobian need the rows
-bool schur_in_line(const Problem &P) { return line_available(P) && !P.jac_ref && P.hw_fwd.nrows == 0; }
+// the Schur product without the rows: hard-surface corrections and the reference's Jacobian need the rows
+bool schur_one_launch(const Problem &P) { return one_launch(P) && !P.jac_ref && P.hw_fwd.nrows == 0; }
 
-// y2 = A22 x2 + A21 t1, t1 = A12 x2 the rho-bar and mean-field rows of J [x2; 0] (scratch: the one-launch
-// 1D form does not write it)
+// y2 = A22 x2 + A21 t1, t1 = A12 x2 the rho-bar and mean-field rows of J [x2; 0] (scratch: the
+// one-launch forms do not write it)
 template <typename T>
 void launch_schur_apply(Problem &P, const double *x, const double *x2, double *t1, double *y2, hipStream_t s)
 {
     const size_t N = P.N;
-    if (schur_in_line(P)) {
-        line_schur<T>(P, x, x2, nullptr, y2, nullptr, s);
+    if (schur_one_launch(P)) {
+        one_launch_schur<T>(P, x, x2, nullptr, y2, nullptr, s);
         return;
     }
     rb_mf_rows<T>(P, x2, true, nullptr, nullptr, t1, nullptr, nullptr, t1 + (size_t)P.nrb * N, s);
@@ -2333,8 +2345,8 @@ template void launch_schur_apply<float>(Problem &, const double *, const double 
 void launch_schur_rhs(Problem &P, const double *x, const double *b, double *bS, hipStream_t s)
 {
     const size_t N = P.N;
-    if (line_available(P) && !P.jac_ref) {
-        line_rows_el<double>(P, true, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, x, b + P.iu_rb * N,
+    if (one_launch(P) && !P.jac_ref) {
+        one_launch_rows_el<double>(P, true, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, x, b + P.iu_rb * N,
                              nullptr, P.nmf ? b + P.iu_mf * N : nullptr, b + P.iu_rho * N, bS, s);
         return;
     }
@@ -2348,8 +2360,8 @@ void launch_schur_backsub(Problem &P, const double *x, const double *b, double *
 {
     (void)x;
     const size_t N = P.N;
-    if (line_available(P))
-        line_rows_el<double>(P, true, dx + P.iu_rho * N, nullptr, b + P.iu_rb * N, dx + P.iu_rb * N, nullptr,
+    if (one_launch(P))
+        one_launch_rows_el<double>(P, true, dx + P.iu_rho * N, nullptr, b + P.iu_rb * N, dx + P.iu_rb * N, nullptr,
                              P.nmf ? b + P.iu_mf * N : nullptr, P.nmf ? dx + P.iu_mf * N : nullptr, nullptr, nullptr,
                              nullptr, nullptr, nullptr, nullptr, s);
     else
