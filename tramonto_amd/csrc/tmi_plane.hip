@@ -16,9 +16,11 @@
 // four SIMDs in turn, so each SIMD gets an equal part of all three.  A Schur product needs the rho-bar
 // sums before the adjoint fields: k_plane_schur forms the fields at the nodes, k_plane then runs the
 // attraction and Euler-Lagrange sums.
-// Bound by the FP64 matrix rate (64 cycles a product and SIMD): 256^2 nodes at dx = 0.05 sigma, attraction
-// reach 2.5 sigma: 1.0e6 products, 26 us.  Measured there: PLANE_ROUGH; 16 pieces of 64 columns at
-// dx = 0.1 sigma (73,088 nodes), Schur product: PLANE_SLITS.
+// Bound by the FP64 matrix rate (64 cycles a product and SIMD) and the window loads before it: 256^2 nodes
+// at dx = 0.05 sigma, attraction reach 2.5 sigma: 1.0e6 products, 26 us; a workgroup spends 40k cycles on
+// its windows and 82k on 62k cycles' worth of products.  There a fill's rows take 59 us, the fill 81 us
+// (132 us as FFT sums); 16 pieces of 64 columns at dx = 0.1 sigma (73,088 nodes): Schur product 42 us
+// (98 us in separate launches), mixed Newton solve of the batch 9.5 ms (16.3 ms).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
