@@ -336,7 +336,7 @@ def bench_workload(spec, label, args, newton_tol=1e-8, newton=True):
         elif fused:
             ft = fx
             tr = XPROD_TRAFFIC_MIB.get(label)
-            kernel = "k_fft_xprod_reg" if dp.info.fft_xreg else "k_fft_xprod"
+            kernel = "k_fft_xgroup" if dp.info.fft_xreg else "k_fft_xprod"
             note = ("fused x passes of one fill: input pairs and distinct spectrum tables read, output pairs "
                     "written (algorithmic), HIP events on the launch stream")
         else:

@@ -81,10 +81,23 @@ struct Term {
     int odd;   // axis in which the table is odd (vector delta d: d), -1 if even
     double coef;
 };
+struct ProductStep;
 struct TermList {
     int nin = 0, nout = 0;
+    ProductStep *steps = nullptr;      // the terms for the register form and each output pair's first step
+    int *start = nullptr;              // (and one past the last), in device memory
     int first[kMaxIn + 2] = {};   // one past the last field is the running end while a list is built
     Term term[kMaxTerms] = {};
+};
+
+// One step of a product in the register form of the fused x pass: an output pair gets, from the two fields
+// of input pair jp, (rot ? i : 1) sum over e of coef[e] K_at[e](k) X_h(k) (times i for output b), e = h
+// (output a, field h) and 2 + h (output b).  The steps of an output pair are in the order of jp.
+struct ProductStep {
+    long long at[4];   // element offset of the table from tk, or -1 - offset from uk
+    double coef[4];
+    int odd[4];        // bits 2 and 3: odd in y, in z
+    int jp, rot;
 };
 
 struct FftPlan {
@@ -1341,182 +1354,210 @@ __global__ __launch_bounds__(kFftBlock) void k_fft_xprod(const Cx<T> *__restrict
     }
 }
 
-// Primary x-lines of the fused register x pass, numbered l = 0, 1, ...: every line (y, z) of the
-// planes 0 < z < M2 - z (z-major, y fastest), then the self-mirror planes (z = 0, and z = M2/2
-// when M2 is even) with 0 <= y <= M1/2.  The mirror lines (-y, -z) of the primary lines are the
-// other lines, each once, except the self-mirror lines (y, z) = (-y, -z).  False past the last.
-__device__ inline bool xprod_line(int l, int M1, int M2, int &y, int &z)
+// Fused x pass with the x transforms in registers, for x-lines of length M = R1 R2 (R2 <= R1 <= 16, powers
+// of two).  A workgroup takes 64 / R2 lines, whole groups of nl = 4 lines (+-y, +-z) (nl = 2: (+-y, z) on
+// grids without z), so that the negative of every line is among them and the lines of a group share
+// their folded table rows; a wave transforms one pair field of all of them.  Lane (i, n2) of a wave
+// loads elements R2 n1 + n2 of line i, runs an R1-point DFT, the twiddles W_M^(n2 k1), a transpose through
+// LDS and R1/R2 R2-point DFTs.  The spectra of up to `slots` input pairs then stand in LDS (index
+// k + k / R2: rows of R2 + 1); each wave forms one output pair at a time in registers, at k = R2 n1 + n2, the order
+// its inverse transform starts from, and stores it.  Products of more input pairs than slots
+// accumulate over several fills of the slots (every wave then has one output pair only: nop <= waves).
+// Its floor is HBM (inputs, tables and outputs once: 62 and 49 us for the density and Euler-Lagrange products
+// of three components at 128^3); with 2 waves per SIMD it is bound by latency, LDS and FP64 issue: 135 and
+// 109 us there, 228 and 132 us as x pass, product kernel and x pass (FP32: 67 and 42, 142 and 78 us); one
+// component at 64^3: 26 us for both products, 30 us with one pair of lines per group and the outputs'
+// spectra accumulated in registers.  Two waves instead of four for the density product: 177 us; one or three slots for
+// the Euler-Lagrange product: 117 and 128 us.
+__device__ __forceinline__ void wave_lds_sync()
 {
-    const int zr = (M2 - 1) / 2;
-    if (l < zr * M1) {
-        z = 1 + l / M1;
-        y = l - (z - 1) * M1;
-        return true;
-    }
-    l -= zr * M1;
-    const int ms = M1 / 2 + 1, nself = (M2 > 1 && M2 % 2 == 0) ? 2 : 1;
-    const int sp = l / ms;
-    if (sp >= nself) return false;
-    z = sp ? M2 / 2 : 0;
-    y = l - sp * ms;
-    return true;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // LDS operations of one wave stay in order
+    __builtin_amdgcn_wave_barrier();
 }
-inline long long xprod_primary_lines(int M1, int M2)
+template <typename T, int R1, int R2, int NL>
+__global__ __launch_bounds__(256, (sizeof(T) == 8 ? 2 : 3) + (R1 == 8 ? 1 : 0)) void k_fft_xgroup(const Cx<T> *__restrict__ Zin, Cx<T> *__restrict__ Oout,
+                                                       long long ns, int M1, int M2, long long S1, long long S2, int slots,
+                                                       int alias, const Cx<T> *__restrict__ twtab,
+                                                       const T *__restrict__ tk, const T *__restrict__ uk, TabGeo tg,
+                                                       const ProductStep *__restrict__ steps, const int *__restrict__ start,
+                                                       int nip, int nop, int xcd)
 {
-    const int zr = (M2 - 1) / 2, nself = (M2 > 1 && M2 % 2 == 0) ? 2 : 1;
-    return (long long)zr * M1 + (long long)nself * (M1 / 2 + 1);
-}
-
-// Fused x pass with the x transforms in registers, for x-lines of length M = R1 R2 (R1 = 8 or 16,
-// R2 = 8 or 4) and NOP output pairs whose NOP x R1 spectrum values fit in registers.  The
-// workgroup has 2 L R2 threads: lanes (i, n2) of the first half take primary line i of L
-// consecutive primary x-lines (y, z) (xprod_line), the second half their mirror lines (-y, -z),
-// so every line is loaded once.  Per input pair every lane loads elements R2 n1 + n2 of its
-// line, runs an R1-point DFT, the twiddles W_M^(n2 k1), a transpose through LDS and R1/R2
-// R2-point DFTs, leaving spectrum values k = n2 + R2 q + R1 k2; those go back to LDS in natural
-// order, every lane reads the partner line's spectrum at -k (the spectrum of its line's
-// negative), splits the pair and accumulates the terms of its own line into output pairs held
-// in registers (the table row of a line and of its mirror is the same folded row).  The outputs
-// return through LDS one pair at a time, through the same two-stage transform with SIGN +1,
-// and both halves store their lines (a self-mirror line once) for the y and z passes.
-template <typename T, int R1, int R2, int NOP>
-__global__ __launch_bounds__(2 * (64 / R2) * R2) void k_fft_xprod_reg(const Cx<T> *__restrict__ Zin,
-                                                                    Cx<T> *__restrict__ Oout, long long ns, int M1,
-                                                                    int M2, long long S1, long long S2, int L,
-                                                                    const Cx<T> *__restrict__ twtab,
-                                                                    const T *__restrict__ tk, const T *__restrict__ uk,
-                                                                    TabGeo tg, TermList tl, int xcd)
-{
-    constexpr int M = R1 * R2, LD = M + 1;
+    constexpr int M = R1 * R2, L = 64 / R2, ROW = R2 + 1, LD = R1 * ROW + 1, NC = R1 / NL;
+    typedef const ProductStep __attribute__((address_space(4))) *Steps;   // scalar loads
+    typedef const int __attribute__((address_space(4))) *Ints;
+    const Steps list = (Steps)steps;
+    const Ints first = (Ints)start;
     extern __shared__ char smem_raw[];
     Cx<T> *tw = reinterpret_cast<Cx<T> *>(smem_raw);   // [M]
-    Cx<T> *buf = tw + M;                               // [2 L][LD]: primary lines, then mirror lines
-    const int tid = threadIdx.x, half = tid / (L * R2), r0 = tid - half * L * R2;
-    const int i = r0 / R2, n2 = r0 - i * R2;
-    const int nth = 2 * L * R2;
-    for (int j = tid; j < M; j += nth) tw[j] = twtab[j];
-    int yp = 0, zp = 0;
-    const bool live = xprod_line((xcd ? xcd_item(blockIdx.x, gridDim.x) : (int)blockIdx.x) * L + i, M1, M2, yp, zp);
-    const int ym = yp ? M1 - yp : 0, zm = zp ? M2 - zp : 0;
-    const bool self = ym == yp && zm == zp;
-    const int y = half ? ym : yp, z = half ? zm : zp;   // this lane's line
+    Cx<T> *spec = tw + M;                              // [slots][L][LD]
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nw = blockDim.x >> 6;
+    T *work = reinterpret_cast<T *>(alias ? spec : spec + (size_t)slots * L * LD) + (size_t)wave * L * LD;
+    T *stage = alias ? reinterpret_cast<T *>(spec + (size_t)slots * L * LD) + wave * 256 : work;   // [4][64]
+    for (int j = threadIdx.x; j < M; j += blockDim.x) tw[j] = twtab[j];
+    const int i = lane / R2, n2 = lane - i * R2;
+    const int hy = M1 / 2 + 1, ngrp = hy * (M2 / 2 + 1);
+    const int g = (xcd ? xcd_item(blockIdx.x, gridDim.x) : (int)blockIdx.x) * (L / NL) + i / NL;
+    const bool live = g < ngrp;
+    const int y0 = live ? g % hy : 0, z0 = live ? g / hy : 0;
+    const int ym = y0 ? M1 - y0 : 0, zm = z0 ? M2 - z0 : 0;
+    const bool my = i & 1, mz = NL == 4 && (i & 2);
+    const int y = my ? ym : y0, z = mz ? zm : z0;
+    const bool store = live && !(my && ym == y0) && !(mz && zm == z0);   // a line and itself mirrored: stored once
     const long long row = (long long)y * S1 + (long long)z * S2;
-    const long long trow = tab_fold(tg, 1, y) * tg.p1 + tab_fold(tg, 2, z) * tg.p2;   // the line's table row
-    const bool neg_y = tab_neg(tg, 1, y), neg_z = tab_neg(tg, 2, z);
-    Cx<T> *mine = buf + (size_t)(half * L + i) * LD;                 // this lane's line in LDS
-    const Cx<T> *partner = buf + (size_t)((1 - half) * L + i) * LD;  // the line of the negative spectrum
-    // spectrum position of register r (= q R2 + k2)
-    auto kpos = [&](int r) { return n2 + R2 * (r / R2) + R1 * (r % R2); };
-    Cx<T> acc[NOP][R1];
-#pragma unroll
-    for (int p = 0; p < NOP; ++p)
-#pragma unroll
-        for (int r = 0; r < R1; ++r) acc[p][r] = Cx<T>{(T)0, (T)0};
+    const unsigned trow = (unsigned)(tab_fold(tg, 1, y) * tg.p1 + tab_fold(tg, 2, z) * tg.p2) + (i % NL) * R2 + n2;
+    const int negs = (tab_neg(tg, 1, y) ? 4 : 0) | (tab_neg(tg, 2, z) ? 8 : 0);
+    const int own = i * LD + n2, neg = (i ^ (NL - 1)) * LD;
+    const int negk = neg + (n2 ? ROW * (R1 - 1) + R2 - n2 : ROW * R1);   // -k at n1 = 0 (n2 > 0); ROW less per n1
     __syncthreads();
-    // forward transform of the lane's line from registers v (elements R2 n1 + n2) into X (positions kpos)
-    auto forward = [&](Cx<T> (&v)[R1], Cx<T> (&X)[R1]) {
-        dft_reg<R1, -1>(v);
+    Cx<T> acc[R1];
+    auto clear = [&]() {
 #pragma unroll
-        for (int k1 = 0; k1 < R1; ++k1) mine[k1 * R2 + n2] = cmul(v[k1], tw[n2 * k1]);
-        __syncthreads();
+        for (int r = 0; r < R1; ++r) acc[r] = Cx<T>{(T)0, (T)0};
+    };
+    // input pair jp into slot sl
+    auto forward = [&](int jp, int sl) {
+        const Cx<T> *src = Zin + (size_t)jp * ns + row + n2;
+        Cx<T> v[R1];
+#pragma unroll
+        for (int n1 = 0; n1 < R1; ++n1) v[n1] = live ? src[R2 * n1] : Cx<T>{(T)0, (T)0};
+        dft_reg<R1, -1>(v);
+        Cx<T> *b = spec + (size_t)sl * L * LD + i * LD;
+#pragma unroll
+        for (int k1 = 0; k1 < R1; ++k1) b[k1 * ROW + n2] = cmul(v[k1], tw[n2 * k1]);
+        wave_lds_sync();
 #pragma unroll
         for (int q = 0; q < R1 / R2; ++q) {
-            const int k1 = n2 + R2 * q;
-            Cx<T> u[R2];
 #pragma unroll
-            for (int m = 0; m < R2; ++m) u[m] = mine[k1 * R2 + m];
-            dft_reg<R2, -1>(u);
-#pragma unroll
-            for (int k2 = 0; k2 < R2; ++k2) X[q * R2 + k2] = u[k2];
+            for (int m = 0; m < R2; ++m) v[q * R2 + m] = b[(n2 + R2 * q) * ROW + m];
+            dft_reg<R2, -1>(v + q * R2);
         }
-        __syncthreads();
+        wave_lds_sync();
+#pragma unroll
+        for (int q = 0; q < R1 / R2; ++q)
+#pragma unroll
+            for (int k2 = 0; k2 < R2; ++k2) b[n2 + ROW * (q + (R1 / R2) * k2)] = v[q * R2 + k2];
     };
-    const int nip = (tl.nin + 1) / 2;
-    for (int jp = 0; jp < nip; ++jp) {
-        const Cx<T> *src = Zin + (size_t)jp * ns;
-        Cx<T> v[R1], X[R1];
+    // The table values of a step: the lines of a group share them, so line l of it loads those at n1 = NL c + l,
+    // for every chunk c of NL values, one step ahead of their use, and the lanes exchange them in LDS (loading
+    // them all in every lane, the CU's texture units were busy for 3/4 of the kernel's time).
+    T kt[NC][4];
+    auto load = [&](int st, int c) {
 #pragma unroll
-        for (int n1 = 0; n1 < R1; ++n1) v[n1] = live ? src[row + R2 * n1 + n2] : Cx<T>{(T)0, (T)0};
-        forward(v, X);
-        // spectra in natural order: every half writes its own line
+        for (int e = 0; e < 4; ++e) {
+            const long long at = list[st].at[e];
+            const char *tab = reinterpret_cast<const char *>(at >= 0 ? tk + at : uk + (-1 - at));
+            kt[c][e] = *reinterpret_cast<const T *>(tab + (trow + NL * R2 * c) * (unsigned)sizeof(T));
+        }
+    };
+    const T *shared = stage + (i - i % NL) * R2 + n2;   // value of n1 = NL c + r at r R2
+    // step st (its input pair in slot sl) into acc; loads the table values of step sn
+    auto accumulate = [&](int st, int sn, int sl) {
+        const Cx<T> *sp = spec + (size_t)sl * L * LD;
+        T cf[4];
 #pragma unroll
-        for (int r = 0; r < R1; ++r) mine[kpos(r)] = X[r];
-        __syncthreads();
-        if (live) {
-            Cx<T> Yr[R1];   // the spectrum at -k
+        for (int e = 0; e < 4; ++e) {
+            const int flip = list[st].odd[e] & negs;   // an odd table changes sign at this line
+            cf[e] = (T)0.5 * (T)list[st].coef[e];
+            if (flip == 4 || flip == 8) cf[e] = -cf[e];
+        }
 #pragma unroll
-            for (int r = 0; r < R1; ++r) {
-                const int k = kpos(r);
-                Yr[r] = partner[k ? M - k : 0];
-            }
-            for (int h = 0; h < 2; ++h) {
-                const int f = 2 * jp + h;
-                if (f >= tl.nin) break;
-                int last = 0x7fffffff;
-                T kt[R1];
-                for (int t = tl.first[f]; t < tl.first[f + 1]; ++t) {
-                    const Term tm = tl.term[t];
-                    if (tm.t != last) {
-                        const T *tab = tm.t >= 0 ? tk + (size_t)tm.t * tg.tn : uk + (size_t)(-tm.t - 1) * tg.tn;
+        for (int c = 0; c < NC; ++c) {
+            wave_lds_sync();
 #pragma unroll
-                        for (int r = 0; r < R1; ++r) kt[r] = tab[trow + kpos(r)];
-                        if ((tm.odd == 1 && neg_y) || (tm.odd == 2 && neg_z)) {
+            for (int e = 0; e < 4; ++e) stage[64 * e + lane] = kt[c][e];
+            wave_lds_sync();
+            load(sn, c);
 #pragma unroll
-                            for (int r = 0; r < R1; ++r) kt[r] = -kt[r];
-                        }
-                        last = tm.t;
-                    }
-                    const int p = tm.o >> 1, odd = tm.o & 1;
-                    const T cf = (T)tm.coef;
+            for (int r = 0; r < NL; ++r) {
+                const int n1 = c * NL + r;
+                const Cx<T> a = sp[own + ROW * n1], b = sp[n1 == 0 && n2 == 0 ? neg : negk - ROW * n1];
+                // twice the spectra of the pair's two fields
+                const Cx<T> X[2] = {Cx<T>{a.x + b.x, a.y - b.y}, Cx<T>{a.y + b.y, b.x - a.x}};
 #pragma unroll
-                    for (int r = 0; r < R1; ++r) {
-                        const T kv = cf * kt[r];
-                        const Cx<T> xh = unpack(X[r], Yr[r], h);
-                        const Cx<T> yv = tm.imag ? Cx<T>{-kv * xh.y, kv * xh.x} : Cx<T>{kv * xh.x, kv * xh.y};
-                        const Cx<T> add = odd ? Cx<T>{-yv.y, yv.x} : yv;
-#pragma unroll
-                        for (int pp = 0; pp < NOP; ++pp)
-                            if (pp == p) acc[pp][r] = cadd(acc[pp][r], add);
-                    }
+                for (int h = 0; h < 2; ++h) {   // (wa + i wb) X
+                    const T wa = cf[h] * shared[64 * h + r * R2], wb = cf[2 + h] * shared[64 * (2 + h) + r * R2];
+                    acc[n1].x += wa * X[h].x - wb * X[h].y;
+                    acc[n1].y += wa * X[h].y + wb * X[h].x;
                 }
             }
         }
-        __syncthreads();
-    }
-    // output pairs back along x, one at a time, every lane its own line
-    const int nop = (tl.nout + 1) / 2;
-    const bool store = live && (half == 0 || !self);
-#pragma unroll
-    for (int p = 0; p < NOP; ++p) {
-        if (p >= nop) break;
-#pragma unroll
-        for (int r = 0; r < R1; ++r) mine[kpos(r)] = acc[p][r];
-        __syncthreads();
-        Cx<T> v[R1];
-#pragma unroll
-        for (int n1 = 0; n1 < R1; ++n1) v[n1] = mine[R2 * n1 + n2];
-        __syncthreads();
-        dft_reg<R1, 1>(v);
+    };
+    // acc back along x: output pair po
+    auto inverse = [&](int po) {
+        dft_reg<R1, 1>(acc);
+        T *b = work + i * LD;
+        wave_lds_sync();   // the table values are read
+        Cx<T> u[R1];
 #pragma unroll
         for (int k1 = 0; k1 < R1; ++k1) {
             Cx<T> w = tw[n2 * k1];
             w.y = -w.y;
-            mine[k1 * R2 + n2] = cmul(v[k1], w);
+            acc[k1] = cmul(acc[k1], w);
+            b[k1 * ROW + n2] = acc[k1].x;
         }
-        __syncthreads();
-        if (store) {
+        wave_lds_sync();
 #pragma unroll
-            for (int q = 0; q < R1 / R2; ++q) {
-                const int k1 = n2 + R2 * q;
-                Cx<T> u[R2];
+        for (int q = 0; q < R1 / R2; ++q)
 #pragma unroll
-                for (int m = 0; m < R2; ++m) u[m] = mine[k1 * R2 + m];
-                dft_reg<R2, 1>(u);
+            for (int m = 0; m < R2; ++m) u[q * R2 + m].x = b[(n2 + R2 * q) * ROW + m];
+        wave_lds_sync();
 #pragma unroll
-                for (int k2 = 0; k2 < R2; ++k2) Oout[(size_t)p * ns + row + k1 + R1 * k2] = u[k2];
+        for (int k1 = 0; k1 < R1; ++k1) b[k1 * ROW + n2] = acc[k1].y;
+        wave_lds_sync();
+        Cx<T> *dst = Oout + (size_t)po * ns + row + n2;
+#pragma unroll
+        for (int q = 0; q < R1 / R2; ++q) {
+#pragma unroll
+            for (int m = 0; m < R2; ++m) u[q * R2 + m].y = b[(n2 + R2 * q) * ROW + m];
+            dft_reg<R2, 1>(u + q * R2);
+            if (store) {
+#pragma unroll
+                for (int k2 = 0; k2 < R2; ++k2) dst[R2 * q + R1 * k2] = u[q * R2 + k2];
             }
         }
+        wave_lds_sync();   // the work rows are read
+    };
+    // acc holds the output pair, divided by i where turned is set
+    int turned = 0;
+    auto turn = [&](int to) {
+        if (to == turned) return;
+#pragma unroll
+        for (int r = 0; r < R1; ++r) acc[r] = to ? Cx<T>{acc[r].y, -acc[r].x} : Cx<T>{-acc[r].y, acc[r].x};
+        turned = to;
+    };
+    clear();
+    int st = wave < nop ? first[wave] : 0;
+#pragma unroll 1
+    for (int j0 = 0; j0 < nip; j0 += slots) {
+        const int nj = min(slots, nip - j0);
+        if (j0) __syncthreads();   // the previous spectra are read
+        if (wave < nop) {
+#pragma unroll
+            for (int c = 0; c < NC; ++c) load(min(st, first[wave + 1] - 1), c);
+        }
+#pragma unroll 1
+        for (int j = wave; j < nj; j += nw) forward(j0 + j, j);
         __syncthreads();
+#pragma unroll 1
+        for (int po = wave; po < nop; po += nw) {
+            if (po != wave) clear();
+            const int last = first[po + 1] - 1, next = po + nw < nop ? first[po + nw] : last;
+#pragma unroll 1
+            while (st <= last && list[st].jp < j0 + nj) {
+                turn(list[st].rot);
+                accumulate(st, st < last ? st + 1 : next, list[st].jp - j0);
+                ++st;
+            }
+            if (alias) break;
+            turn(0);
+            st = next;
+            inverse(po);
+        }
+    }
+    if (alias) {   // the work rows take the spectra's place
+        __syncthreads();
+        turn(0);
+        if (wave < nop) inverse(wave);
     }
 }
 
@@ -2029,6 +2070,7 @@ void fft3d(const FftPlan &F, Cx<T> *data, int nfield, int sign, hipStream_t s)
 
 // LDS budget of the fused x pass
 constexpr size_t kXprodLds = 64 * 1024;
+constexpr size_t kXgroupLds = 80 * 1024;   // its register form: two workgroups per CU
 
 // Lines per workgroup of the fused x pass for nop output pairs: the largest power of two up to 8
 // whose LDS fits kXprodLds and that leaves about kFftGroups workgroups; 0 when one line does not fit.
@@ -2046,8 +2088,8 @@ int xprod_lpb(const FftPlan &F, int nop)
     return (M * sizeof(Cx<double>) + lpb * per_line <= kXprodLds) ? lpb : 0;
 }
 
-// the register form of the fused x pass where the x length has register radices and the output
-// pairs' spectrum values fit in registers (NOP R1 <= 32); false otherwise
+// products reported as running in registers throughout: register radices and output pairs whose spectrum
+// values fit in one lane's registers (NOP R1 <= 32)
 inline bool xreg_fits(const FftPlan &F, const TermList &tl, int &R1, int &R2)
 {
     if (!F.xreg || !reg_radices(F.M[0], R1, R2)) return false;
@@ -2055,43 +2097,55 @@ inline bool xreg_fits(const FftPlan &F, const TermList &tl, int &R1, int &R2)
     return nop <= 4 && nop * R1 <= 32;
 }
 
+// The register form of the fused x pass, where the x length has register radices.  A product of more than
+// two output pairs keeps every input spectrum in LDS and deals the outputs to up to 4 waves; one of few
+// outputs runs two waves that refill two slots, which leaves LDS for more workgroups, or, where there
+// are too few workgroups for that to matter, one wave and slot per input pair.
 template <typename T>
 bool xprod_reg(const FftPlan &F, const Cx<T> *Z, Cx<T> *O, const TermList &tl, const T *tk, const T *uk, hipStream_t s)
 {
     int R1 = 0, R2 = 0;
-    if (!xreg_fits(F, tl, R1, R2)) return false;
-    const int nop = (tl.nout + 1) / 2;
-    const int L = 64 / R2;
-    const long long lines = xprod_primary_lines(F.M[1], F.M[2]);
-    const dim3 grid((unsigned)((lines + L - 1) / L)), block(2 * L * R2);
-    const size_t lds = sizeof(Cx<T>) * ((size_t)F.M[0] + 2 * (size_t)L * (F.M[0] + 1));
+    if (!F.xreg || !F.fold || F.tn >= (1LL << 29) || !reg_radices(F.M[0], R1, R2)) return false;
+    if (!tl.steps) return false;
+    const int nip = (tl.nin + 1) / 2, nop = (tl.nout + 1) / 2, L = 64 / R2;
+    const int nl = F.M[2] > 1 ? 4 : 2, per = L / nl;
+    const long long groups = (long long)(F.M[1] / 2 + 1) * (F.M[2] / 2 + 1), wgs = (groups + per - 1) / per;
+    int waves, slots;
+    if (nop > 2) {
+        waves = std::min(nop, 4);
+        slots = nip;
+    } else {
+        waves = slots = std::min(nip, wgs < 4 * 256 ? 4 : 2);
+        waves = std::max(waves, nop);
+    }
+    const bool alias = nop <= waves;
+    const size_t line = (size_t)L * (R1 * (R2 + 1) + 1);   // elements of a slot
+    // twiddles, spectra, then each wave's work rows; or each wave's 256 table values, and the work rows in the spectra's place
+    const size_t lds = (size_t)F.M[0] * sizeof(Cx<T>) +
+                       (alias ? std::max((size_t)slots * line * sizeof(Cx<T>) + waves * 256 * sizeof(T), waves * line * sizeof(T))
+                              : (size_t)slots * line * sizeof(Cx<T>) + waves * line * sizeof(T));
+    if (lds > kXgroupLds) return false;
     auto go = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, grid, block, lds, s, Z, O, F.ns, F.M[1], F.M[2], F.S1, F.S2, L, twiddles<T>(F, 0), tk,
-                           uk, tab_geo(F), tl, F.xcdmap);
+        if (lds > 64 * 1024)
+            TMI_HIP_CHECK(hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        hipLaunchKernelGGL(kernel, dim3((unsigned)wgs), dim3(64 * waves), lds, s, Z, O, F.ns, F.M[1], F.M[2], F.S1, F.S2, slots,
+                           alias ? 1 : 0, twiddles<T>(F, 0), tk, uk, tab_geo(F), tl.steps, tl.start, nip, nop, F.xcdmap);
     };
-    auto by_nop = [&](auto r1, auto r2) {
+    auto by_lines = [&](auto r1, auto r2) {
         constexpr int A = decltype(r1)::value, B = decltype(r2)::value;
-        if constexpr (A * 1 <= 32) {
-            if (nop == 1) go(k_fft_xprod_reg<T, A, B, 1>);
-        }
-        if constexpr (A * 2 <= 32) {
-            if (nop == 2) go(k_fft_xprod_reg<T, A, B, 2>);
-        }
-        if constexpr (A * 3 <= 32) {
-            if (nop == 3) go(k_fft_xprod_reg<T, A, B, 3>);
-        }
-        if constexpr (A * 4 <= 32) {
-            if (nop == 4) go(k_fft_xprod_reg<T, A, B, 4>);
-        }
+        if (nl == 4)
+            go(k_fft_xgroup<T, A, B, 4>);
+        else
+            go(k_fft_xgroup<T, A, B, 2>);
     };
     if (R1 == 8 && R2 == 4)
-        by_nop(std::integral_constant<int, 8>{}, std::integral_constant<int, 4>{});
+        by_lines(std::integral_constant<int, 8>{}, std::integral_constant<int, 4>{});
     else if (R1 == 8 && R2 == 8)
-        by_nop(std::integral_constant<int, 8>{}, std::integral_constant<int, 8>{});
+        by_lines(std::integral_constant<int, 8>{}, std::integral_constant<int, 8>{});
     else if (R1 == 16 && R2 == 8)
-        by_nop(std::integral_constant<int, 16>{}, std::integral_constant<int, 8>{});
+        by_lines(std::integral_constant<int, 16>{}, std::integral_constant<int, 8>{});
     else
-        by_nop(std::integral_constant<int, 16>{}, std::integral_constant<int, 16>{});
+        by_lines(std::integral_constant<int, 16>{}, std::integral_constant<int, 16>{});
     return true;
 }
 
@@ -2150,6 +2204,52 @@ inline const T *fmt_spectra(const FftPlan &F)
         return reinterpret_cast<const T *>(F.tf);
 }
 
+// tl as steps in device memory; none where an output takes a field twice
+void free_steps(TermList &tl)
+{
+    (void)hipFree(tl.steps);
+    (void)hipFree(tl.start);
+    tl.steps = nullptr;
+    tl.start = nullptr;
+}
+void upload_steps(const FftPlan &F, TermList &tl)
+{
+    const int nip = (tl.nin + 1) / 2, nop = (tl.nout + 1) / 2;
+    std::vector<ProductStep> steps;
+    std::vector<int> start(1, 0);
+    for (int po = 0; po < nop; ++po) {
+        for (int jp = 0; jp < nip; ++jp)
+            for (int rot = 0; rot < 2; ++rot) {
+                ProductStep st{};
+                bool any = false;
+                st.jp = jp;
+                st.rot = rot;
+                for (int h = 0; h < 2 && 2 * jp + h < tl.nin; ++h)
+                    for (int t = tl.first[2 * jp + h]; t < tl.first[2 * jp + h + 1]; ++t) {
+                        const Term &m = tl.term[t];
+                        const int e = 2 * (m.o & 1) + h;
+                        if (m.o >> 1 != po || (m.imag ? 1 : 0) != rot) continue;
+                        if (st.coef[e] != 0.0) return;
+                        st.at[e] = m.t >= 0 ? (long long)m.t * F.tn : -1 - (long long)(-m.t - 1) * F.tn;
+                        st.coef[e] = m.coef;
+                        st.odd[e] = (m.odd == 1 ? 4 : 0) | (m.odd == 2 ? 8 : 0);
+                        any = true;
+                    }
+                for (int h = 0; h < 2; ++h)   // an output without this field: the other's table again, times 0
+                    for (int e : {h, 2 + h})
+                        if (st.coef[e] == 0.0) st.at[e] = st.at[e ^ 2];
+                if (any) steps.push_back(st);
+            }
+        if ((int)steps.size() == start.back()) return;   // no pair without input
+        start.push_back((int)steps.size());
+    }
+    if (steps.empty()) return;
+    TMI_HIP_CHECK(hipMalloc((void **)&tl.start, start.size() * sizeof(int)));
+    TMI_HIP_CHECK(hipMemcpy(tl.start, start.data(), start.size() * sizeof(int), hipMemcpyHostToDevice));
+    TMI_HIP_CHECK(hipMalloc((void **)&tl.steps, steps.size() * sizeof(ProductStep)));
+    TMI_HIP_CHECK(hipMemcpy(tl.steps, steps.data(), steps.size() * sizeof(ProductStep), hipMemcpyHostToDevice));
+}
+
 void free_plan(FftPlan *F)
 {
     if (!F) return;
@@ -2164,6 +2264,7 @@ void free_plan(FftPlan *F)
     (void)hipFree(F->pqr);
     (void)hipFree(F->pqr_f);
     (void)hipFree(F->ss);
+    for (TermList *tl : {&F->tfwd[0], &F->tfwd[1], &F->tel, &F->tel_d, &F->tvr, &F->tvb, &F->tpc}) free_steps(*tl);
     for (int d = 0; d < 3; ++d) {
         (void)hipFree(F->twd[d]);
         (void)hipFree(F->twf[d]);
@@ -2525,6 +2626,8 @@ void fft_setup(Problem &P, bool mf, bool fmt)
             }
             F->fmt_ok = parity_ok;
         }
+        for (TermList *tl : {&F->tfwd[0], &F->tfwd[1], &F->tel, &F->tel_d, &F->tvr, &F->tvb})
+            if (tl->nin && tl->nout) upload_steps(*F, *tl);
         TMI_HIP_CHECK(hipGetLastError());
         TMI_HIP_CHECK(hipDeviceSynchronize());
     } catch (...) {
@@ -3228,6 +3331,7 @@ void precond_setup(Problem &P)
                            (long long)qr.size());
         TMI_HIP_CHECK(hipStreamSynchronize(0));
         TermList &tl = F.tpc;
+        free_steps(tl);
         tl = TermList();
         tl.nout = C;
         for (int j = 0; j < C; ++j) {   // input component j feeds every output i through table i + C j
@@ -3235,6 +3339,7 @@ void precond_setup(Problem &P)
             ++tl.nin;
             tl.first[tl.nin + 1] = tl.first[tl.nin];
         }
+        upload_steps(F, tl);
         F.pc_fused = true;
     }
 }
