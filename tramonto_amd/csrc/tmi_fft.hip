@@ -2235,9 +2235,10 @@ void upload_steps(const FftPlan &F, TermList &tl)
                         st.odd[e] = (m.odd == 1 ? 4 : 0) | (m.odd == 2 ? 8 : 0);
                         any = true;
                     }
-                for (int h = 0; h < 2; ++h)   // an output without this field: the other's table again, times 0
-                    for (int e : {h, 2 + h})
-                        if (st.coef[e] == 0.0) st.at[e] = st.at[e ^ 2];
+                // absent factors: a present one's table again, times 0 (a plan need not hold both kinds of table)
+                for (int p = 3; p >= 0; --p)
+                    for (int e = 0; e < 4; ++e)
+                        if (st.coef[p] != 0.0 && st.coef[e] == 0.0) st.at[e] = st.at[p];
                 if (any) steps.push_back(st);
             }
         if ((int)steps.size() == start.back()) return;   // no pair without input
