@@ -1561,6 +1561,144 @@ __global__ __launch_bounds__(256, (sizeof(T) == 8 ? 2 : 3) + (R1 == 8 ? 1 : 0)) 
     }
 }
 
+// The point stage of a 3D grid with the z transforms around it: dPhi/dn (residual) or H(n) dn (linear) at the
+// nodes, packed as pairs of adjoint fields and transformed along z; in INV form (Schur products) dn comes
+// from the pairs of the density product, transformed back along z here, so the rho-bar rows never reach
+// memory.  A workgroup takes L = 64 / R2 consecutive x at one y, all z, one wave per pair field; the values
+// of its L M nodes stand in LDS as [pair][z][x] (80 KB in FP64: two workgroups per CU), where the waves'
+// transposes of the register transforms (k_fft_strided) take place too.
+// More waves than pairs share the nodes' work (8 for a residual, 6 where the Hessian's registers leave 3 waves
+// per SIMD: with 5 a 128^3 residual took 113 us), and bound it: HBM alone would take 70 us.  128^3, ten rows in and
+// five pairs out: residual 99 us (point kernel 66, z pass 55); FP32 Schur product 121 and 22 us for the
+// mean-field rows (rows pass 65, point kernel 88, z pass 27).  64^3, one component: 10.4 us (8.2 and 8.4).
+struct PointArgs {
+    int C, func, N, nx0, nx1, xg, xcd;
+    long long ns, S1, S2;
+    int nin, nadj;      // INV: pairs of the density product; pairs of adjoint fields
+    int dform;
+    const double *xrb, *dnrb;
+    int src[10], nmf, mfsrc[kNC];   // INV: outputs of the rho-bar and mean-field rows and their factors
+    double scale[10], mfscale[kNC];
+    double *out_mf;
+    CompConsts cc;
+};
+template <typename T, int MODE, bool INV, int R1, int R2>
+__global__ __launch_bounds__(MODE ? 384 : 512, MODE ? 3 : 4) void k_point_z(PointArgs a, const Cx<T> *__restrict__ O, Cx<T> *__restrict__ Z,
+                                                                         const Cx<T> *__restrict__ tw)
+{
+    constexpr int M = R1 * R2, L = 64 / R2, ND = 3, NR = 4 + 2 * ND, NQ = R1 / R2;
+    extern __shared__ char smem_raw[];
+    Cx<T> *val = reinterpret_cast<Cx<T> *>(smem_raw);   // [pairs][M][L]
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int bx = a.xcd ? xcd_item(blockIdx.x, gridDim.x) : (int)blockIdx.x;
+    const int y = bx / a.xg, x0 = (bx % a.xg) * L;
+    const int i = lane % L, n2 = lane / L;
+    const bool live = x0 + i < a.nx0;
+    const long long base = x0 + i + (long long)y * a.S1;
+    Cx<T> *own = val + (size_t)wave * M * L;
+    Cx<T> v[R1];
+    // v (elements R2 n1 + n2 of the lane's line) -> v[q R2 + k2], elements n2 + R2 q + R1 k2
+    auto transform = [&](auto sign) {
+        constexpr int SIGN = decltype(sign)::value;
+        dft_reg<R1, SIGN>(v);
+        Cx<T> u[R1];
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) {
+            wave_lds_sync();
+#pragma unroll
+            for (int t = 0; t < R2; ++t) {
+                Cx<T> w = tw[n2 * (R2 * q + t)];
+                if constexpr (SIGN > 0) w.y = -w.y;
+                own[(t * R2 + n2) * L + i] = cmul(v[R2 * q + t], w);
+            }
+            wave_lds_sync();
+#pragma unroll
+            for (int m = 0; m < R2; ++m) u[q * R2 + m] = own[(n2 * R2 + m) * L + i];
+            dft_reg<R2, SIGN>(u + q * R2);
+        }
+        wave_lds_sync();
+#pragma unroll
+        for (int r = 0; r < R1; ++r) v[r] = u[r];
+    };
+    const size_t N = a.N;
+    auto node_of = [&](int e) { return min(x0 + e % L, a.nx0 - 1) + (size_t)a.nx0 * (y + (size_t)a.nx1 * (e / L)); };
+    constexpr bool DN = MODE == 1 && !INV;
+    if constexpr (INV) {
+        if (wave < a.nin) {
+            const Cx<T> *src = O + (size_t)wave * a.ns + base;
+#pragma unroll
+            for (int n1 = 0; n1 < R1; ++n1) v[n1] = live ? src[(R2 * n1 + n2) * a.S2] : Cx<T>{(T)0, (T)0};
+            transform(std::integral_constant<int, 1>{});
+#pragma unroll
+            for (int r = 0; r < R1; ++r) own[(n2 + R2 * (r / R2) + R1 * (r % R2)) * L + i] = v[r];
+        }
+        __syncthreads();
+    }
+#pragma unroll 1
+    for (int e = tid; e < M * L; e += blockDim.x) {
+        double rb[NR], dr[NR], n[NR], dn[NR], out[NR];
+        const size_t node = node_of(e);
+#pragma unroll
+        for (int q = 0; q < NR; ++q) {
+            rb[q] = a.xrb[q * N + node];
+            if constexpr (DN) dr[q] = a.dnrb[q * N + node];
+        }
+        // solution order (n3 n2 n1 n0 nv2 nv1) -> n order
+        auto reorder = [](const double *r, double *o) {
+            for (int q = 0; q < 4; ++q) o[q] = r[3 - q];
+            for (int d = 0; d < ND; ++d) {
+                o[4 + d] = r[4 + ND + d];
+                o[4 + ND + d] = r[4 + d];
+            }
+        };
+        reorder(rb, n);
+        if constexpr (DN) reorder(dr, dn);
+        if constexpr (INV) {
+            auto output = [&](int o) {
+                const Cx<T> p = val[(o >> 1) * M * L + e];
+                return (double)((o & 1) ? p.y : p.x);
+            };
+#pragma unroll
+            for (int q = 0; q < NR; ++q) dr[q] = output(a.src[q]) * a.scale[q];
+            for (int m = 0; m < a.nmf; ++m)
+                if (x0 + e % L < a.nx0 && a.mfsrc[m] < 2 * a.nin) a.out_mf[m * N + node] = output(a.mfsrc[m]) * a.mfscale[m];
+            reorder(dr, dn);
+        }
+        if constexpr (MODE == 0)
+            fmt_dphi<ND>(a.func, n, out);
+        else
+            fmt_hvp<ND>(a.func, n, dn, out);
+        if (a.dform) {   // the derivatives themselves, rho-bar order
+            val[e] = Cx<T>{(T)out[3], (T)out[2]};
+            val[M * L + e] = Cx<T>{(T)out[1], (T)out[0]};
+            val[2 * M * L + e] = Cx<T>{(T)out[7], (T)out[8]};
+            val[3 * M * L + e] = Cx<T>{(T)out[9], (T)out[4]};
+            val[4 * M * L + e] = Cx<T>{(T)out[5], (T)out[6]};
+        } else {   // A_c, B_c,d of each component, then S3
+            T *f = reinterpret_cast<T *>(val);
+            auto put = [&](int k, double w) { f[2 * ((k >> 1) * M * L + e) + (k & 1)] = (T)w; };
+#pragma unroll
+            for (int c = 0; c < kNC; ++c)
+                if (c < a.C) {
+                    put(c * (1 + ND), out[0] * a.cc.i4pirsq[c] + out[1] * a.cc.i4pir[c] + out[2]);
+                    for (int d = 0; d < ND; ++d) put(c * (1 + ND) + 1 + d, out[4 + d] * a.cc.i4pir[c] + out[4 + ND + d]);
+                }
+            put(a.C * (1 + ND), out[3]);
+            if ((a.C * (1 + ND) + 1) & 1) put(a.C * (1 + ND) + 1, 0.0);
+        }
+    }
+    __syncthreads();
+    if (wave >= a.nadj) return;
+#pragma unroll
+    for (int n1 = 0; n1 < R1; ++n1) v[n1] = own[(R2 * n1 + n2) * L + i];
+    transform(std::integral_constant<int, -1>{});
+    if (live) {
+        Cx<T> *dst = Z + (size_t)wave * a.ns + base;
+#pragma unroll
+        for (int r = 0; r < R1; ++r) dst[(n2 + R2 * (r / R2) + R1 * (r % R2)) * a.S2] = v[r];
+    }
+}
+
 // Euler-Lagrange rows from the sums E_c, as k_el_rows:
 //  residual: E + ln x + mu [+ V_ext] [+ x_MF]      ; zero rows: x   (in_rho)
 //  linear  : E + v/x + v_MF                        ; zero rows: v
@@ -2724,13 +2862,113 @@ PassIO rows_io(const Problem &P, int w, const double *rho_nodes, const double *i
     return io;
 }
 
+// pairs of the density product that hold rho-bar rows
+int point_pairs_in(const FftPlan &F)
+{
+    int o = 0;
+    for (int q = 0; q < F.rows[1].nrb; ++q) o = std::max(o, F.rows[1].src[q]);
+    return o / 2 + 1;
+}
+
+// The point stage runs with the z transforms around it (k_point_z): 3D wrapping grids whose z axis takes the
+// register pass, up to five pairs of adjoint fields (all that arise outside the reference-Jacobian mode)
+template <typename T>
+bool point_z_radices(const Problem &P, bool linear, int &R1, int &R2)
+{
+    if (!P.fft || !P.fft->fmt || !P.fft->wraps || P.p.ndim != 3 || (linear && P.jac_ref)) return false;
+    const FftPlan &F = *P.fft;
+    const int nadj = (el_dform(P, linear) ? 10 : P.p.ncomp * 4 + 1), np = (nadj + 1) / 2;
+    return (linear || sizeof(T) == 8) && np <= 5 && F.M[2] > 1 && use_reg_pass(F, 2, np, R1, R2);
+}
+
+// xrb: rho-bar rows; dnrb: their direction (linear), null for the INV form, which reads the density product's pairs
+// and writes the mean-field rows among them to out_mf
+template <typename T>
+void launch_point_z(Problem &P, const double *xrb, const double *dnrb, bool linear, bool inv, double *out_mf, int R1, int R2,
+                    hipStream_t s)
+{
+    const FftPlan &F = *P.fft;
+    PointArgs a{};
+    a.C = P.p.ncomp;
+    a.func = P.p.type_func;
+    a.N = P.N;
+    a.nx0 = P.p.nx[0];
+    a.nx1 = P.p.nx[1];
+    a.xcd = F.xcdmap;
+    a.ns = F.ns;
+    a.S1 = F.S1;
+    a.S2 = F.S2;
+    a.dform = el_dform(P, linear) ? 1 : 0;
+    a.nadj = ((a.dform ? 10 : a.C * 4 + 1) + 1) / 2;
+    a.xrb = xrb;
+    a.dnrb = dnrb;
+    a.cc = make_consts(P);
+    const RowMap &rm = F.rows[1];
+    if (inv) {
+        a.nin = point_pairs_in(F);
+        a.nmf = rm.nmf;
+        a.out_mf = out_mf;
+        for (int q = 0; q < 10; ++q) a.src[q] = rm.src[q], a.scale[q] = rm.scale[q];
+        for (int m = 0; m < rm.nmf; ++m) a.mfsrc[m] = rm.src[rm.nrb + m], a.mfscale[m] = rm.scale[rm.nrb + m];
+    }
+    const int L = 64 / R2, pairs = std::max(a.nadj, a.nin), waves = linear ? 6 : 8;
+    a.xg = (F.M[0] + L - 1) / L;
+    const size_t lds = (size_t)pairs * 64 * R1 * sizeof(Cx<T>);
+    auto go = [&](auto kernel) {
+        if (lds > 64 * 1024)
+            TMI_HIP_CHECK(hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        hipLaunchKernelGGL(kernel, dim3((unsigned)(a.xg * F.M[1])), dim3(64 * waves), lds, s, a,
+                           reinterpret_cast<const Cx<T> *>(F.obuf), reinterpret_cast<Cx<T> *>(F.zbuf), twiddles<T>(F, 2));
+    };
+    auto by_mode = [&](auto r1, auto r2) {
+        constexpr int A = decltype(r1)::value, B = decltype(r2)::value;
+        if (!linear) {   // residuals are FP64
+            if constexpr (sizeof(T) == 8) go(k_point_z<T, 0, false, A, B>);
+        } else if (!inv)
+            go(k_point_z<T, 1, false, A, B>);
+        else
+            go(k_point_z<T, 1, true, A, B>);
+    };
+    if (R1 == 8 && R2 == 4)
+        by_mode(std::integral_constant<int, 8>{}, std::integral_constant<int, 4>{});
+    else if (R1 == 8 && R2 == 8)
+        by_mode(std::integral_constant<int, 8>{}, std::integral_constant<int, 8>{});
+    else if (R1 == 16 && R2 == 8)
+        by_mode(std::integral_constant<int, 16>{}, std::integral_constant<int, 8>{});
+    else
+        by_mode(std::integral_constant<int, 16>{}, std::integral_constant<int, 16>{});
+    TMI_HIP_CHECK(hipGetLastError());
+}
+
+template <typename T>
+bool fft_point(Problem &P, const double *x_rb, const double *dn_rb, bool linear, hipStream_t s)
+{
+    int R1 = 0, R2 = 0;
+    if (!point_z_radices<T>(P, linear, R1, R2)) return false;
+    launch_point_z<T>(P, x_rb, dn_rb, linear, false, nullptr, R1, R2, s);
+    return true;
+}
+template bool fft_point<double>(Problem &, const double *, const double *, bool, hipStream_t);
+template bool fft_point<float>(Problem &, const double *, const double *, bool, hipStream_t);
+
+template <typename T>
+bool fft_schur_fused(const Problem &P)
+{
+    int R1 = 0, R2 = 0;
+    return fft_node_input(P) && P.hw_fwd.nrows == 0 && point_z_radices<T>(P, true, R1, R2);
+}
+template bool fft_schur_fused<double>(const Problem &);
+template bool fft_schur_fused<float>(const Problem &);
+
 // Density products from the halo-padded densities in workspace<T>(P).rho_pad:
 // with_rb: the rho-bar rows (out_rb = sums - in_rb - sub_rb), then the
 // mean-field rows when they are in FFT form; else the mean-field rows only.
+// point_rb (fft_schur_fused): the rho-bar rows are not written; the point stage at these rho-bars takes them
+// on to the adjoint fields, transformed along z, as fft_point leaves them.
 template <typename T>
 void fft_rb_mf(Problem &P, const double *rho_nodes, bool with_rb, const double *in_rb, const double *sub_rb,
                double *out_rb, const double *in_mf, const double *sub_mf, double *out_mf, hipStream_t s, double *ss,
-               long long *nss)
+               long long *nss, const double *point_rb)
 {
     if (nss) *nss = 0;
     const FftPlan &F = *P.fft;
@@ -2787,6 +3025,23 @@ void fft_rb_mf(Problem &P, const double *rho_nodes, bool with_rb, const double *
             }
             fft_pass<T>(F, O, nop, +1, 0, s);
         }
+        if (point_rb) {   // the rho-bar pairs go on through the point stage; the others write their rows
+            int R1 = 0, R2 = 0;
+            if (!ends || !point_z_radices<T>(P, true, R1, R2)) throw std::logic_error("the point stage is not fused here");
+            fft_pass<T>(F, O, nop, +1, 1, s);
+            launch_point_z<T>(P, point_rb, nullptr, true, true, out_mf, R1, R2, s);
+            const int np = point_pairs_in(F);
+            io.nout = d.nout - 2 * np;
+            for (int o = 0; o < io.nout; ++o) {
+                io.nrow[o] = F.onrow[w][o + 2 * np];
+                for (int k = 0; k < 3; ++k) {
+                    io.row[o][k] = F.orow[w][o + 2 * np][k];
+                    io.scale[o][k] = F.oscale[w][o + 2 * np][k];
+                }
+            }
+            fft_pass<T>(F, O + (size_t)np * F.ns, nop - np, +1, 2, s, kPassRows, io);
+            return;
+        }
         if (ends) io.ss = ss;
         long long blocks = 0;
         for (int a : inv_axes)
@@ -2802,9 +3057,9 @@ void fft_rb_mf(Problem &P, const double *rho_nodes, bool with_rb, const double *
     TMI_HIP_CHECK(hipGetLastError());
 }
 template void fft_rb_mf<double>(Problem &, const double *, bool, const double *, const double *, double *,
-                                const double *, const double *, double *, hipStream_t, double *, long long *);
+                                const double *, const double *, double *, hipStream_t, double *, long long *, const double *);
 template void fft_rb_mf<float>(Problem &, const double *, bool, const double *, const double *, double *,
-                               const double *, const double *, double *, hipStream_t, double *, long long *);
+                               const double *, const double *, double *, hipStream_t, double *, long long *, const double *);
 
 // Euler-Lagrange rows from the adjoint fields (as el_rows): in workspace<T>(P).adj_pad,
 // or, on wrapping grids, already paired in the transform buffer (fft_pairs)
@@ -2848,7 +3103,8 @@ void fft_el(Problem &P, bool linear, const double *x_rho, const double *in_rho, 
         int last = -1;
         for (int a : {1, 2})
             if (F.M[a] > 1) last = a;
-        fft_pass<T>(F, Z, nip, -1, 2, s);
+        int R1 = 0, R2 = 0;
+        if (!point_z_radices<T>(P, linear, R1, R2)) fft_pass<T>(F, Z, nip, -1, 2, s);   // fft_point did it
         fft_pass<T>(F, Z, nip, -1, 1, s);
         if (F.xlpb[1]) {
             fft_xprod<T>(F, Z, O, df ? F.tel_d : F.tel, F.xlpb[1], fmt_spectra<T>(F), attr_spectra<T>(F), s);
@@ -3062,6 +3318,8 @@ void fft_time_kernels(Problem &P, int which, int reps, double *ms, double *bytes
         // which passes run with fused ends (those are other kernels): the density product's first and last
         // strided passes when it reads the node arrays, the Euler-Lagrange product's last one on wrapping grids
         const bool rb_ends = fft_node_input(P), el_ends = F.wraps;
+        int r1 = 0, r2 = 0;
+        const bool point_z = point_z_radices<double>(P, false, r1, r2);
         int first_strided = -1, last_strided = -1;
         for (int a : {2, 1})
             if (F.M[a] > 1 && first_strided < 0) first_strided = a;
@@ -3075,7 +3333,7 @@ void fft_time_kernels(Problem &P, int which, int reps, double *ms, double *bytes
         };
         const Set sets[4] = {{Z, (C + 1) / 2, -1, F.xlpb[0] > 0, rb_ends ? first_strided : -1},
                              {O, (F.fwd[1].nout + 1) / 2, +1, F.xlpb[0] > 0, rb_ends ? last_strided : -1},
-                             {Z, (nadj + 1) / 2, -1, F.xlpb[1] > 0, -1},
+                             {Z, (nadj + 1) / 2, -1, F.xlpb[1] > 0, point_z ? 2 : -1},
                              {O, (C + 1) / 2, +1, F.xlpb[1] > 0, el_ends ? last_strided : -1}};
         auto runs = [&](const Set &t, int axis) {
             return F.M[axis] > 1 && !(t.fused && axis == 0) && axis != t.skip;

@@ -325,7 +325,13 @@ void fft_set_fused(Problem &P, int mask);     // fused x pass for the density (b
 template <typename T>
 void fft_rb_mf(Problem &P, const double *rho_nodes, bool with_rb, const double *in_rb, const double *sub_rb,
                double *out_rb, const double *in_mf, const double *sub_mf, double *out_mf, hipStream_t s,
-               double *ss = nullptr, long long *nss = nullptr);
+               double *ss = nullptr, long long *nss = nullptr, const double *point_rb = nullptr);
+// the point stage with the z transforms around it: false where it does not apply; a Schur product's takes the
+// density product's pairs without rho-bar rows (fft_rb_mf with point_rb)
+template <typename T>
+bool fft_point(Problem &P, const double *x_rb, const double *dn_rb, bool linear, hipStream_t s);
+template <typename T>
+bool fft_schur_fused(const Problem &P);
 // pair buffer of a wrapping FFT grid: field f of node (x, y, z) at element 2 ((f / 2) ns + x + y S1 + z S2) + f % 2
 struct FftPairs {
     void *buf;

@@ -1859,6 +1859,7 @@ void rb_mf_rows(Problem &P, const double *rho, bool linear, const double *in_rb,
 template <typename T>
 void fmt_point(Problem &P, const double *x_rb, const double *dn_rb, bool linear, hipStream_t s)
 {
+    if (fft_point<T>(P, x_rb, dn_rb, linear, s)) return;
     Geo gf = make_geo(P, P.pad_f);
     const CompConsts cc = make_consts(P);
     T *adj = workspace<T>(P).adj_pad;
@@ -2323,7 +2324,7 @@ void launch_init_fields(Problem &P, double *x, hipStream_t s)
 bool schur_one_launch(const Problem &P) { return one_launch(P) && !P.jac_ref && P.hw_fwd.nrows == 0; }
 
 // y2 = A22 x2 + A21 t1, t1 = A12 x2 the rho-bar and mean-field rows of J [x2; 0] (scratch: the
-// one-launch forms do not write it)
+// one-launch forms do not write it, the fused point stage only its mean-field rows)
 template <typename T>
 void launch_schur_apply(Problem &P, const double *x, const double *x2, double *t1, double *y2, hipStream_t s)
 {
@@ -2332,9 +2333,14 @@ void launch_schur_apply(Problem &P, const double *x, const double *x2, double *t
         one_launch_schur<T>(P, x, x2, nullptr, y2, nullptr, s);
         return;
     }
-    rb_mf_rows<T>(P, x2, true, nullptr, nullptr, t1, nullptr, nullptr, t1 + (size_t)P.nrb * N, s);
-    hw_apply(P.hw_fwd, x2, t1, s);
-    fmt_point<T>(P, x + P.iu_rb * N, t1, true, s);
+    if (fft_schur_fused<T>(P)) {   // t1: the mean-field rows alone
+        fft_rb_mf<T>(P, x2, true, nullptr, nullptr, nullptr, nullptr, nullptr, t1 + (size_t)P.nrb * N, s, nullptr, nullptr,
+                     x + P.iu_rb * N);
+    } else {
+        rb_mf_rows<T>(P, x2, true, nullptr, nullptr, t1, nullptr, nullptr, t1 + (size_t)P.nrb * N, s);
+        hw_apply(P.hw_fwd, x2, t1, s);
+        fmt_point<T>(P, x + P.iu_rb * N, t1, true, s);
+    }
     el_rows<T>(P, true, x + P.iu_rho * N, x2, P.nmf ? t1 + (size_t)P.nrb * N : nullptr, nullptr, y2, s);
     TMI_HIP_CHECK(hipGetLastError());
 }
