@@ -44,7 +44,7 @@ XPROD_TRAFFIC_MIB = {"periodic64": (7.5 + 12.0 + 14.9 + 4.0) / 2, "solute128": N
 AXIS_TRAFFIC_MIB = {"periodic64": None, "solute128": None}
 # HBM bytes of one whole fill in FFT form (every launch of the fill, FETCH + WRITE in MiB, from the
 # same counter runs): the fill kernels' measured traffic, against the fill's live time
-FILL_TRAFFIC_MIB = {"periodic64": 245.6, "solute128": 4595.7}
+FILL_TRAFFIC_MIB = {"periodic64": 221.5, "solute128": 3205.2}
 
 
 def stencil_flops_per_node(dp, spec):
