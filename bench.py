@@ -40,7 +40,7 @@ COPY_PROBE_BYTES = 512 << 20
 ROWS_TRAFFIC_MIB = {"periodic64": 35.7 + 24.6, "solute128": 534.6 + 234.3}
 # The same for the fused x pass (mean per launch) and the plain FFT axis passes, where they are the
 # dominant kernel
-XPROD_TRAFFIC_MIB = {"periodic64": (7.5 + 12.0 + 14.9 + 4.0) / 2, "solute128": None}
+XPROD_TRAFFIC_MIB = {"periodic64": (7.4 + 12.0 + 14.8 + 4.0) / 2, "solute128": None}
 AXIS_TRAFFIC_MIB = {"periodic64": None, "solute128": None}
 # HBM bytes of one whole fill in FFT form (every launch of the fill, FETCH + WRITE in MiB, from the
 # same counter runs): the fill kernels' measured traffic, against the fill's live time
