@@ -91,3 +91,31 @@ def test_line_matches_row_kernels(kind, monkeypatch):
         da, _ = rows.schur_solve(x, Fa, rtol=1e-12)
         db, _ = line.schur_solve(x, Fa, rtol=1e-12)
         _compare(da, db, blocks, 1e-8)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nodes", [201, 20000, 40000])   # one, two and four positions per lane
+def test_pair_without_attraction(nodes, monkeypatch):
+    """A binary fluid whose unlike pair has eps = 0: its attraction stencil has no point at all.  The
+    residual of both forms against the oracle, products and the first Krylov steps against each other."""
+    from oracle.oracle import Oracle
+    spec = slit_pore_1d(H=0.02 * (nodes - 1), dx=0.02, seed=8)
+    spec.eps_ff = np.array([[1.0, 0.0], [0.0, 0.9]])
+    rows, line = _problems(lambda: DeviceProblem(spec), monkeypatch)
+    assert line.info.sten_len[2][1] == 0 and line.info.sten_len[2][0] > 0
+    o = Oracle.from_spec(spec)
+    x = o.init_fields(spec.initial_x())
+    rng = np.random.default_rng(3)
+    x[2:] *= 1.0 + 0.01 * rng.uniform(-1, 1, x[2:].shape)
+    xd = torch.from_numpy(np.ascontiguousarray(x)).cuda()
+    v = torch.from_numpy(rng.uniform(-1, 1, x.shape)).cuda()
+    blocks = ((0, 2), (2, 8), (8, 10))
+    Fo = torch.from_numpy(np.asarray(o.residual(x))).reshape(x.shape).cuda()
+    Fa, Fb = rows.fill_residual(xd)[0], line.fill_residual(xd)[0]
+    _compare(Fo, Fa, blocks, 1e-12)
+    _compare(Fo, Fb, blocks, 1e-12)
+    _compare(rows.apply_jacobian(xd, v), line.apply_jacobian(xd, v), blocks, 1e-12)
+    _compare(rows.apply_jacobian(xd, v, fp32=True), line.apply_jacobian(xd, v, fp32=True), blocks, 1e-5)
+    da, _ = rows.schur_solve(xd, Fo, rtol=1e-30, restart=4, maxit=4)
+    db, _ = line.schur_solve(xd, Fo, rtol=1e-30, restart=4, maxit=4)
+    _compare(da, db, blocks, 1e-8)

@@ -193,8 +193,9 @@ template <typename T>
 void upload_row1d(Problem &P, int type, int idx, int comp, DevRow1DT<T> &dr)
 {
     const HostStencil &hs = P.hs[type][idx];
-    if (hs.L == 0) return;
-    int lo = 1 << 30, hi = -(1 << 30);
+    // an empty stencil (a pair without attraction) keeps a row of zeros: the row kernels read their first
+    // weights before, or without, looking at the length
+    int lo = hs.L ? 1 << 30 : 0, hi = hs.L ? -(1 << 30) : -1;
     for (int k = 0; k < hs.L; ++k) {
         lo = std::min(lo, hs.off[3 * (size_t)k]);
         hi = std::max(hi, hs.off[3 * (size_t)k]);
