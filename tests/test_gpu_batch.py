@@ -263,3 +263,33 @@ def test_batch_newton_segment_lengths(nodes, graph, monkeypatch):
         xs = dp.initial_state()
         assert dp.newton(xs, resid_tol=1e-10, gmres_tol=1e-9, max_iter=60, gmres_restart=7)["converged"]
         assert float((xs - x[:, o[i]:o[i + 1]]).abs().max()) < 1e-8
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("ndim", [1, 2])
+def test_batch_graphs_follow_the_jacobian_mode(ndim, monkeypatch):
+    """set_jacobian between two batched solves on one handle: the replayed graphs run the mode in force, as
+    direct launches do.  FMT4's reference Jacobian is inexact, so two steps of either mode differ."""
+    from tramonto_amd.batch import BatchSpec, DeviceBatch
+    from tramonto_amd.device import JAC_EXACT, JAC_REFERENCE
+    from tramonto_amd.problem import rough_slit_pore_2d, slit_pore_1d
+    pores = [slit_pore_1d(H=3.0, dx=0.05, rho_b=(0.25, 0.25), eps_ff=0.5, seed=i) if ndim == 1 else
+             rough_slit_pore_2d(seed=i, nx=53, ny=33, eps_ff=0.5) for i in range(2)]
+    for p in pores:
+        p.type_func = 3
+    db = DeviceBatch(BatchSpec(pores))
+    x0 = db.initial_state()
+
+    def two_steps(graph):
+        monkeypatch.setenv("TMI_BATCH_GRAPH", graph)
+        x = x0.clone()
+        db.newton(x, max_iter=2, resid_tol=1e-30, gmres_tol=1e-10)
+        return x
+
+    exact = two_steps("1")
+    for mode in (JAC_REFERENCE, JAC_EXACT):
+        db.set_jacobian(mode)
+        graph, direct = two_steps("1"), two_steps("0")
+        assert float((graph - direct).abs().max()) < 1e-10
+        moved = float((graph - exact).abs().max())
+        assert moved > 1e-6 if mode == JAC_REFERENCE else moved < 1e-10

@@ -532,7 +532,8 @@ struct BatchWork {
     // graphs
     hipGraphExec_t g_pre = nullptr, g_start0 = nullptr, g_start = nullptr, g_finish = nullptr, g_post = nullptr;
     std::vector<hipGraphExec_t> g_steps;   // Arnoldi steps [j*kChunk, (j+1)*kChunk)
-    int graph_prec = -1;
+    // what their launches depend on besides the buffers (graph_prec -1: none captured)
+    int graph_prec = -1, graph_rev = 0;
     double graph_tol[2] = {0, 0};
 };
 
@@ -802,15 +803,19 @@ int batch_newton_solve(Problem &P, double *x_caller, const tmi_newton_opts &o, t
     };
     auto enqueue_finish = [&] { stage_cycle_finish(P, W, s); };
     auto enqueue_post = [&] { stage_post(P, W, x, o.update_scaling, s); };
-    if (use_graph && (W.graph_prec != o.precision || W.graph_tol[0] != o.gmres_tol ||
+    if (use_graph && (W.graph_prec != o.precision || W.graph_rev != P.launch_rev || W.graph_tol[0] != o.gmres_tol ||
                       W.graph_tol[1] != o.update_scaling)) {
+        W.graph_prec = -1;   // until every part is captured
         for (hipGraphExec_t *g : {&W.g_pre, &W.g_start0, &W.g_start, &W.g_finish, &W.g_post})
             if (*g) {
                 (void)hipGraphExecDestroy(*g);
                 *g = nullptr;
             }
         for (hipGraphExec_t &g : W.g_steps)
-            if (g) (void)hipGraphExecDestroy(g);
+            if (g) {
+                (void)hipGraphExecDestroy(g);
+                g = nullptr;
+            }
         W.g_steps.assign(nchunks, nullptr);
         W.g_pre = capture(s, enqueue_pre);
         W.g_start0 = capture(s, enqueue_start0);
@@ -819,6 +824,7 @@ int batch_newton_solve(Problem &P, double *x_caller, const tmi_newton_opts &o, t
         W.g_finish = capture(s, enqueue_finish);
         W.g_post = capture(s, enqueue_post);
         W.graph_prec = o.precision;
+        W.graph_rev = P.launch_rev;
         W.graph_tol[0] = o.gmres_tol;
         W.graph_tol[1] = o.update_scaling;
     }

@@ -1264,7 +1264,9 @@ int tmi_problem_set_jacobian(void *handle, int mode)
     return guarded([&] {
         Problem *P = as_problem(handle);
         if (mode != TMI_JAC_EXACT && mode != TMI_JAC_REFERENCE) throw std::invalid_argument("Jacobian mode");
-        P->jac_ref = mode == TMI_JAC_REFERENCE;
+        const bool ref = mode == TMI_JAC_REFERENCE;
+        if (ref != P->jac_ref) ++P->launch_rev;
+        P->jac_ref = ref;
         return 0;
     });
 }
@@ -1433,6 +1435,7 @@ int tmi_row_tuning_set(void *handle, int prec, int kind, int per_lane, int lanes
         P->tune[prec][kind].B = per_lane;
         P->tune[prec][kind].wg = lanes;
         P->tune[prec][kind].ms = 0.0;
+        ++P->launch_rev;
         return 0;
     });
 }

@@ -192,6 +192,7 @@ struct Problem {
     // Jacobian-vector products with the reference's delta-stencil Hessian rows (TMI_JAC_REFERENCE:
     // its assembled entries, including the inexact ones) instead of the exact Hessian
     bool jac_ref = false;
+    int launch_rev = 0;   // counts the settings that changed which kernels a call launches: captured graphs follow it
     double *d_mfw2 = nullptr;   // 2D direct form: dense (2 hy + 1) x (2 hx + 1) attraction weights per component pair
     bool mf2d_mfma = true;      // FP64 dense 2D sums on the matrix cores (TMI_MF2D_MFMA=0: the FMA kernel)
     double *d_rbw2 = nullptr;   // 2D, one component: dense theta, delta, delta x and delta y weights [4][2 fy + 1][2 fx + 1]
