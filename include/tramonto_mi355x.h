@@ -88,9 +88,10 @@ typedef struct tmi_info {
     int precond;  /* preconditioner of the Schur GMRES: TMI_PRECOND_DIAG or TMI_PRECOND_BULK */
     int fft_fold; /* 1: the stencil spectra of the FFT sums are stored for k_y, k_z >= 0 only (every stencil
                      symmetric under the reflection of y and of z), 0: for the whole FFT grid or no FFT sums */
-    int fft_xreg; /* the fused x pass runs in registers (x length 32-256, few enough outputs): bit 0 for the
-                     density product, bit 1 for the Euler-Lagrange product; 0 in LDS or not fused */
-    int fft_regpass; /* strided FFT axes of length 32-256: 0 LDS Stockham passes (TMI_FFT_REGPASS=0), 1 the
+    int fft_xreg; /* the fused x pass runs in its register form, over groups of mirror lines (x length 32, 64, 128 or
+                     256, folded spectra, spectra of a group within LDS): bit 0 for the density product, bit 1 for
+                     the Euler-Lagrange product of an FP64 fill; 0 in LDS or not fused */
+    int fft_regpass; /* strided FFT axes of length 32, 64, 128 or 256: 0 LDS Stockham passes (TMI_FFT_REGPASS=0), 1 the
                         one-wave register pass where a pass has at least 1024 waves, 2 wherever the length
                         allows (TMI_FFT_REGPASS=2); read at creation */
     int jacobian;    /* TMI_JAC_EXACT or TMI_JAC_REFERENCE (tmi_problem_set_jacobian) */

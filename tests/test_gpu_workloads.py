@@ -114,10 +114,10 @@ def test_config2_fft_products_match_direct_sums(config2, monkeypatch, fused):
 
 
 KERNEL_CASES = {
-    # case: (fft_xreg expected with the fused x pass forced, strided register pass expected)
-    "3d_x64": 3,        # k_fft_xprod_reg<T, 8, 8, 3> (density) and <T, 8, 8, 1> (Euler-Lagrange)
-    "3d_x128": 2,       # <T, 16, 8, 1> (Euler-Lagrange); the density product's 3 pairs run in LDS
-    "3d_mix3_x128": 2,  # <T, 16, 8, 2>: three components' Euler-Lagrange rows
+    # case: fft_xreg with the fused x pass forced (bit 0 density, bit 1 Euler-Lagrange product)
+    "3d_x64": 3,        # k_fft_xgroup<T, 8, 8, 4>, both products
+    "3d_x128": 3,       # <T, 16, 8, 4>
+    "3d_mix3_x128": 1,  # the Euler-Lagrange product's four spectrum slots do not fit in LDS
     "3d_yz64": 0,       # x = 12: LDS fused pass; y and z through k_fft_strided<T, +-1, mode, 8, 8>
     "3d_y128_z32": 0,   # y through k_fft_strided<T, +-1, mode, 16, 8>, z through <T, +-1, mode, 8, 4>
 }

@@ -43,6 +43,7 @@ def test_mirror_line_groups_match_lds_form(n, ncomp, monkeypatch):
     monkeypatch.setenv("TMI_FFT_XREG", "0")
     lds = DeviceProblem(spec)
     assert reg.info.fmt_fft == 2 and lds.info.fmt_fft == 2 and reg.info.fft_fold == 1
+    assert reg.info.fft_xreg & 1 and lds.info.fft_xreg == 0   # the forms compared are two forms
     x = reg.initial_state()
     g = torch.Generator(device="cuda").manual_seed(9)
     rnd = lambda: 2 * torch.rand(x.shape, generator=g, device="cuda", dtype=torch.float64) - 1  # noqa: E731

@@ -2226,61 +2226,64 @@ int xprod_lpb(const FftPlan &F, int nop)
     return (M * sizeof(Cx<double>) + lpb * per_line <= kXprodLds) ? lpb : 0;
 }
 
-// products reported as running in registers throughout: register radices and output pairs whose spectrum
-// values fit in one lane's registers (NOP R1 <= 32)
-inline bool xreg_fits(const FftPlan &F, const TermList &tl, int &R1, int &R2)
-{
-    if (!F.xreg || !reg_radices(F.M[0], R1, R2)) return false;
-    const int nop = (tl.nout + 1) / 2;
-    return nop <= 4 && nop * R1 <= 32;
-}
-
 // The register form of the fused x pass, where the x length has register radices.  A product of more than
 // two output pairs keeps every input spectrum in LDS and deals the outputs to up to 4 waves; one of few
 // outputs runs two waves that refill two slots, which leaves LDS for more workgroups, or, where there
 // are too few workgroups for that to matter, one wave and slot per input pair.
+struct XgroupShape {
+    int R1, R2, nl, waves, slots;   // radices, lines of a group, waves and spectrum slots of a workgroup
+    bool alias;                     // one output pair per wave: the work rows take the spectra's place
+    long long wgs;
+    size_t lds;
+};
+template <typename T>
+bool xgroup_shape(const FftPlan &F, const TermList &tl, XgroupShape &g)
+{
+    if (!F.xreg || !F.fold || F.tn >= (1LL << 29) || !reg_radices(F.M[0], g.R1, g.R2) || !tl.steps) return false;
+    const int nip = (tl.nin + 1) / 2, nop = (tl.nout + 1) / 2, L = 64 / g.R2;
+    g.nl = F.M[2] > 1 ? 4 : 2;
+    const int per = L / g.nl;
+    const long long groups = (long long)(F.M[1] / 2 + 1) * (F.M[2] / 2 + 1);
+    g.wgs = (groups + per - 1) / per;
+    if (nop > 2) {
+        g.waves = std::min(nop, 4);
+        g.slots = nip;
+    } else {
+        g.waves = g.slots = std::min(nip, g.wgs < 4 * 256 ? 4 : 2);
+        g.waves = std::max(g.waves, nop);
+    }
+    g.alias = nop <= g.waves;
+    const size_t line = (size_t)L * (g.R1 * (g.R2 + 1) + 1);   // elements of a slot
+    // twiddles, spectra, then each wave's work rows; or each wave's 256 table values, and the work rows in the spectra's place
+    g.lds = (size_t)F.M[0] * sizeof(Cx<T>) +
+            (g.alias ? std::max((size_t)g.slots * line * sizeof(Cx<T>) + g.waves * 256 * sizeof(T), g.waves * line * sizeof(T))
+                     : (size_t)g.slots * line * sizeof(Cx<T>) + g.waves * line * sizeof(T));
+    return g.lds <= kXgroupLds;
+}
 template <typename T>
 bool xprod_reg(const FftPlan &F, const Cx<T> *Z, Cx<T> *O, const TermList &tl, const T *tk, const T *uk, hipStream_t s)
 {
-    int R1 = 0, R2 = 0;
-    if (!F.xreg || !F.fold || F.tn >= (1LL << 29) || !reg_radices(F.M[0], R1, R2)) return false;
-    if (!tl.steps) return false;
-    const int nip = (tl.nin + 1) / 2, nop = (tl.nout + 1) / 2, L = 64 / R2;
-    const int nl = F.M[2] > 1 ? 4 : 2, per = L / nl;
-    const long long groups = (long long)(F.M[1] / 2 + 1) * (F.M[2] / 2 + 1), wgs = (groups + per - 1) / per;
-    int waves, slots;
-    if (nop > 2) {
-        waves = std::min(nop, 4);
-        slots = nip;
-    } else {
-        waves = slots = std::min(nip, wgs < 4 * 256 ? 4 : 2);
-        waves = std::max(waves, nop);
-    }
-    const bool alias = nop <= waves;
-    const size_t line = (size_t)L * (R1 * (R2 + 1) + 1);   // elements of a slot
-    // twiddles, spectra, then each wave's work rows; or each wave's 256 table values, and the work rows in the spectra's place
-    const size_t lds = (size_t)F.M[0] * sizeof(Cx<T>) +
-                       (alias ? std::max((size_t)slots * line * sizeof(Cx<T>) + waves * 256 * sizeof(T), waves * line * sizeof(T))
-                              : (size_t)slots * line * sizeof(Cx<T>) + waves * line * sizeof(T));
-    if (lds > kXgroupLds) return false;
+    XgroupShape g;
+    if (!xgroup_shape<T>(F, tl, g)) return false;
+    const int nip = (tl.nin + 1) / 2, nop = (tl.nout + 1) / 2;
     auto go = [&](auto kernel) {
-        if (lds > 64 * 1024)
-            TMI_HIP_CHECK(hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-        hipLaunchKernelGGL(kernel, dim3((unsigned)wgs), dim3(64 * waves), lds, s, Z, O, F.ns, F.M[1], F.M[2], F.S1, F.S2, slots,
-                           alias ? 1 : 0, twiddles<T>(F, 0), tk, uk, tab_geo(F), tl.steps, tl.start, nip, nop, F.xcdmap);
+        if (g.lds > 64 * 1024)
+            TMI_HIP_CHECK(hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)g.lds));
+        hipLaunchKernelGGL(kernel, dim3((unsigned)g.wgs), dim3(64 * g.waves), g.lds, s, Z, O, F.ns, F.M[1], F.M[2], F.S1, F.S2, g.slots,
+                           g.alias ? 1 : 0, twiddles<T>(F, 0), tk, uk, tab_geo(F), tl.steps, tl.start, nip, nop, F.xcdmap);
     };
     auto by_lines = [&](auto r1, auto r2) {
         constexpr int A = decltype(r1)::value, B = decltype(r2)::value;
-        if (nl == 4)
+        if (g.nl == 4)
             go(k_fft_xgroup<T, A, B, 4>);
         else
             go(k_fft_xgroup<T, A, B, 2>);
     };
-    if (R1 == 8 && R2 == 4)
+    if (g.R1 == 8 && g.R2 == 4)
         by_lines(std::integral_constant<int, 8>{}, std::integral_constant<int, 4>{});
-    else if (R1 == 8 && R2 == 8)
+    else if (g.R1 == 8 && g.R2 == 8)
         by_lines(std::integral_constant<int, 8>{}, std::integral_constant<int, 8>{});
-    else if (R1 == 16 && R2 == 8)
+    else if (g.R1 == 16 && g.R2 == 8)
         by_lines(std::integral_constant<int, 16>{}, std::integral_constant<int, 8>{});
     else
         by_lines(std::integral_constant<int, 16>{}, std::integral_constant<int, 16>{});
@@ -2810,9 +2813,10 @@ int fft_xreg_mask(const Problem &P)
 {
     if (!P.fft || !P.fft->fmt) return 0;
     const FftPlan &F = *P.fft;
-    int R1 = 0, R2 = 0, m = 0;
-    if (F.xlpb[0] && xreg_fits(F, F.tfwd[1], R1, R2)) m |= 1;
-    if (F.xlpb[1] && xreg_fits(F, F.tel, R1, R2)) m |= 2;
+    XgroupShape g;
+    int m = 0;
+    if (F.xlpb[0] && xgroup_shape<double>(F, F.tfwd[1], g)) m |= 1;
+    if (F.xlpb[1] && xgroup_shape<double>(F, F.dform ? F.tel_d : F.tel, g)) m |= 2;
     return m;
 }
 int fft_regpass_mode(const Problem &P) { return P.fft ? P.fft->regpass : 0; }
