@@ -117,7 +117,7 @@ KERNEL_CASES = {
     # case: fft_xreg with the fused x pass forced (bit 0 density, bit 1 Euler-Lagrange product)
     "3d_x64": 3,        # k_fft_xgroup<T, 8, 8, 4>, both products
     "3d_x128": 3,       # <T, 16, 8, 4>
-    "3d_mix3_x128": 1,  # the Euler-Lagrange product's four spectrum slots do not fit in LDS
+    "3d_mix3_x128": 1,  # the Euler-Lagrange product's four spectrum slots do not fit: LDS form on so few lines
     "3d_yz64": 0,       # x = 12: LDS fused pass; y and z through k_fft_strided<T, +-1, mode, 8, 8>
     "3d_y128_z32": 0,   # y through k_fft_strided<T, +-1, mode, 16, 8>, z through <T, +-1, mode, 8, 4>
 }

@@ -33,7 +33,8 @@ def _fluid(n, ncomp):
 @pytest.mark.gpu
 @pytest.mark.parametrize("n,ncomp", [((32, 15, 16), 1), ((64, 16, 15), 2), ((128, 16, 15), 3), ((128, 15, 18), 4),
                                      ((256, 16, 15), 1), ((256, 15, 15), 3), ((32, 27), 2), ((64, 16), 1), ((128, 25), 3),
-                                     ((256, 18), 1), ((64, 64, 64), 4)])
+                                     ((256, 18), 1), ((64, 64, 64), 4),
+                                     ((128, 32, 32), 3), ((128, 46, 46), 3)])   # three and two slots for five input pairs
 def test_mirror_line_groups_match_lds_form(n, ncomp, monkeypatch):
     from tramonto_amd.device import DeviceProblem
     spec = _fluid(n, ncomp)
@@ -43,7 +44,9 @@ def test_mirror_line_groups_match_lds_form(n, ncomp, monkeypatch):
     monkeypatch.setenv("TMI_FFT_XREG", "0")
     lds = DeviceProblem(spec)
     assert reg.info.fmt_fft == 2 and lds.info.fmt_fft == 2 and reg.info.fft_fold == 1
-    assert reg.info.fft_xreg & 1 and lds.info.fft_xreg == 0   # the forms compared are two forms
+    # the forms compared are two forms (a product of many pairs on few lines of 128 or 256 keeps the LDS form)
+    assert reg.info.fft_xreg == 3 if max(n[1:]) >= 32 else reg.info.fft_xreg & 1
+    assert lds.info.fft_xreg == 0
     x = reg.initial_state()
     g = torch.Generator(device="cuda").manual_seed(9)
     rnd = lambda: 2 * torch.rand(x.shape, generator=g, device="cuda", dtype=torch.float64) - 1  # noqa: E731

@@ -2229,7 +2229,10 @@ int xprod_lpb(const FftPlan &F, int nop)
 // The register form of the fused x pass, where the x length has register radices.  A product of more than
 // two output pairs keeps every input spectrum in LDS and deals the outputs to up to 4 waves; one of few
 // outputs runs two waves that refill two slots, which leaves LDS for more workgroups, or, where there
-// are too few workgroups for that to matter, one wave and slot per input pair.
+// are too few workgroups for that to matter, one wave and slot per input pair.  Where those do not fit: two
+// slots again if the workgroups cover the CUs (128 x 64^2, three components: fill 211 us, with three slots or the
+// LDS form 221), else three (128 x 32^2: 103, with two 105, LDS form 109); a few workgroups leave the lines
+// to the LDS form, which spreads them over more (128^2, two components: 77, with two or three slots 79).
 struct XgroupShape {
     int R1, R2, nl, waves, slots;   // radices, lines of a group, waves and spectrum slots of a workgroup
     bool alias;                     // one output pair per wave: the work rows take the spectra's place
@@ -2245,20 +2248,23 @@ bool xgroup_shape(const FftPlan &F, const TermList &tl, XgroupShape &g)
     const int per = L / g.nl;
     const long long groups = (long long)(F.M[1] / 2 + 1) * (F.M[2] / 2 + 1);
     g.wgs = (groups + per - 1) / per;
-    if (nop > 2) {
-        g.waves = std::min(nop, 4);
-        g.slots = nip;
-    } else {
-        g.waves = g.slots = std::min(nip, g.wgs < 4 * 256 ? 4 : 2);
-        g.waves = std::max(g.waves, nop);
-    }
-    g.alias = nop <= g.waves;
     const size_t line = (size_t)L * (g.R1 * (g.R2 + 1) + 1);   // elements of a slot
-    // twiddles, spectra, then each wave's work rows; or each wave's 256 table values, and the work rows in the spectra's place
-    g.lds = (size_t)F.M[0] * sizeof(Cx<T>) +
-            (g.alias ? std::max((size_t)g.slots * line * sizeof(Cx<T>) + g.waves * 256 * sizeof(T), g.waves * line * sizeof(T))
-                     : (size_t)g.slots * line * sizeof(Cx<T>) + g.waves * line * sizeof(T));
-    return g.lds <= kXgroupLds;
+    auto fits = [&](int waves, int slots) {
+        g.waves = std::min(std::max(waves, nop), 4);
+        g.slots = slots;
+        g.alias = nop <= g.waves;
+        // twiddles, spectra, then each wave's work rows; or each wave's 256 table values, and the work rows in the spectra's place
+        g.lds = (size_t)F.M[0] * sizeof(Cx<T>) +
+                (g.alias ? std::max((size_t)slots * line * sizeof(Cx<T>) + g.waves * 256 * sizeof(T), g.waves * line * sizeof(T))
+                         : (size_t)slots * line * sizeof(Cx<T>) + g.waves * line * sizeof(T));
+        return g.lds <= kXgroupLds;
+    };
+    if (nop > 2) return fits(0, nip);
+    const int most = std::min(nip, g.wgs < 4 * 256 ? 4 : 2);
+    if (fits(most, most)) return true;
+    // lines of 128 and 256 in FP64 hold three slots (4 and more input pairs: mixtures)
+    const int less = g.wgs >= 256 ? 2 : 3;
+    return g.wgs >= 128 && fits(less, less);
 }
 template <typename T>
 bool xprod_reg(const FftPlan &F, const Cx<T> *Z, Cx<T> *O, const TermList &tl, const T *tk, const T *uk, hipStream_t s)
