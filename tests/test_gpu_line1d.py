@@ -119,3 +119,29 @@ def test_pair_without_attraction(nodes, monkeypatch):
     da, _ = rows.schur_solve(xd, Fo, rtol=1e-30, restart=4, maxit=4)
     db, _ = line.schur_solve(xd, Fo, rtol=1e-30, restart=4, maxit=4)
     _compare(da, db, blocks, 1e-8)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("nodes", [2600, 4096, 4097, 8192])   # one workgroup's sweep ends at step 76, 48, 17, 8
+def test_long_krylov_cycles(nodes, precision, monkeypatch):
+    """Cycles that go on past the basis one workgroup sweeps, restarted ones and ones cut by the iteration limit
+    among them: the same steps as the general GMRES (TMI_LINE1D=0).  rtol 1e-9 bounds the distance of two
+    updates by the condition of a dense fluid's Schur system, below 1e3; in mixed precision the FP32 product
+    carries 1e-6 of the update, and the general solver's basis is FP32 too."""
+    from tramonto_amd.device import PREC_FP64, PREC_MIXED
+    spec = hard_wall_1d(seed=2, size=0.05 * (nodes - 1), dx=0.05, rho_b=0.8)
+    rows, line = _problems(lambda: DeviceProblem(spec), monkeypatch)
+    x = rows.initial_state()
+    F, _ = rows.fill_residual(x)
+    prec, tol = (PREC_FP64, 1e-6) if precision == "fp64" else (PREC_MIXED, 1e-3)
+    for restart, maxit in ((200, 400), (30, 400), (200, 55)):
+        da, ia = rows.schur_solve(x, F, rtol=1e-9, restart=restart, maxit=maxit, precision=prec)
+        db, ib = line.schur_solve(x, F, rtol=1e-9, restart=restart, maxit=maxit, precision=prec)
+        assert 50 < ib <= maxit
+        if precision == "fp64":
+            assert abs(ia - ib) <= 1
+        if ia < maxit and ib < maxit:
+            assert float((da - db).abs().max()) <= tol * float(da.abs().max())
+        elif precision == "fp64":   # cut after the same number of steps
+            assert ia == ib and float((da - db).abs().max()) <= tol * float(da.abs().max())

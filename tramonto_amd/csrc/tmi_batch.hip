@@ -183,6 +183,37 @@ __global__ __launch_bounds__(kSegBlock) void k_seg_normalize(const double *__res
     }
 }
 
+// One thread: the new Hessenberg column h[0 .. k] and norm hn of segment p under the rotations cs, sn of the
+// columns before it (h, cs, sn: LDS), its own rotation, the residual and the convergence flag; mirror
+// (optional, pinned host memory): the flag and the step count.
+__device__ inline void givens_column(double *h, double hn, int k, const double *cs, const double *sn, const GmresState &st, int p,
+                                     double tol, double *mirror)
+{
+    const int m = st.m;
+    double up = h[0];
+    for (int j = 0; j < k; ++j) {
+        const double b = h[j + 1];
+        h[j] = cs[j] * up + sn[j] * b;
+        up = -sn[j] * up + cs[j] * b;
+    }
+    const double den = sqrt(up * up + hn * hn);
+    const double c = den > 0.0 ? up / den : 1.0, sv = den > 0.0 ? hn / den : 0.0;
+    h[k] = den;
+    st.cs[(size_t)p * m + k] = c;
+    st.sn[(size_t)p * m + k] = sv;
+    double *g = st.g + (size_t)p * (m + 1);
+    const double gk = g[k], gn = -sv * gk;
+    g[k + 1] = gn;
+    g[k] = c * gk;
+    st.kdone[p] = k + 1;
+    const int done = fabs(gn) <= tol * st.bn[p] || hn == 0.0;
+    if (done) st.done[p] = 1;
+    if (mirror) {
+        mirror[0] = done;
+        mirror[1] = k + 1;
+    }
+}
+
 // One Arnoldi step of every segment in one launch: classical Gram-Schmidt of w against V_0 .. V_k with
 // one reorthogonalisation pass, the normalised result as V_k+1, the new Hessenberg column with its
 // Givens rotations, and the convergence flag.  One workgroup per segment (the segments are
@@ -295,30 +326,7 @@ __global__ __launch_bounds__(BT) void k_seg_ortho(double *__restrict__ V, long l
     }
     __syncthreads();
     const double hn = nrm;
-    if (tid == 0) {   // previous rotations, the new one, the residual
-        double up = h[0];
-        for (int j = 0; j < k; ++j) {
-            const double b = h[j + 1];
-            h[j] = cs[j] * up + sn[j] * b;
-            up = -sn[j] * up + cs[j] * b;
-        }
-        const double den = sqrt(up * up + hn * hn);
-        const double c = den > 0.0 ? up / den : 1.0, sv = den > 0.0 ? hn / den : 0.0;
-        h[k] = den;
-        st.cs[(size_t)p * m + k] = c;
-        st.sn[(size_t)p * m + k] = sv;
-        double *g = st.g + (size_t)p * (m + 1);
-        const double gk = g[k], gn = -sv * gk;
-        g[k + 1] = gn;
-        g[k] = c * gk;
-        st.kdone[p] = k + 1;
-        const int done = fabs(gn) <= tol * st.bn[p] || hn == 0.0;
-        if (done) st.done[p] = 1;
-        if (mirror) {
-            mirror[0] = done;
-            mirror[1] = k + 1;
-        }
-    }
+    if (tid == 0) givens_column(h, hn, k, cs, sn, st, p, tol, mirror);
     const double inv = hn > 0.0 ? 1.0 / hn : 0.0;
     double *out = V + (size_t)(k + 1) * ldv;
 #pragma unroll
@@ -359,6 +367,25 @@ __global__ void k_line_start(GmresState st, const int *__restrict__ active, doub
         mirror[0] = done;
         mirror[1] = 0.0;
     }
+}
+
+// the column of one problem's step k whose Gram-Schmidt ran over the chip (dev_cgs2's coefficients, |w|^2 last)
+__global__ __launch_bounds__(64) void k_line_givens(GmresState st, int k, const double *__restrict__ coef, double tol,
+                                                    double *__restrict__ mirror)
+{
+    __shared__ double h[kOrthoMaxM + 1], cs[kOrthoMaxM], sn[kOrthoMaxM];
+    const int m = st.m;
+    for (int j = threadIdx.x; j <= k; j += 64) {
+        h[j] = coef[j] + coef[k + 1 + j];
+        if (j < k) {
+            cs[j] = st.cs[j];
+            sn[j] = st.sn[j];
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) givens_column(h, sqrt(coef[2 * (k + 1)]), k, cs, sn, st, 0, tol, mirror);
+    __syncthreads();
+    for (int j = threadIdx.x; j <= k; j += 64) st.H[(size_t)j * m + k] = h[j];
 }
 
 // Arnoldi step k: new column (h1 + h2, hn) of each active pore's Hessenberg
@@ -901,14 +928,18 @@ int batch_newton_solve(Problem &P, double *x_caller, const tmi_newton_opts &o, t
 
 // One small 1D problem (the whole vector is one segment): two launches per Arnoldi step, and the host
 // reads the convergence flag every kLineSteps steps; steps past convergence return at once.
-// The rule: the Schur product in one launch, and a basis that one workgroup sweeps faster than eight
-// launches over the chip do (up to 8192 unknowns; 601 nodes of two components: Newton 4.1 -> 2.2 ms).
+// The rule: the Schur product in one launch, up to 8192 unknowns (601 nodes of two components: Newton 4.1 ->
+// 2.2 ms), and while the basis is one that a workgroup sweeps faster than eight launches over the chip do:
+// `sweep` values of it, fewer where a thread holds more than four values of w.  From there on the
+// Gram-Schmidt passes run over the chip, with the rotations still on the device and one host read per step.
+// A step on average, 84 of them at 3001 unknowns: 105 us in one workgroup throughout, 102 so, 136 with the rotations
+// on the host (gmres_schur_t); 83 at 8001: 222, 108 and 136 us.
 bool gmres_line(Problem &P, const double *x, const double *bS, double *x2, double rtol, int m, int maxit, int prec,
                 double *work, int *iters, hipStream_t s)
 {
     constexpr int kLineSteps = 4, kLineMax = 8192;
     const int C = P.p.ncomp, N = P.N;
-    const long long n = (long long)C * N;
+    const long long n = (long long)C * N, sweep = n <= 4096 ? 200000 : 70000;
     if (P.npores > 0 || !line_available(P) || !schur_one_launch(P) || n > kLineMax || m > kOrthoMaxM) return false;
     if (P.line_gs_m != m) {
         (void)hipFree(P.d_line_gs);
@@ -960,9 +991,18 @@ bool gmres_line(Problem &P, const double *x, const double *bS, double *x2, doubl
         const int steps = std::min(m, maxit - its);
         int k = 0, done = 0;
         while (k < steps && !done) {
-            for (const int end = std::min(steps, k + kLineSteps); k < end; ++k) {
-                product(V + (size_t)k * n, dinv, st.done);
-                launch_ortho(V, n, k, w, C, N, off, 1, (int)n, st, rtol, P.h_red_dev, s);
+            const int narrow = (int)std::min<long long>(steps, sweep / n);   // steps of one workgroup
+            if (k < narrow) {
+                for (const int end = std::min(narrow, k + kLineSteps); k < end; ++k) {
+                    product(V + (size_t)k * n, dinv, st.done);
+                    launch_ortho(V, n, k, w, C, N, off, 1, (int)n, st, rtol, P.h_red_dev, s);
+                }
+            } else {
+                double *coef = P.d_red + kRedPartials;
+                product(V + (size_t)k * n, dinv, nullptr);
+                dev_cgs2<double>(P, V, n, k + 1, w, n, V + (size_t)(k + 1) * n, coef, s);
+                hipLaunchKernelGGL(k_line_givens, dim3(1), dim3(64), 0, s, st, k, coef, rtol, P.h_red_dev);
+                ++k;
             }
             TMI_HIP_CHECK(hipStreamSynchronize(s));
             done = P.h_red[0] != 0.0;

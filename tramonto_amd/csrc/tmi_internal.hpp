@@ -111,6 +111,8 @@ struct Grid {
     int N;
 };
 
+constexpr long long kRedPartials = 512 * 1024;   // partial sums in Problem::d_red, clear of the Arnoldi coefficients past them
+
 struct Problem;
 struct BatchWork;
 struct FftPlan;

@@ -2264,7 +2264,6 @@ void residual_sumsq_device(Problem &P, const double *x, double *F, double *parti
     TMI_HIP_CHECK(hipGetLastError());
 }
 
-constexpr long long kRedPartials = 512 * 1024;   // partial sums in P.d_red, clear of the Arnoldi coefficients past them
 double residual_sumsq(Problem &P, const double *x, double *F, hipStream_t s)
 {
     long long cap = 0, cnt = 0;
