@@ -276,6 +276,12 @@ int tmi_newton_solve(void *handle, double *x_d, const tmi_newton_opts *opts, tmi
 int tmi_schur_solve(void *handle, const double *x_d, const double *F_d, double *dx_d, double rtol, int restart,
                     int maxit, int precision, int *iters, void *stream);
 
+/* The form in which a residual fill's rows run (no counterpart in the reference): *form 0 separate stencil
+ * kernels or FFT sums (tmi_info.fmt_fft, mf_fft), 1 every row of a 1D problem or batch in one launch, 2 every
+ * row of a one-component 2D problem or batch in one launch on the matrix cores; *width the positions per
+ * lane (1, 2, 4) of form 1, the wavefronts per workgroup (8, 16) of form 2 in FP64, else 0.  Either may be
+ * NULL. */
+int tmi_row_form(void *handle, int *form, int *width);
 /* Launch shapes the autotuner chose for the 1D row kernels (1D problems and
  * batches; no counterpart in the reference): shape[prec][kind][2] = outputs
  * per lane and lanes per workgroup, ms[prec][kind] = measured time, prec 0

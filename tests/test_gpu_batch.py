@@ -28,6 +28,19 @@ def small():
     return b, oracles, DeviceBatch(b)
 
 
+@pytest.fixture(scope="module")
+def small_rows(small):
+    """the same batch through the separate row kernels"""
+    from tramonto_amd.batch import DeviceBatch
+    b, oracles, _ = small
+    old = os.environ.get("TMI_LINE1D")
+    os.environ["TMI_LINE1D"] = "0"
+    try:
+        return b, oracles, DeviceBatch(b)
+    finally:
+        os.environ.pop("TMI_LINE1D") if old is None else os.environ.update(TMI_LINE1D=old)
+
+
 def dev(a):
     return torch.from_numpy(np.ascontiguousarray(a)).to("cuda")
 
@@ -135,12 +148,13 @@ def test_batch_newton_matches_single_pore_solves(small):
 @pytest.mark.gpu
 @pytest.mark.parametrize("per_lane", [4, 8, 16])
 @pytest.mark.parametrize("lanes", [64, 128, 256])
-def test_every_row_kernel_shape_matches_oracle(small, per_lane, lanes):
+def test_every_row_kernel_shape_matches_oracle(small_rows, per_lane, lanes):
     """Every launch shape the 1D autotuner can choose (outputs per lane x lanes per workgroup, for the
     rho-bar, mean-field and Euler-Lagrange row kernels, FP64 and FP32), forced with
     tmi_row_tuning_set: residual and J v per pore against the oracle to 1e-12, the FP32 product
     against FP64 to 1e-5."""
-    b, oracles, db = small
+    b, oracles, db = small_rows
+    assert db.row_form()[0] == 0   # the row kernels, not all rows in one launch
     db.set_row_tuning(per_lane, lanes)
     tun = db.row_tuning()
     assert all(tun[p][k][:2] == (per_lane, lanes) for p in tun for k in tun[p] if tun[p][k][0])

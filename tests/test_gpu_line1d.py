@@ -9,9 +9,10 @@ import pytest
 torch = pytest.importorskip("torch")
 
 from tramonto_amd.batch import DeviceBatch, slit_pore_batch  # noqa: E402
-from tramonto_amd.device import DeviceProblem  # noqa: E402
+from tramonto_amd.device import PREC_MIXED, DeviceProblem  # noqa: E402
 from tramonto_amd.problem import (FMT3, IN_BULK, IN_WALL, PERIODIC, REFLECT, hard_wall_1d, slit_pore_1d,  # noqa: E402
                                   small_case)
+from linear_update import check_batch_step, check_update, row_scale  # noqa: E402
 
 
 def _single(kind):
@@ -44,7 +45,9 @@ def _problems(make, monkeypatch):
     monkeypatch.setenv("TMI_LINE1D", "0")
     a = make()
     monkeypatch.setenv("TMI_LINE1D", "1")
-    return a, make()
+    b = make()
+    assert a.row_form()[0] == 0 and b.row_form()[0] == 1   # the forms compared are two forms
+    return a, b
 
 
 def _compare(a, b, blocks, tol):
@@ -87,10 +90,23 @@ def test_line_matches_row_kernels(kind, monkeypatch):
     v = noise()
     _compare(rows.apply_jacobian(x, v), line.apply_jacobian(x, v), blocks, 1e-12)
     _compare(rows.apply_jacobian(x, v, fp32=True), line.apply_jacobian(x, v, fp32=True), blocks, 1e-5)
-    if not batch:   # Schur product, right-hand side and back-substitution: one Newton update
-        da, _ = rows.schur_solve(x, Fa, rtol=1e-12)
-        db, _ = line.schur_solve(x, Fa, rtol=1e-12)
-        _compare(da, db, blocks, 1e-8)
+    # Schur product, right-hand side and back-substitution: one Newton update
+    da, _ = rows.schur_solve(x, Fa, rtol=1e-12)
+    db, _ = line.schur_solve(x, Fa, rtol=1e-12)
+    _compare(da, db, blocks, 1e-8)
+    dm, _ = line.schur_solve(x, Fa, rtol=1e-8, restart=500, maxit=2500, precision=PREC_MIXED)
+    check_update(rows, x, Fa, dm, C, row_scale(rows, x, C, g), mixed=True)
+    assert line.row_form()[1] == {"long2": 2, "long4": 4, "batch_large": 4}.get(kind, 1)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mixed", [False, True])
+@pytest.mark.parametrize("npores", [5, 80])   # one and four positions per lane
+def test_batched_step_solves_each_pore(npores, mixed, monkeypatch):
+    """Batched Schur products: the direction scaled on the way in, workgroups of finished pores skipped."""
+    spec = slit_pore_batch(npores=npores, seed=5)
+    rows, line = _problems(lambda: DeviceBatch(spec), monkeypatch)
+    check_batch_step(line, rows, mixed, torch.Generator(device="cuda").manual_seed(2))
 
 
 @pytest.mark.gpu
@@ -129,7 +145,7 @@ def test_long_krylov_cycles(nodes, precision, monkeypatch):
     among them: the same steps as the general GMRES (TMI_LINE1D=0).  rtol 1e-9 bounds the distance of two
     updates by the condition of a dense fluid's Schur system, below 1e3; in mixed precision the FP32 product
     carries 1e-6 of the update, and the general solver's basis is FP32 too."""
-    from tramonto_amd.device import PREC_FP64, PREC_MIXED
+    from tramonto_amd.device import PREC_FP64
     spec = hard_wall_1d(seed=2, size=0.05 * (nodes - 1), dx=0.05, rho_b=0.8)
     rows, line = _problems(lambda: DeviceProblem(spec), monkeypatch)
     x = rows.initial_state()

@@ -9,9 +9,10 @@ import pytest
 torch = pytest.importorskip("torch")
 
 from tramonto_amd.batch import BatchSpec, DeviceBatch, rough_slit_pore_batch_2d  # noqa: E402
-from tramonto_amd.device import DeviceProblem  # noqa: E402
+from tramonto_amd.device import PREC_MIXED, DeviceProblem  # noqa: E402
 from tramonto_amd.problem import (IN_BULK, IN_WALL, PERIODIC, REFLECT, ProblemSpec, SplitMix64, rough_slit_pore_2d,  # noqa: E402
                                   rough_wall_2d, small_case)
+from linear_update import check_batch_step, check_update, row_scale  # noqa: E402
 
 
 def _box(nx, ny, bc, cut=1.5, dx=0.1, func=0, seed=3):
@@ -64,6 +65,8 @@ def test_plane_matches_separate_kernels(kind, monkeypatch):
         monkeypatch.delenv(v)
     monkeypatch.setenv("TMI_PLANE2D", "2")   # the matrix-core form without the timing against the others
     plane = make()
+    # the forms compared are two forms
+    assert rows.row_form()[0] == 0 and plane.row_form() == (2, 16 if kind == "fine" else 8)
     C, R = 1, 8
     x = rows.initial_state()
     blocks = ((0, C), (C, C + R), (C + R, x.shape[0]))
@@ -78,7 +81,27 @@ def test_plane_matches_separate_kernels(kind, monkeypatch):
     v = noise()
     _compare(rows.apply_jacobian(x, v), plane.apply_jacobian(x, v), blocks, 1e-12)
     _compare(rows.apply_jacobian(x, v, fp32=True), plane.apply_jacobian(x, v, fp32=True), blocks, 1e-5)
-    if not batch:   # Schur product, right-hand side and back-substitution: one Newton update
-        da, _ = rows.schur_solve(x, Fa, rtol=1e-12)
-        db, _ = plane.schur_solve(x, Fa, rtol=1e-12)
-        _compare(da, db, blocks, 1e-8)
+    # Schur product, right-hand side and back-substitution: one Newton update
+    da, _ = rows.schur_solve(x, Fa, rtol=1e-12)
+    db, _ = plane.schur_solve(x, Fa, rtol=1e-12)
+    _compare(da, db, blocks, 1e-8)
+    dm, _ = plane.schur_solve(x, Fa, rtol=1e-8, restart=500, maxit=2500, precision=PREC_MIXED)   # hard systems among them
+    check_update(rows, x, Fa, dm, C, row_scale(rows, x, C, g), mixed=True)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mixed", [False, True])
+@pytest.mark.parametrize("walls", [False, True])
+def test_batched_step_solves_each_piece(walls, mixed, monkeypatch):
+    """Batched Schur products of 2D pieces: walls between pieces (and at their x ends), tiles of finished
+    pieces skipped."""
+    spec = rough_slit_pore_batch_2d(npores=4, seed=4, nx=53, h_range=(3.0, 5.0))
+    if walls:
+        for p in spec.pores:
+            p.bc = [[IN_WALL, IN_WALL], [IN_WALL, IN_WALL]]
+    monkeypatch.setenv("TMI_PLANE2D", "0")
+    rows = DeviceBatch(spec)
+    monkeypatch.setenv("TMI_PLANE2D", "2")
+    plane = DeviceBatch(spec)
+    assert rows.row_form()[0] == 0 and plane.row_form()[0] == 2
+    check_batch_step(plane, rows, mixed, torch.Generator(device="cuda").manual_seed(2))

@@ -81,7 +81,7 @@ DECLARED_SYMBOLS = [
     "tmi_last_error", "tmi_version", "tmi_problem_create", "tmi_problem_destroy", "tmi_problem_info",
     "tmi_stencil_get", "tmi_bulk_get", "tmi_host_stencil", "tmi_host_bulk", "tmi_apply_jacobian_fp32", "tmi_fill_residual_timed", "tmi_fill_residual_noalloc", "tmi_fft_timed", "tmi_fill_residual", "tmi_apply_jacobian", "tmi_apply_jacobian_transpose",
     "tmi_init_fields", "tmi_set_hard_surface_masks", "tmi_compute_force", "tmi_newton_solve", "tmi_schur_solve", "tmi_set_active_problem",
-    "tmi_batch_create", "tmi_batch_info", "tmi_batch_newton_solve", "tmi_row_tuning", "tmi_row_tuning_set",
+    "tmi_batch_create", "tmi_batch_info", "tmi_batch_newton_solve", "tmi_row_form", "tmi_row_tuning", "tmi_row_tuning_set",
     "tmi_problem_set_rho_b", "tmi_problem_set_vext", "tmi_problem_set_preconditioner", "tmi_problem_set_jacobian", "tmi_compute_observables",
     "fill_resid_and_matrix_control", "tmi_linprobmgr_last_solve",
     "dft_parameterlist_create", "dft_parameterlist_destruct", "dft_parameterlist_set_int", "dft_parameterlist_set_double",
@@ -131,6 +131,7 @@ def lib() -> ct.CDLL:
     L.tmi_newton_solve.argtypes = [vp, vp, ct.POINTER(TmiNewtonOpts), ct.POINTER(TmiNewtonStats), vp]
     L.tmi_schur_solve.argtypes = [vp, vp, vp, vp, d, i, i, i, ct.POINTER(i), vp]
     L.tmi_set_active_problem.argtypes = [vp, vp]
+    L.tmi_row_form.argtypes = [vp, ct.POINTER(i), ct.POINTER(i)]
     L.tmi_row_tuning.argtypes = [vp, vp, vp]
     L.tmi_row_tuning_set.argtypes = [vp, i, i, i, i]
     L.tmi_problem_set_rho_b.argtypes = [vp, vp]

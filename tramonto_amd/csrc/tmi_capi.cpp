@@ -1406,6 +1406,17 @@ int tmi_newton_solve(void *handle, double *x_d, const tmi_newton_opts *opts, tmi
     });
 }
 
+int tmi_row_form(void *handle, int *form, int *width)
+{
+    return guarded([&] {
+        Problem *P = as_problem(handle);
+        const int f = plane_on(*P) ? 2 : (line_available(*P) ? 1 : 0);
+        if (form) *form = f;
+        if (width) *width = f == 2 ? plane_waves(*P) : (f == 1 ? line_lanes(*P) : 0);
+        return 0;
+    });
+}
+
 int tmi_row_tuning(void *handle, int *shape, double *ms)
 {
     return guarded([&] {

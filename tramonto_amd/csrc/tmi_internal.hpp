@@ -245,6 +245,7 @@ void launch_schur_backsub(Problem &P, const double *x, const double *b, double *
 // direction's rho-bar rows dn_rb; ss (optional): *_partials sums of the squares of the rows written.
 // *_schur: y2 = S (mul x2) (mul null: S x2); done (optional, batches): pores whose rows are not wanted.
 bool line_available(const Problem &P);
+int line_lanes(const Problem &P);    // positions per lane
 long long line_partials(const Problem &P);
 template <typename T>
 void line_rows_el(Problem &P, bool linear, const double *rho, const double *in_rb, const double *sub_rb, double *out_rb,
@@ -258,6 +259,7 @@ void plane_free(Problem &P);
 void plane_set(Problem &P, bool on);
 bool plane_built(const Problem &P);
 bool plane_on(const Problem &P);
+int plane_waves(const Problem &P);   // wavefronts per workgroup in FP64
 long long plane_partials(const Problem &P);
 template <typename T>
 void plane_rows_el(Problem &P, bool linear, const double *rho, const double *in_rb, const double *sub_rb, double *out_rb,

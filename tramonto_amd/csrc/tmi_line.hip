@@ -28,6 +28,15 @@
 #include "tmi_internal.hpp"
 
 namespace tmi {
+
+// Positions per lane by the span: 64 B positions a workgroup, so that small problems still reach many
+// CUs and large ones read LDS once per 4 outputs.
+int line_lanes(const Problem &P)
+{
+    const long long span = (long long)P.pad_u.P[0] - 2LL * P.pad_u.h[0];
+    return span <= 64LL * 256 ? 1 : (span <= 128LL * 256 ? 2 : 4);
+}
+
 namespace {
 
 using namespace dev;
@@ -430,14 +439,7 @@ __global__ __launch_bounds__(kLineBlock, B == 1 ? 2 : 6) void k_line(LineArgs<T>
     }
 }
 
-// Positions per lane by the span: 64 B positions a workgroup, so that small problems still reach many
-// CUs and large ones read LDS once per 4 outputs.  A call's LDS must fit (wide stencils on fine
-// grids and many components keep the row kernels).
-int line_lanes(const Problem &P)
-{
-    const long long span = (long long)P.pad_u.P[0] - 2LL * P.pad_u.h[0];
-    return span <= 64LL * 256 ? 1 : (span <= 128LL * 256 ? 2 : 4);
-}
+// A call's LDS must fit (wide stencils on fine grids and many components keep the row kernels).
 struct LineShape {
     int B, TN, hr, hf, rho_ld, rb_ld, mf_ld, adj_ld, chain_ld, blocks;
     size_t elems;

@@ -426,6 +426,7 @@ PlaneShape plane_shape(const PlanePlan &L)
     return s;
 }
 constexpr size_t kPlaneTwo = 80 * 1024;   // LDS of a workgroup of which a CU holds two
+inline int plane_waves_for(size_t lds) { return lds <= kPlaneTwo - 1024 ? 8 : 16; }
 
 template <typename T>
 PlaneArgs<T> plane_args(const Problem &P, const PlaneShape &s)
@@ -478,7 +479,7 @@ void plane_launch(const Problem &P, const PlaneShape &s, const PlaneArgs<T> &a, 
                                               (int)lds));
         hipLaunchKernelGGL(kernel, dim3((unsigned)P.plane->ntiles), dim3(64 * nw), lds, st, a);
     };
-    if (lds <= kPlaneTwo - 1024)
+    if (plane_waves_for(lds) == 8)
         go(k_plane<T, MODE, 8>, 8);
     else
         go(k_plane<T, MODE, 16>, 16);
@@ -493,6 +494,7 @@ void plane_set(Problem &P, bool on)
 {
     if (P.plane) P.plane->on = on;
 }
+int plane_waves(const Problem &P) { return P.plane ? plane_waves_for(plane_shape<double>(*P.plane).elems * sizeof(double)) : 0; }
 long long plane_partials(const Problem &P) { return plane_on(P) ? P.plane->ntiles : 0; }
 
 void plane_free(Problem &P)

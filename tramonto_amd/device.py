@@ -89,6 +89,14 @@ class DeviceProblem:
         _lib.check(_lib.lib().tmi_bulk_get(self.handle, out.ctypes.data_as(ct.c_void_p)), "tmi_bulk_get")
         return out
 
+    def row_form(self) -> Tuple[int, int]:
+        """(form, width) of a residual fill's rows (tmi_row_form): form 0 separate kernels or FFT sums, 1 a
+        1D problem's in one launch (width: positions per lane), 2 a one-component 2D problem's in one
+        launch on the matrix cores (width: wavefronts per workgroup)."""
+        form, width = ct.c_int(), ct.c_int()
+        _lib.check(_lib.lib().tmi_row_form(self.handle, ct.byref(form), ct.byref(width)), "tmi_row_form")
+        return form.value, width.value
+
     def row_tuning(self) -> Dict:
         """Autotuned launch shapes of the 1D row kernels: {precision: {kind: (per_lane, lanes, ms)}}."""
         shape = np.zeros(12, dtype=np.int32)
