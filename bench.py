@@ -47,6 +47,11 @@ AXIS_TRAFFIC_MIB = {"periodic64": None, "solute128": None}
 FILL_TRAFFIC_MIB = {"periodic64": 221.5, "solute128": 3205.2}
 
 
+def stage_names(dp):
+    """The stages that fill_residual_timed reports (one when every row runs in one launch)."""
+    return ["rows in one launch"] if dp.row_form()[0] else ["pad_rho", "rb_rows", "mf_rows", "fmt_point+pad_adj", "el_rows"]
+
+
 def stencil_flops_per_node(dp, spec):
     """Direct-form flops per node of one residual fill (2 per stencil point and product)."""
     nd, C = spec.ndim, spec.ncomp
@@ -147,8 +152,7 @@ def bench_batch(b, workload):
     out = {"workload": workload,
            "pores": npores, "nodes": int(b.nnodes), "pore_nodes_min_max": [int(b.nodes.min()), int(b.nodes.max())],
            "fill_ms": fill_ms, "fill_gnode_s": b.nnodes / (fill_ms * 1e-3) / 1e9, "fill_ms_host_norm": fill_ms_host,
-           "fill_stage_ms": dict(zip(["pad_rho", "rb_rows", "mf_rows", "fmt_point+pad_adj", "el_rows"],
-                                     [float(v) for v in db.fill_residual_timed(x0, 10)]))}
+           "fill_stage_ms": dict(zip(stage_names(db), [float(v) for v in db.fill_residual_timed(x0, 10)]))}
     sols = {}
     for name, prec, graph in (("batched_fp64_graph", PREC_FP64, "1"), ("batched_fp64_direct", PREC_FP64, "0"),
                               ("batched_mixed_graph", PREC_MIXED, "1"), ("batched_mixed_direct", PREC_MIXED, "0")):
@@ -353,7 +357,7 @@ def bench_workload(spec, label, args, newton_tol=1e-8, newton=True):
                              "FETCH_SIZE/WRITE_SIZE scaled by a 512 MiB copy"),
             "note": note, "axis_passes": axis}
     else:
-        names = ["pad_rho", "rb_rows", "mf_rows", "fmt_point+pad_adj", "el_rows"]
+        names = stage_names(dp)
         out["fill_stage_ms"] = dict(zip(names, [float(v) for v in stages]))
         per_stage_flops = [0.0, f_fwd, 0.0 if dp.info.mf_fft else f_mf, 0.0, f_adj]
         priced = [i for i in range(5) if per_stage_flops[i] > 0]

@@ -231,7 +231,9 @@ int tmi_fill_residual(void *handle, const double *x_d, double *F_d, double *sums
 int tmi_fill_residual_noalloc(void *handle, const double *x_d, double *F_d, double *sumsq_d, void *stream);
 /* The residual fill with HIP events recorded on `stream` between its stages;
  * stage_ms[0..4] receive the mean over `reps` fills of: density halo,
- * rho-bar rows, mean-field rows, pointwise FMT + adjoint halo, EL rows. */
+ * rho-bar rows, mean-field rows, pointwise FMT + adjoint halo, EL rows.  Rows
+ * in one launch (tmi_row_form) have no such stages: stage_ms[0] receives the
+ * launch, the others 0. */
 int tmi_fill_residual_timed(void *handle, const double *x_d, double *F_d, int reps, double *stage_ms, void *stream);
 /* Measurement hook, no counterpart in the reference: when the FMT sums run in
  * FFT form (tmi_info.fmt_fft), times one kernel family of a residual fill on

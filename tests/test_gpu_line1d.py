@@ -90,6 +90,8 @@ def test_line_matches_row_kernels(kind, monkeypatch):
     v = noise()
     _compare(rows.apply_jacobian(x, v), line.apply_jacobian(x, v), blocks, 1e-12)
     _compare(rows.apply_jacobian(x, v, fp32=True), line.apply_jacobian(x, v, fp32=True), blocks, 1e-5)
+    ms = line.fill_residual_timed(x, reps=2)   # the stage of the launch that a fill runs
+    assert ms[0] > 0 and not ms[1:].any() and (rows.fill_residual_timed(x, reps=2)[[0, 1, 3, 4]] > 0).all()
     # Schur product, right-hand side and back-substitution: one Newton update
     da, _ = rows.schur_solve(x, Fa, rtol=1e-12)
     db, _ = line.schur_solve(x, Fa, rtol=1e-12)

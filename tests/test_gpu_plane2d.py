@@ -81,6 +81,8 @@ def test_plane_matches_separate_kernels(kind, monkeypatch):
     v = noise()
     _compare(rows.apply_jacobian(x, v), plane.apply_jacobian(x, v), blocks, 1e-12)
     _compare(rows.apply_jacobian(x, v, fp32=True), plane.apply_jacobian(x, v, fp32=True), blocks, 1e-5)
+    ms = plane.fill_residual_timed(x, reps=2)   # the stage of the launch that a fill runs
+    assert ms[0] > 0 and not ms[1:].any() and (rows.fill_residual_timed(x, reps=2)[[0, 1, 3, 4]] > 0).all()
     # Schur product, right-hand side and back-substitution: one Newton update
     da, _ = rows.schur_solve(x, Fa, rtol=1e-12)
     db, _ = plane.schur_solve(x, Fa, rtol=1e-12)

@@ -1129,10 +1129,11 @@ int tmi_fill_residual_timed(void *handle, const double *x_d, double *F_d, int re
         hipEvent_t ev[6];
         for (auto &e : ev) TMI_HIP_CHECK(hipEventCreate(&e));
         for (int q = 0; q < 5; ++q) stage_ms[q] = 0.0;
+        const int stages = one_launch(*P) ? 1 : 5;
         for (int r = 0; r < reps; ++r) {
             launch_residual(*P, xi, Fi, s, ev);
-            TMI_HIP_CHECK(hipEventSynchronize(ev[5]));
-            for (int q = 0; q < 5; ++q) {
+            TMI_HIP_CHECK(hipEventSynchronize(ev[stages]));
+            for (int q = 0; q < stages; ++q) {
                 float ms = 0.f;
                 TMI_HIP_CHECK(hipEventElapsedTime(&ms, ev[q], ev[q + 1]));
                 stage_ms[q] += ms / reps;

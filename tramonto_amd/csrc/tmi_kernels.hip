@@ -2094,7 +2094,7 @@ void choose_fmt_form(Problem &P)
 
 // ---------------------------------------------------------------- public launchers
 // ev (optional): 6 events recorded between the stages pad_rho | rb_rows |
-// mf_rows | fmt_point+pad_adj | el_rows
+// mf_rows | fmt_point+pad_adj | el_rows; rows in one launch record the first two around it
 namespace {
 // ss (optional): partial sums of F^2 from the fused last passes; *nss their number when they cover
 // every row, else 0
@@ -2103,12 +2103,14 @@ void residual_impl(Problem &P, const double *x, double *F, hipStream_t s, hipEve
     const size_t N = P.N;
     long long n_rb = 0, n_el = 0;
     if (P.hw_fwd.nrows || P.one_size) ss = nullptr;   // the rho-bar rows change after the fused passes
-    if (!ev && one_launch(P)) {
+    if (one_launch(P)) {
+        if (ev) TMI_HIP_CHECK(hipEventRecord(ev[0], s));
         one_launch_rows_el<double>(P, false, x + P.iu_rho * N, x + P.iu_rb * N, nullptr, F + P.iu_rb * N,
                              P.nmf ? x + P.iu_mf * N : nullptr, nullptr, F + P.iu_mf * N, x, nullptr, x + P.iu_rho * N,
                              P.nmf ? x + P.iu_mf * N : nullptr, nullptr, F + P.iu_rho * N, s, ss);
         hw_apply(P.hw_fwd, x + P.iu_rho * N, F + P.iu_rb * N, s);
         one_size_rows(P, x + P.iu_rb * N, F + P.iu_rb * N, s);
+        if (ev) TMI_HIP_CHECK(hipEventRecord(ev[1], s));
         if (nss) *nss = ss ? one_launch_partials(P) : 0;
         return;
     }

@@ -191,7 +191,8 @@ class DeviceProblem:
                    "tmi_fill_residual_noalloc")
 
     def fill_residual_timed(self, x: torch.Tensor, reps: int = 10) -> np.ndarray:
-        """Mean per-stage milliseconds of `reps` fills (HIP events on the launch stream)."""
+        """Mean per-stage milliseconds of `reps` fills (HIP events on the launch stream); rows in one launch
+        (row_form) are one stage, the first."""
         F = self.zeros()
         ms = np.zeros(5)
         _lib.check(_lib.lib().tmi_fill_residual_timed(self.handle, _ptr(x), _ptr(F), reps,
