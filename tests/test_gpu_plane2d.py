@@ -107,3 +107,18 @@ def test_batched_step_solves_each_piece(walls, mixed, monkeypatch):
     plane = DeviceBatch(spec)
     assert rows.row_form()[0] == 0 and plane.row_form()[0] == 2
     check_batch_step(plane, rows, mixed, torch.Generator(device="cuda").manual_seed(2))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("env,forms", [({"TMI_MF_FFT": "1"}, (1, None)), ({"TMI_FMT_FFT": "1"}, (None, 2)),
+                                       ({"TMI_MF_FFT": "0"}, (0, None)), ({"TMI_FMT_FFT": "0"}, (None, 0))])
+def test_forced_forms_leave_the_matrix_core_rows(env, forms, monkeypatch):
+    """TMI_MF_FFT and TMI_FMT_FFT force a form of the separate sums, in batches the direct one."""
+    for k, v in env.items():
+        monkeypatch.setenv(k, v)
+    dp = DeviceProblem(small_case("2d_rough_wall"))
+    assert dp.row_form()[0] == 0
+    for got, want in zip((dp.info.mf_fft, dp.info.fmt_fft), forms):
+        assert want is None or got == want
+    if "0" in env.values():
+        assert DeviceBatch(rough_slit_pore_batch_2d(npores=2, seed=4, nx=53, h_range=(3.0, 4.0))).row_form()[0] == 0

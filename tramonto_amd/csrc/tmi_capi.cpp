@@ -613,16 +613,16 @@ Problem *create_problem(const tmi_params &p_in, const double *vext, const unsign
         // stencils are wide (TMI_MF_FFT=1 forces it, 0 keeps the direct sums), the FMT sums when
         // that form fills faster (TMI_FMT_FFT=1 / 0 forces the FFT / direct form)
         if (!symbol_only) plane_setup(*P);
+        const char *fe = std::getenv("TMI_MF_FFT"), *fm = std::getenv("TMI_FMT_FFT");
+        // a forced form of any of the sums means the separate kernels (batches know the direct form only)
+        if (batch ? (fe && std::string(fe) == "0") || (fm && std::string(fm) == "0") : fe || fm) plane_free(*P);
         if (batch) plane_set(*P, true);
         if (nd >= 2 && !batch) {   // batches of 2D pieces keep the direct sums (their padded copy has gap rows)
-            const char *fe = std::getenv("TMI_MF_FFT"), *fm = std::getenv("TMI_FMT_FFT");
             long long lsum = 0;
             if (p.type_attr >= 0)
                 for (int q = 0; q < C * C; ++q) lsum += P->hs[TMI_UATT][q].L;
             const bool mf = p.type_attr >= 0 && (fe ? std::string(fe) == "1" : lsum >= kFftMinStencil);
             const bool fmt = !(fm && std::string(fm) == "0");
-            // a forced direct form of any of the sums means the separate kernels
-            if ((fe && std::string(fe) == "0") || !fmt) plane_free(*P);
             fft_setup(*P, mf, fmt);
             if (!symbol_only) {
                 choose_fmt_form(*P);
