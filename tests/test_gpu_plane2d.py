@@ -122,3 +122,28 @@ def test_forced_forms_leave_the_matrix_core_rows(env, forms, monkeypatch):
         assert want is None or got == want
     if "0" in env.values():
         assert DeviceBatch(rough_slit_pore_batch_2d(npores=2, seed=4, nx=53, h_range=(3.0, 4.0))).row_form()[0] == 0
+
+
+@pytest.mark.gpu
+def test_reference_jacobian_beside_the_matrix_core_rows(monkeypatch):
+    """Where the timing picks the matrix-core rows, products with the reference's Jacobian run in the separate
+    forms that the timing kept beside them: the same rows as with those forms forced."""
+    from tramonto_amd.device import JAC_REFERENCE
+    spec = _box(64, 64, [[PERIODIC, PERIODIC], [PERIODIC, PERIODIC]], cut=2.5, func=3)
+    plane = DeviceProblem(spec)
+    assert plane.row_form()[0] == 2 and (plane.info.mf_fft, plane.info.fmt_fft, plane.info.fft_xreg) == (0, 0, 0)
+    with pytest.raises(RuntimeError):
+        plane.fft_timed(0, 1)   # no such launches in its fill
+    monkeypatch.setenv("TMI_FMT_FFT", "0")
+    monkeypatch.setenv("TMI_MF_FFT", "0")
+    direct = DeviceProblem(spec)
+    x = direct.initial_state()
+    g = torch.Generator(device="cuda").manual_seed(4)
+    v = 2 * torch.rand(x.shape, generator=g, device="cuda", dtype=torch.float64) - 1
+    for p in (plane, direct):
+        p.set_jacobian(JAC_REFERENCE)
+    _compare(direct.apply_jacobian(x, v), plane.apply_jacobian(x, v), ((0, 1), (1, 9), (9, 10)), 1e-12)
+    F, _ = direct.fill_residual(x)
+    da, _ = direct.schur_solve(x, F, rtol=1e-12)
+    db, _ = plane.schur_solve(x, F, rtol=1e-12)
+    _compare(da, db, ((0, 1), (1, 9), (9, 10)), 1e-8)

@@ -986,11 +986,12 @@ int tmi_problem_info(void *handle, tmi_info *info)
         info->n_mf = P->ext_mf ? 0 : P->nmf;
         for (int t = 0; t < 3; ++t)
             for (int q = 0; q < kNC * kNC; ++q) info->sten_len[t][q] = P->hs[t][q].L;
-        info->mf_fft = fft_mf(*P) ? 1 : 0;
-        info->fmt_fft = fft_fmt(*P) ? (fft_fused(*P) ? 2 : 1) : 0;
+        const bool sums = !plane_on(*P);   // the matrix-core rows take neither form (tmi_row_form)
+        info->mf_fft = sums && fft_mf(*P) ? 1 : 0;
+        info->fmt_fft = sums && fft_fmt(*P) ? (fft_fused(*P) ? 2 : 1) : 0;
         info->precond = precond_active(*P) ? 1 : 0;
         info->fft_fold = fft_folded(*P) ? 1 : 0;
-        info->fft_xreg = fft_xreg_mask(*P);
+        info->fft_xreg = sums ? fft_xreg_mask(*P) : 0;
         info->fft_regpass = fft_regpass_mode(*P);
         info->jacobian = P->jac_ref ? TMI_JAC_REFERENCE : TMI_JAC_EXACT;
         return 0;

@@ -3197,7 +3197,8 @@ bool fft_vjp(Problem &P, const double *x, const double *w, double *y, hipStream_
     fft_pass<T>(F, Z, F.vz, -1, 2, s);
     fft_pass<T>(F, Z, F.vz, -1, 1, s);
     // the fused x pass where the fill uses it, or where it fits when the fill runs the direct sums
-    const int lpb_b = F.fmt ? F.xlpb[0] : F.xfit[0], lpb_r = F.fmt ? F.xlpb[1] : F.xfit[1];
+    const bool chosen = F.fmt && !plane_on(P);
+    const int lpb_b = chosen ? F.xlpb[0] : F.xfit[0], lpb_r = chosen ? F.xlpb[1] : F.xfit[1];
     if (lpb_r) {
         fft_xprod<T>(F, Z, Or, F.tvr, lpb_r, fmt_spectra<T>(F), attr_spectra<T>(F), s);
     } else {
@@ -3281,7 +3282,7 @@ template bool fft_vjp<float>(Problem &, const double *, const double *, double *
 // contents are scratch between products.
 void fft_time_kernels(Problem &P, int which, int reps, double *ms, double *bytes, int *launches, hipStream_t s)
 {
-    if (!fft_fmt(P)) throw std::logic_error("the FMT sums are not in FFT form");
+    if (!fft_fmt(P) || plane_on(P)) throw std::logic_error("the FMT sums are not in FFT form");
     const FftPlan &F = *P.fft;
     if (which == 1 && !(F.xlpb[0] || F.xlpb[1])) throw std::logic_error("the fused x pass is not in use");
     const int C = P.p.ncomp, nadj = F.dform ? 4 + 2 * P.p.ndim : C * (1 + P.p.ndim) + 1;

@@ -2025,14 +2025,21 @@ void autotune_rows1d(Problem &P)
 // ---------------------------------------------------------------- FMT form
 // Times residual fills with the FMT sums as direct stencil sums, as FFT
 // convolutions with separate x passes and product kernels, and with the fused
-// x pass for the density product, the Euler-Lagrange product or both (state:
-// every unknown 4.8e-4, a positive byte pattern), and keeps the fastest.
+// x pass for the density product, the Euler-Lagrange product or both, and (2D, one
+// component) with every row in one launch on the matrix cores (state: every unknown
+// 4.8e-4, a positive byte pattern), and keeps the fastest.  Beside the matrix-core rows
+// the fastest of the separate forms stays set: products that those rows do not
+// serve (the reference's Jacobian, Schur products under hard surfaces) run in it
+// (256^2 rough wall, reference Jacobian: 105 us, the direct form 117; 64^2 periodic: 48 and 69).
 // TMI_FMT_FFT=1 / 0 forces the FFT / direct form (the fused x pass is then
 // used for both products where it fits, unless TMI_FFT_XFUSE=0).
 void choose_fmt_form(Problem &P)
 {
     if (!fft_fmt_available(P)) {
-        plane_set(P, true);   // against the separate direct kernels
+        // against the separate direct kernels alone (lines of more than 768 nodes), and in batches, the
+        // matrix-core rows always filled faster: 1000 x 300 with attraction 246 -> 132 us, hard spheres 98 -> 45,
+        // 1000 x 24 43 -> 16; 16 slits 110 -> 48
+        plane_set(P, true);
         return;
     }
     const char *pe = std::getenv("TMI_PLANE2D");
@@ -2051,14 +2058,21 @@ void choose_fmt_form(Problem &P)
     const size_t n = (size_t)P.nunk * P.N;
     double *x = nullptr, *F = nullptr;
     hipEvent_t e0 = nullptr, e1 = nullptr;
-    // forms: 0 direct (2D, one component: every row on the matrix cores where its windows fit); 1 + mask:
-    // FFT with the fused x pass for the products in mask (bit 0 density, bit 1 EL)
+    // forms of the separate sums: 0 direct; 1 + mask: FFT with the fused x pass for the products in mask
+    // (bit 0 density, bit 1 EL)
     const int nform = fft_fused_available(P) ? 5 : 2;
-    float ms[5] = {0.f, 0.f, 0.f, 0.f, 0.f};
+    float ms[5] = {0.f, 0.f, 0.f, 0.f, 0.f}, ms_plane = 0.f;
     auto set_form = [&](int form) {
-        plane_set(P, form == 0);
         fft_set_fmt(P, form > 0);
         fft_set_fused(P, form > 0 ? form - 1 : 0);
+    };
+    auto time_fills = [&](float *out) {
+        launch_residual(P, x, F, 0);
+        TMI_HIP_CHECK(hipEventRecord(e0, 0));
+        for (int r = 0; r < 3; ++r) launch_residual(P, x, F, 0);
+        TMI_HIP_CHECK(hipEventRecord(e1, 0));
+        TMI_HIP_CHECK(hipEventSynchronize(e1));
+        TMI_HIP_CHECK(hipEventElapsedTime(out, e0, e1));
     };
     try {
         TMI_HIP_CHECK(hipMalloc((void **)&x, n * sizeof(double)));
@@ -2068,12 +2082,11 @@ void choose_fmt_form(Problem &P)
         TMI_HIP_CHECK(hipEventCreate(&e1));
         for (int form = 0; form < nform; ++form) {
             set_form(form);
-            launch_residual(P, x, F, 0);
-            TMI_HIP_CHECK(hipEventRecord(e0, 0));
-            for (int r = 0; r < 3; ++r) launch_residual(P, x, F, 0);
-            TMI_HIP_CHECK(hipEventRecord(e1, 0));
-            TMI_HIP_CHECK(hipEventSynchronize(e1));
-            TMI_HIP_CHECK(hipEventElapsedTime(&ms[form], e0, e1));
+            time_fills(&ms[form]);
+        }
+        if (plane_built(P)) {
+            plane_set(P, true);
+            time_fills(&ms_plane);
         }
     } catch (...) {
         (void)hipFree(x);
@@ -2090,6 +2103,7 @@ void choose_fmt_form(Problem &P)
     for (int form = 1; form < nform; ++form)
         if (ms[form] < ms[best]) best = form;
     set_form(best);
+    plane_set(P, ms_plane < ms[best]);
 }
 
 // ---------------------------------------------------------------- public launchers
