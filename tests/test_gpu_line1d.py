@@ -35,6 +35,8 @@ def _single(kind):
         return sp
     if kind == "long2":
         return hard_wall_1d(seed=6, size=0.05 * 20000, dx=0.05, rho_b=0.6)
+    if kind == "long_rows":   # the rows alone go to the row kernels
+        return hard_wall_1d(seed=6, size=0.05 * 140000, dx=0.05, rho_b=0.4)
     if kind == "long4":
         return slit_pore_1d(H=0.05 * 40001, dx=0.05, seed=7)
     return small_case(kind)
@@ -58,7 +60,7 @@ def _compare(a, b, blocks, tol):
 
 
 KINDS = ["1d_hw", "1d_reflect_wca", "1d_pore_mix", "1d_reflect_slab", "periodic", "reflect", "reflect_bulk", "reflect_hs",
-         "three", "long2", "long4", "batch_small", "batch_large"]
+         "three", "long2", "long4", "long_rows", "batch_small", "batch_large"]
 
 
 @pytest.mark.gpu
@@ -98,7 +100,7 @@ def test_line_matches_row_kernels(kind, monkeypatch):
     _compare(da, db, blocks, 1e-8)
     dm, _ = line.schur_solve(x, Fa, rtol=1e-8, restart=500, maxit=2500, precision=PREC_MIXED)
     check_update(rows, x, Fa, dm, C, row_scale(rows, x, C, g), mixed=True)
-    assert line.row_form()[1] == {"long2": 2, "long4": 4, "batch_large": 4}.get(kind, 1)
+    assert line.row_form()[1] == {"long2": 2, "long4": 4, "long_rows": 4, "batch_large": 4}.get(kind, 1)
 
 
 @pytest.mark.gpu

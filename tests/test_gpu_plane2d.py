@@ -147,3 +147,23 @@ def test_reference_jacobian_beside_the_matrix_core_rows(monkeypatch):
     da, _ = direct.schur_solve(x, F, rtol=1e-12)
     db, _ = plane.schur_solve(x, F, rtol=1e-12)
     _compare(da, db, ((0, 1), (1, 9), (9, 10)), 1e-8)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("cut", [0.0, 2.5])
+def test_rows_alone_beside_the_matrix_core_fill(cut, monkeypatch):
+    """Initial fields and back-substitution run in whichever form the set-up timed faster for the rows alone
+    (hard spheres: mostly the separate kernels beside a matrix-core fill): the forced forms' rows."""
+    spec = _box(64, 48, [[PERIODIC, PERIODIC], [IN_WALL, IN_BULK]], cut=cut)
+    plane = DeviceProblem(spec)
+    assert plane.row_form()[0] == 2
+    monkeypatch.setenv("TMI_FMT_FFT", "0")
+    monkeypatch.setenv("TMI_MF_FFT", "0")
+    direct = DeviceProblem(spec)
+    x = direct.initial_state()
+    blocks = ((0, 1), (1, 9), (9, x.shape[0]))
+    _compare(x, plane.initial_state(), blocks, 1e-12)
+    F, _ = direct.fill_residual(x)
+    da, _ = direct.schur_solve(x, F, rtol=1e-12)
+    db, _ = plane.schur_solve(x, F, rtol=1e-12)
+    _compare(da, db, blocks, 1e-8)

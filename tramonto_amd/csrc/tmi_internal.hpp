@@ -259,6 +259,8 @@ void plane_free(Problem &P);
 void plane_set(Problem &P, bool on);
 bool plane_built(const Problem &P);
 bool plane_on(const Problem &P);
+void plane_set_rows(Problem &P, bool on);   // calls for the rows alone as well
+bool plane_rows(const Problem &P);
 int plane_waves(const Problem &P);   // wavefronts per workgroup in FP64
 long long plane_partials(const Problem &P);
 template <typename T>

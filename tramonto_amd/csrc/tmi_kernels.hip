@@ -2061,19 +2061,24 @@ void choose_fmt_form(Problem &P)
     // forms of the separate sums: 0 direct; 1 + mask: FFT with the fused x pass for the products in mask
     // (bit 0 density, bit 1 EL)
     const int nform = fft_fused_available(P) ? 5 : 2;
-    float ms[5] = {0.f, 0.f, 0.f, 0.f, 0.f}, ms_plane = 0.f;
+    float ms[5] = {0.f, 0.f, 0.f, 0.f, 0.f};
     auto set_form = [&](int form) {
         fft_set_fmt(P, form > 0);
         fft_set_fused(P, form > 0 ? form - 1 : 0);
     };
-    auto time_fills = [&](float *out) {
-        launch_residual(P, x, F, 0);
+    auto time_calls = [&](auto &&call) {
+        float t = 0.f;
+        call();
         TMI_HIP_CHECK(hipEventRecord(e0, 0));
-        for (int r = 0; r < 3; ++r) launch_residual(P, x, F, 0);
+        for (int r = 0; r < 3; ++r) call();
         TMI_HIP_CHECK(hipEventRecord(e1, 0));
         TMI_HIP_CHECK(hipEventSynchronize(e1));
-        TMI_HIP_CHECK(hipEventElapsedTime(out, e0, e1));
+        TMI_HIP_CHECK(hipEventElapsedTime(&t, e0, e1));
+        return t;
     };
+    auto fill = [&] { launch_residual(P, x, F, 0); };
+    int best = 0;
+    bool plane = false;
     try {
         TMI_HIP_CHECK(hipMalloc((void **)&x, n * sizeof(double)));
         TMI_HIP_CHECK(hipMalloc((void **)&F, n * sizeof(double)));
@@ -2082,11 +2087,21 @@ void choose_fmt_form(Problem &P)
         TMI_HIP_CHECK(hipEventCreate(&e1));
         for (int form = 0; form < nform; ++form) {
             set_form(form);
-            time_fills(&ms[form]);
+            ms[form] = time_calls(fill);
+            if (ms[form] < ms[best]) best = form;
         }
+        set_form(best);
         if (plane_built(P)) {
             plane_set(P, true);
-            time_fills(&ms_plane);
+            plane = time_calls(fill) < ms[best];
+            // the rows alone (a quarter of the matrix-core waves at work without attraction: 64^2 to 512^2 hard
+            // spheres at dx = 0.1 sigma 20 -> 23 and 46 -> 56 us, at dx = 0.25 sigma 18 -> 16)
+            auto rows = [&] { launch_init_fields(P, F, 0); };
+            TMI_HIP_CHECK(hipMemset(F, 0x3f, n * sizeof(double)));
+            plane_set_rows(P, false);
+            const float apart = time_calls(rows);
+            plane_set_rows(P, true);
+            plane_set_rows(P, time_calls(rows) <= apart);
         }
     } catch (...) {
         (void)hipFree(x);
@@ -2099,11 +2114,7 @@ void choose_fmt_form(Problem &P)
     (void)hipFree(F);
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
-    int best = 0;
-    for (int form = 1; form < nform; ++form)
-        if (ms[form] < ms[best]) best = form;
-    set_form(best);
-    plane_set(P, ms_plane < ms[best]);
+    plane_set(P, plane);
 }
 
 // ---------------------------------------------------------------- public launchers
@@ -2322,10 +2333,20 @@ void launch_jvp(Problem &P, const double *x, const double *v, double *Jv, hipStr
 template void launch_jvp<double>(Problem &, const double *, const double *, double *, hipStream_t);
 template void launch_jvp<float>(Problem &, const double *, const double *, double *, hipStream_t);
 
+// Calls for the rho-bar and mean-field rows alone (initial fields, back-substitution) through the one-launch
+// rows: on the matrix cores as the set-up timed them; in 1D unless nothing but one component's short sums
+// is left of the launch's work (hard spheres, 200,000 nodes: 18 us, row kernels 14; 100,000: both 12; with
+// attraction 21 and 22)
+static bool rows_one_launch(const Problem &P)
+{
+    if (plane_on(P)) return plane_rows(P);
+    return line_available(P) && !(P.p.ncomp == 1 && P.nmf == 0 && P.N > 131072);
+}
+
 void launch_init_fields(Problem &P, double *x, hipStream_t s)
 {
     const size_t N = P.N;
-    if (one_launch(P))
+    if (rows_one_launch(P))
         one_launch_rows_el<double>(P, false, x + P.iu_rho * N, nullptr, nullptr, x + P.iu_rb * N, nullptr, nullptr,
                              x + P.iu_mf * N, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, s);
     else
@@ -2381,7 +2402,7 @@ void launch_schur_backsub(Problem &P, const double *x, const double *b, double *
 {
     (void)x;
     const size_t N = P.N;
-    if (one_launch(P))
+    if (rows_one_launch(P))
         one_launch_rows_el<double>(P, true, dx + P.iu_rho * N, nullptr, b + P.iu_rb * N, dx + P.iu_rb * N, nullptr,
                              P.nmf ? b + P.iu_mf * N : nullptr, P.nmf ? dx + P.iu_mf * N : nullptr, nullptr, nullptr,
                              nullptr, nullptr, nullptr, nullptr, s);

@@ -46,7 +46,7 @@ struct PlanePlan {
     int2 *kf = nullptr, *ku = nullptr;
     int fx = 0, fy = 0, hx = 0, hy = 0;
     void *adj = nullptr;     // [4][N] adjoint fields at the nodes (Schur products)
-    bool on = false;
+    bool on = false, rows = true;   // serves the problem; calls for the rows alone as well
 };
 
 namespace {
@@ -494,6 +494,11 @@ void plane_set(Problem &P, bool on)
 {
     if (P.plane) P.plane->on = on;
 }
+void plane_set_rows(Problem &P, bool on)
+{
+    if (P.plane) P.plane->rows = on;
+}
+bool plane_rows(const Problem &P) { return P.plane && P.plane->rows; }
 int plane_waves(const Problem &P) { return P.plane ? plane_waves_for(plane_shape<double>(*P.plane).elems * sizeof(double)) : 0; }
 long long plane_partials(const Problem &P) { return plane_on(P) ? P.plane->ntiles : 0; }
 
