@@ -55,3 +55,26 @@ def test_spectral_transpose_matches_gather(case, env, monkeypatch):
             err = float((a[lo:hi] - b[lo:hi]).abs().max()) / scale
             assert err < RTOL, (lo, err)
     assert np.isfinite(float(b.abs().max()))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,dx,gathers", [(64, 0.1, False), (300, 0.25, True)])
+def test_short_2d_stencils_keep_the_gathers(n, dx, gathers, monkeypatch):
+    """2D hard spheres: the gathers where the rule expects them to be faster (then the very kernels of a problem
+    without spectra, bit for bit), else the spectral products."""
+    from tramonto_amd.device import DeviceProblem
+    from tramonto_amd.problem import IN_BULK, IN_WALL, PERIODIC, ProblemSpec, SplitMix64
+    rho = 0.4 * (1 + 0.2 * SplitMix64(3).uniform(n * n, -1, 1))
+    spec = ProblemSpec(name="hs", ndim=2, ncomp=1, nx=[n, n], dx=[dx, dx], bc=[[IN_WALL, IN_BULK], [PERIODIC, PERIODIC]],
+                       type_func=0, type_attr=-1, hs_diam=[1.0], sigma_ff=np.ones((1, 1)), eps_ff=np.ones((1, 1)),
+                       cut_ff=np.ones((1, 1)), rho_b=[0.4], rho0=rho[None, :])
+    chosen = DeviceProblem(spec)
+    monkeypatch.setenv("TMI_FMT_FFT", "0")
+    direct = DeviceProblem(spec)
+    x = direct.initial_state()
+    g = torch.Generator(device="cuda").manual_seed(5)
+    w = 2 * torch.rand(x.shape, generator=g, device="cuda", dtype=torch.float64) - 1
+    a, b = direct.apply_jacobian_transpose(x, w), chosen.apply_jacobian_transpose(x, w)
+    for lo, hi in ((0, 1), (1, 9)):
+        assert float((a[lo:hi] - b[lo:hi]).abs().max()) <= RTOL * float(a[lo:hi].abs().max())
+    assert torch.equal(a, b) == gathers

@@ -19,7 +19,7 @@
 //
 // On 2D/3D grids whose spectra are built the three steps run as spectral products (fft_vjp,
 // tmi_fft.hip); the gathers here serve 1D problems and 2D/3D ones whose stencils stay direct
-// (a small attraction stencil, TMI_FMT_FFT=0 or TMI_MF_FFT=0).
+// (a small attraction stencil, TMI_FMT_FFT=0 or TMI_MF_FFT=0) or so short that the gathers are faster.
 #include <hip/hip_runtime.h>
 
 #include "tmi_device.hpp"

@@ -3161,12 +3161,27 @@ template void fft_el<double>(Problem &, bool, const double *, const double *, co
 template void fft_el<float>(Problem &, bool, const double *, const double *, const double *, const double *, double *,
                             hipStream_t, double *, long long *);
 
+// 2D hard spheres, whose stencils are short: whether the gathers take less time than the spectral products.
+// Microseconds by launches, stencil points L and grid points, fitted to 114 problems of 48^2 to 720^2 nodes,
+// dx 0.05 to 0.34 sigma, one to three components (both within 8 % on average; the choice loses 0.3 %):
+// 400^2 at dx = 0.25 sigma, gathers 65, products 112; 256^2 at dx = 0.1, gathers 105, products 70.  In 3D, and
+// with attraction spectra, the products were faster throughout.
+bool vjp_gathers(const Problem &P)
+{
+    if (P.p.ndim != 2 || P.nmf > 0) return false;
+    const FftPlan &F = *P.fft;
+    const double C = P.p.ncomp, N = 1e-6 * P.N;
+    double L = 0.0;
+    for (int c = 0; c < P.p.ncomp; ++c) L += P.hs[TMI_THETA][c].L + P.hs[TMI_DELTA][c].L;
+    return 26.0 + 7.2 * C + 0.17 * L + N * (1.6 * L + 34.0 * C) < 42.0 + 4.4 * C + 1e-6 * F.n * (208.0 + 182.0 * C);
+}
+
 // y = J(x)^T w as spectral products (w, y: node rows of the internal layout).  Both products share
-// their z and y passes.  False where the plan lacks a spectrum (the caller then runs the gathers).
+// their z and y passes.  False where the plan lacks a spectrum or the gathers are faster (the caller runs them).
 template <typename T>
 bool fft_vjp(Problem &P, const double *x, const double *w, double *y, hipStream_t s)
 {
-    if (!P.fft || !P.fft->fmt_ok || (P.nmf > 0 && !P.fft->mf)) return false;
+    if (!P.fft || !P.fft->fmt_ok || (P.nmf > 0 && !P.fft->mf) || vjp_gathers(P)) return false;
     FftPlan &F = *P.fft;
     const size_t N = P.N;
     const int C = P.p.ncomp, nd = P.p.ndim;

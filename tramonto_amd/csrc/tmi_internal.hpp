@@ -350,7 +350,7 @@ bool fft_node_input(const Problem &P);   // every density product reads the node
 template <typename T>
 void fft_el(Problem &P, bool linear, const double *x_rho, const double *in_rho, const double *in_mf, const double *add,
             double *out_el, hipStream_t s, double *ss = nullptr, long long *nss = nullptr);
-// transpose product as spectral products; false where the plan lacks a spectrum it needs
+// transpose product as spectral products; false where the plan lacks a spectrum it needs or the gathers are faster
 template <typename T>
 bool fft_vjp(Problem &P, const double *x, const double *w, double *y, hipStream_t s);
 double *fft_ss_buffer(const Problem &P, long long *cap);   // partial sums of F^2 of the fused last passes
