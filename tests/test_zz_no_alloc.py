@@ -2,8 +2,8 @@
 
 Called through the C ABI on two problems in a row, the second smaller, then the first again: F and
 the sum of squares it writes to device memory equal tmi_fill_residual's bit for bit.  The first
-problem fills in FFT form (the partial sums come from the fused last passes), the second in direct
-1D form (the partial sums of one dot product), the third in the ATTInA22Block layout.  The scratch
+problem fills in FFT form (the partial sums come from the fused last passes), the second in one 1D
+launch (one partial sum per workgroup), the third in the ATTInA22Block layout.  The scratch
 array keeps the previous call's contents, so a stale partial sum would show.
 """
 import ctypes as ct
@@ -60,3 +60,28 @@ def test_noalloc_fill_equals_the_allocating_fill(monkeypatch):
         assert np.array_equal(F1, F2)
         assert s1 == s2, (s1, s2)
         assert abs(s1 - float((F1 ** 2).sum())) <= 1e-12 * s1
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("blocks", [131072, 131073])
+def test_noalloc_fill_at_the_scratch_limit(blocks):
+    """A 1D problem of as many workgroups as the scratch has partial sums, and of one more: accepted, and the sum
+    is tmi_fill_residual's, bit for bit, and the dot product of F (1e-12)."""
+    from tramonto_amd.device import DeviceProblem
+    from tramonto_amd.problem import IN_BULK, ProblemSpec
+    n = 256 * blocks   # 256 positions a workgroup
+    rho0 = 0.4 + 0.1 * np.sin(np.arange(n) * 0.37)
+    spec = ProblemSpec(name="long", ndim=1, ncomp=1, nx=[n], dx=[0.25], bc=[[IN_BULK, IN_BULK]], type_func=0, type_attr=-1,
+                       hs_diam=[1.0], sigma_ff=np.ones((1, 1)), eps_ff=np.ones((1, 1)), cut_ff=np.ones((1, 1)), rho_b=[0.4],
+                       rho0=rho0[None, :])
+    dp = DeviceProblem(spec)
+    assert dp.row_form() == (1, 4)
+    x = dp.initial_state()
+    x[1:] *= 1.001
+    F = dp.zeros()
+    s2 = torch.full((1,), np.nan, dtype=torch.float64, device="cuda")
+    dp.fill_residual_device_norm(x, F, s2)
+    F1, s1 = dp.fill_residual(x)
+    assert torch.equal(F, F1) and float(s2) == s1
+    ref = float((F1 * F1).sum())
+    assert abs(s1 - ref) <= 1e-12 * ref

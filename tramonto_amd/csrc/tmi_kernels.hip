@@ -2274,17 +2274,24 @@ void observables_sums(Problem &P, const double *x, const int *nh_d, const int *n
     for (int v = 0; v < kObsVals; ++v) sums[v] = P.h_red[v];
 }
 
+// Rows in one launch sum F^2 by workgroup where the partial sums fit the allocation-free fill's scratch (33.5
+// million nodes in 1D and 2D); larger problems take a dot product, as the separate kernels do
+static bool one_launch_sums(const Problem &P)
+{
+    return one_launch(P) && one_launch_partials(P) <= kNoAllocScratchDoubles;
+}
+
 long long residual_sumsq_partials(const Problem &P)
 {
     long long cap = 0;
     fft_ss_buffer(P, &cap);
-    return std::max<long long>({cap, one_launch_partials(P), 1024});
+    return std::max<long long>({cap, one_launch_sums(P) ? one_launch_partials(P) : 0, 1024});
 }
 
 void residual_sumsq_device(Problem &P, const double *x, double *F, double *partials, double *sumsq_d, hipStream_t s)
 {
     long long cnt = 0;
-    residual_impl(P, x, F, s, nullptr, P.fft || one_launch(P) ? partials : nullptr, &cnt);
+    residual_impl(P, x, F, s, nullptr, (one_launch(P) ? one_launch_sums(P) : P.fft != nullptr) ? partials : nullptr, &cnt);
     if (cnt > 0) {
         hipLaunchKernelGGL(k_sum_partials, dim3(1), dim3(kSumBlock), 0, s, partials, (int)cnt, sumsq_d, nullptr);
     } else {   // the blocks and order of dev_dot
@@ -2300,8 +2307,9 @@ double residual_sumsq(Problem &P, const double *x, double *F, hipStream_t s)
 {
     long long cap = 0, cnt = 0;
     double *ss = fft_ss_buffer(P, &cap);
-    if (one_launch(P) && one_launch_partials(P) <= kRedPartials) {
-        ss = P.d_red;
+    if (one_launch(P)) {
+        static_assert(kNoAllocScratchDoubles <= kRedPartials, "");
+        ss = one_launch_sums(P) ? P.d_red : nullptr;
         cap = kRedPartials;
     }
     residual_impl(P, x, F, s, nullptr, ss, &cnt);
