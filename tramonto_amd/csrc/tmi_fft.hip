@@ -1747,7 +1747,7 @@ __global__ void k_el_extract(FftGeo f, Geo g, CompConsts cc, int linear, int nwa
 // (for_each_image); a wrapping axis has summed them already.
 // Bound by HBM and launches like the fill's passes, where the per-point reversed gather
 // (k_corr_rho) does L_u multiply-adds per padded position: 64^3 with a 71,831-point attraction
-// stencil 84.5 ms -> 0.101 ms, 256^2 rough wall (8217 points) 1.61 ms -> 0.078 ms.
+// stencil 84.5 ms -> 0.096 ms, 256^2 rough wall (8217 points) 1.61 ms -> 0.082 ms.
 
 // Input pairs of both products at every FFT-grid point (zero off the nodes): the density columns'
 // fields (DF: the weights themselves, rho-bar order, then w_mf), then the EL rows' weights
@@ -1788,7 +1788,7 @@ __global__ void k_vjp_gather(FftGeo f, Geo g, const double *__restrict__ w_rb, c
     }
 }
 
-// Geometry whose images k_vjp_fold enumerates: halo h on the padded axes, none on the wrapping ones,
+// Geometry whose images k_vjp_point enumerates: halo h on the padded axes, none on the wrapping ones,
 // where the circular product has summed the periodic images
 inline Geo vjp_geo(const FftPlan &F, Geo g)
 {
