@@ -2088,17 +2088,19 @@ void choose_fmt_form(Problem &P)
         for (int form = 0; form < nform; ++form) {
             set_form(form);
             ms[form] = time_calls(fill);
-            // one component's FFT sums beside direct mean-field rows launch six kernels more, which each Krylov step
-            // waits for: they have to gain over 7 % (cut-off 1.3 sigma at dx = 0.25 sigma, fill and a Schur solve of 5
-            // steps: 64^3 147 and 1358 us against 154 and 1296 direct, 72^3 297 and 2333 against 323 and 2326; two
-            // components come out even)
-            if (form > 0 && P.p.ncomp == 1 && P.nmf > 0 && !fft_mf(P)) ms[form] *= 1.07f;
+            // FFT sums beside direct mean-field rows launch six kernels more, which each Krylov step waits for (it ends
+            // on a host read): they have to gain as much, 16 us a fill (cut-off 1.3 sigma at dx = 0.25 sigma, fill and
+            // a Schur solve of 5 steps: 64^3 147 and 1358 us against 154 and 1296 direct, 72^3 297 and 2333 against 323
+            // and 2326)
+            if (form > 0 && P.nmf > 0 && !fft_mf(P)) ms[form] += 3 * 0.016f;
             if (ms[form] < ms[best]) best = form;
         }
         set_form(best);
         if (plane_built(P)) {
             plane_set(P, true);
             plane = time_calls(fill) < ms[best];
+        }
+        if (plane) {
             // the rows alone (a quarter of the matrix-core waves at work without attraction: 64^2 to 512^2 hard
             // spheres at dx = 0.1 sigma 20 -> 23 and 46 -> 56 us, at dx = 0.25 sigma 18 -> 16)
             auto rows = [&] { launch_init_fields(P, F, 0); };
