@@ -597,10 +597,15 @@ static BatchWork &batch_work(Problem &P, int m)
                       (size_t)(P.nrb + P.nmf) * P.N /*t1*/ + (2 + (size_t)P.nunk) * (size_t)Pn +
                       (size_t)Pn * ((size_t)(m + 1) * m + 2 * m + (m + 1) + m + 2 * (m + 1) + 2);
     const size_t ni = (size_t)Pn * 6 + 2;
-    TMI_HIP_CHECK(hipStreamCreateWithFlags(&W->stream, hipStreamNonBlocking));
-    TMI_HIP_CHECK(hipMalloc((void **)&W->buf, nd * sizeof(double)));
-    TMI_HIP_CHECK(hipMalloc((void **)&W->ibuf, ni * sizeof(int)));
-    TMI_HIP_CHECK(hipHostMalloc((void **)&W->h_counts, 2 * sizeof(int), hipHostMallocDefault));
+    try {
+        TMI_HIP_CHECK(hipStreamCreateWithFlags(&W->stream, hipStreamNonBlocking));
+        TMI_HIP_CHECK(hipMalloc((void **)&W->buf, nd * sizeof(double)));
+        TMI_HIP_CHECK(hipMalloc((void **)&W->ibuf, ni * sizeof(int)));
+        TMI_HIP_CHECK(hipHostMalloc((void **)&W->h_counts, 2 * sizeof(int), hipHostMallocDefault));
+    } catch (...) {   // no half-built work for the next solve of this length to take
+        free_batch_work(P);
+        throw;
+    }
     double *q = W->buf;
     auto take = [&](size_t n) {
         double *r = q;
